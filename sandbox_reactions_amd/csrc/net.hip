@@ -7,13 +7,14 @@
 //
 //   * activations are channels-last BF16 (pixel-major, channels contiguous), so a lane's eight consecutive K values
 //     of the implicit GEMM are one 16-byte load;
-//   * k_conv is the implicit-GEMM 3x3 convolution on the matrix cores: M = pixels (16 per MFMA tile, a 32 x 4
-//     pixel tile per block with its input staged in LDS), N = output channels, K = 9 taps x input channels in chunks
-//     of 32 (v_mfma_f32_16x16x32_bf16). The same kernel computes the backward-data pass with mirrored, transposed
-//     weights and the ReLU mask applied while staging; upsample + concat of the decoder is folded into the staging;
+//   * k_conv is the implicit-GEMM 3x3 convolution on the matrix cores: M = output channels, N = pixels (16 x R rows per
+//     wave, the tile's input staged in LDS 32 channels at a time), K = taps x input channels in chunks of 32
+//     (v_mfma_f32_16x16x32_bf16). The same kernel computes the backward-data pass with mirrored, transposed weights and
+//     the ReLU mask applied while staging; upsample + concat of the decoder is folded into the staging, the encoder's
+//     2x2 pooling and the output 1x1 layer into the epilogue;
 //   * the weight gradient (k_dw) is a reduction over pixels: FP32 on the vector units from LDS tiles, per-block
 //     partials summed in a fixed order by k_dw_reduce (deterministic, no atomics);
-//   * the output 1x1 layer, the features and the energy-norm loss are elementwise / stencil kernels.
+//   * the features and the energy-norm loss are elementwise / stencil kernels.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -26,6 +27,7 @@
 namespace sr {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define NTH 256
@@ -33,6 +35,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define DW_SEG 32
 #define DW_BLOCKS 256
 #define LOG_CLAMP 20.0f
+#define CONV_FILL 512  // blocks that a convolution's launch keeps the chip busy with
 
 __device__ __forceinline__ bf16x8 ld8(const bf16 *p) { return *(const bf16x8 *)p; }
 __device__ __forceinline__ void st8(bf16 *p, bf16x8 v) { *(bf16x8 *)p = v; }
@@ -88,140 +91,285 @@ __global__ void __launch_bounds__(NTH) k_feat(int w, int h, const float *__restr
 }
 
 // ------------------------------------------------------------------------------------------- implicit-GEMM conv 3x3
+// K's order. Input channels go by slabs of 32 (the last what is left: 8 or 16); within a slab by row tap ty, then the
+// (column tap tx, channel octet) pairs, tx-major, four pairs of eight channels to a chunk of 32, the last chunk's missing
+// pairs zero. A chunk holds one row tap alone, so the pixels' operand of an input row serves all three output rows
+// around it.
+__host__ __device__ constexpr int conv_chunks(int sc) { return (3 * (sc / 8) + 3) / 4; }
+__host__ __device__ constexpr int conv_kp(int cin) {
+    return cin / 32 * 3 * 32 * conv_chunks(32) + (cin % 32 ? 3 * 32 * conv_chunks(cin % 32) : 0);
+}
+// the tap (3 ty + tx) and channel of K index k, false for the padding
+__device__ inline bool conv_k(int cin, int k, int &tap, int &ci) {
+    const int per = 3 * 32 * conv_chunks(32);
+    int slab = k / per, sc = 32;
+    if (slab >= cin / 32) {
+        slab = cin / 32;
+        sc = cin % 32;
+    }
+    k -= slab * per;
+    const int oct = sc / 8, c32 = 32 * conv_chunks(sc), ty = k / c32, pair = (k - ty * c32) / 8;
+    if (pair >= 3 * oct) return false;
+    tap = 3 * ty + pair / oct;
+    ci = 32 * slab + 8 * (pair % oct) + k % 8;
+    return true;
+}
+
 struct ConvArgs {
     const bf16 *in;    // (H, W, CIN - cup): channels [cup, CIN)
-    const bf16 *up;    // (H/2, W/2, cup): channels [0, cup), nearest-upsampled; null when cup == 0
+    const bf16 *up;    // (H/2, W/2, cup): channels [0, cup), nearest-upsampled; null when cup == 0 (a multiple of 32)
     const bf16 *mask;  // (H, W, CIN): entries whose mask is not > 0 read as zero; or null (only with cup == 0)
-    const bf16 *wt;    // (COUT, KP), k = tap * CIN + ci, zero past 9 CIN
+    const bf16 *wt;    // (COUT, conv_kp(CIN))
     const float *bias; // (COUT) or null
     bf16 *out;         // (H, W, COUT)
     int H, W, cup, relu;
+    bf16 *half = nullptr;  // CONV_POOL, CONV_SPLIT: the half-resolution output
+    // CONV_OUT: zn = (b + w . out) s d^-1/2, z = zadd + zn and/or err = zn - e (each null when not wanted)
+    const float *wout = nullptr, *scal = nullptr, *dis = nullptr, *zadd = nullptr, *e = nullptr;
+    float *z = nullptr, *err = nullptr;
 };
 
-// A block computes a tile of TW x TH pixels (a row of TW per wave, two 16-pixel MFMA tiles) x all COUT channels. Its
-// input -- rows y0 - 1 .. y0 + TH, columns x0 - 1 .. x0 + TW, every input channel, upsampled and concatenated or
-// masked as the layer reads it -- is staged once in LDS, so the nine taps read LDS instead of global memory. Lane l
-// of an MFMA holds A[m = l % 16][k = 8 (l / 16) + j], B[k = 8 (l / 16) + j][n = l % 16] and D[m = 4 (l / 16) + j]
-// [n = l % 16]; K runs over 9 taps x CIN channels in chunks of 32, zero past 9 CIN.
-#define TW 32
-#define TH 4
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(NTH) k_conv(ConvArgs a) {
-    constexpr int KP = (9 * CIN + 31) / 32 * 32;
-    constexpr int NT = COUT / 16;
-    constexpr int CP = CIN + 8;                    // pixel stride in LDS (bf16), staggering the banks
-    constexpr int RW = TW + 2, RH = TH + 2, OCT = CIN / 8;
-    static_assert(CIN % 8 == 0 && COUT % 16 == 0, "channel counts");
-    __shared__ __attribute__((aligned(16))) bf16 tile[RH * RW * CP];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c16 = lane & 15;
-    const int H = a.H, W = a.W, cup = a.cup, cs = CIN - cup;
-    const int x0 = blockIdx.x * TW, y0 = blockIdx.y * TH;
-    // stage the input tile (zero outside the image)
-    for (int t = threadIdx.x; t < RH * RW * OCT; t += NTH) {
-        const int o = t % OCT, px = t / OCT, lx = px % RW, ly = px / RW;
-        const int xx = x0 + lx - 1, yy = y0 + ly - 1, ci = 8 * o;
-        bf16x8 v = {};
-        if (xx >= 0 && xx < W && yy >= 0 && yy < H) {
-            if (ci < cup)
-                v = ld8(a.up + ((size_t)(yy >> 1) * (W >> 1) + (xx >> 1)) * cup + ci);
-            else
-                v = ld8(a.in + ((size_t)yy * W + xx) * cs + (ci - cup));
-            if (a.mask) {
-                const bf16x8 mv = ld8(a.mask + ((size_t)yy * W + xx) * CIN + ci);
+// What a convolution does with its result (rounded to BF16) besides storing it; the fused forms take an even H and W
+enum {
+    CONV_PLAIN,
+    CONV_POOL,   // also its 2x2 mean into half (H/2, W/2, COUT)
+    CONV_OUT,    // COUT = 16: also the output 1x1 layer and the scaling back to the system's units
+    CONV_SPLIT,  // a concat's gradient: channels [0, 32) (COUT = 48) or [0, 64) (96), summed over 2x2 pixels, into
+                 // half, the rest into out (H, W, COUT - those)
+    CONV_UNPOOL  // a pooled gradient: a quarter of it added to each of the four pixels of out (2 H, 2 W, COUT)
+};
+
+#define TW 64
+// One slab of a tile's input: SC channels from channel cb. The loads of a thread's items are issued together and the next
+// slab's go out before this one's products, whose time covers them; in LDS the pixel stride is an odd number of 16-byte
+// slots, so eight lanes' reads take eight slots. The tile is zero outside the image.
+template <int CIN, int R, int S> struct ConvSlab {
+    static constexpr int SC = 32 * S < CIN / 32 * 32 ? 32 : CIN % 32, OCT = SC / 8, CP = SC == 8 ? 8 : SC + 8;
+    static constexpr int RW = TW + 2, RH = R + 2, N = RH * RW * OCT, IT = (N + NTH - 1) / NTH, CB = 32 * S;
+    static constexpr int C = conv_chunks(SC), KB = S * 3 * 32 * conv_chunks(32);
+    bf16x8 v[IT];
+    __device__ inline void load(const ConvArgs &a, int x0, int y0) {
+        const int H = a.H, W = a.W, cup = a.cup, cs = CIN - cup;
 #pragma unroll
-                for (int j = 0; j < 8; j++)
-                    if (!((float)mv[j] > 0.0f)) v[j] = (bf16)0.0f;
-            }
-        }
-        st8(tile + (size_t)px * CP + ci, v);
-    }
-    __syncthreads();
-    f32x4 acc[2][NT];
+        for (int k = 0; k < IT; k++) {
+            const int t = threadIdx.x + k * NTH;
+            const int o = t % OCT, px = t / OCT, lx = px % RW, ly = px / RW;
+            const int xx = x0 + lx - 1, yy = y0 + ly - 1, ci = CB + 8 * o;
+            v[k] = bf16x8{};
+            if (t < N && xx >= 0 && xx < W && yy >= 0 && yy < H) {
+                if (ci < cup)
+                    v[k] = ld8(a.up + ((size_t)(yy >> 1) * (W >> 1) + (xx >> 1)) * cup + ci);
+                else
+                    v[k] = ld8(a.in + ((size_t)yy * W + xx) * cs + (ci - cup));
+                if (a.mask) {
+                    const bf16x8 mv = ld8(a.mask + ((size_t)yy * W + xx) * CIN + ci);
 #pragma unroll
-    for (int m = 0; m < 2; m++)
-#pragma unroll
-        for (int t = 0; t < NT; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int kc = 0; kc < KP; kc += 32) {
-        const int k0 = kc + 8 * g;
-        const int tap = k0 / CIN, ci = k0 - tap * CIN;
-        const int ty = tap / 3, tx = tap - 3 * ty;
-        bf16x8 bv[NT];
-#pragma unroll
-        for (int t = 0; t < NT; t++) bv[t] = ld8(a.wt + (size_t)(t * 16 + c16) * KP + k0);
-#pragma unroll
-        for (int m = 0; m < 2; m++) {
-            bf16x8 av = {};
-            if (tap < 9) av = ld8(tile + (size_t)((wave + ty) * RW + 16 * m + c16 + tx) * CP + ci);
-#pragma unroll
-            for (int t = 0; t < NT; t++)
-                acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[t], acc[m][t], 0, 0, 0);
-        }
-    }
-    const int y = y0 + wave;
-    if (y >= H) return;
-#pragma unroll
-    for (int m = 0; m < 2; m++)
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const int co = t * 16 + c16;
-            const float b = a.bias ? a.bias[co] : 0.0f;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int x = x0 + 16 * m + 4 * g + j;
-                if (x < W) {
-                    float v = acc[m][t][j] + b;
-                    if (a.relu) v = fmaxf(v, 0.0f);
-                    a.out[((size_t)y * W + x) * COUT + co] = (bf16)v;
+                    for (int j = 0; j < 8; j++)
+                        if (!((float)mv[j] > 0.0f)) v[k][j] = (bf16)0.0f;
                 }
             }
         }
-}
-
-template <int CIN, int COUT> static void conv(hipStream_t s, const ConvArgs &a) {
-    const dim3 grid((a.W + TW - 1) / TW, (a.H + TH - 1) / TH);
-    hipLaunchKernelGGL((k_conv<CIN, COUT>), grid, dim3(NTH), 0, s, a);
-}
-
-// 2x2 mean, one thread per (output pixel, channel octet)
-__global__ void __launch_bounds__(NTH) k_pool(const bf16 *__restrict__ in, int H, int W, int C, bf16 *__restrict__ out) {
-    const int Ho = H / 2, Wo = W / 2, oct = C / 8;
-    const int idx = blockIdx.x * NTH + threadIdx.x;
-    if (idx >= Ho * Wo * oct) return;
-    const int o = idx % oct, p = idx / oct, Y = p / Wo, X = p - Y * Wo;
-    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int dy = 0; dy < 2; dy++)
-#pragma unroll
-        for (int dx = 0; dx < 2; dx++) {
-            const bf16x8 v = ld8(in + ((size_t)(2 * Y + dy) * W + 2 * X + dx) * C + 8 * o);
-#pragma unroll
-            for (int j = 0; j < 8; j++) s[j] += (float)v[j];
-        }
-    bf16x8 r;
-#pragma unroll
-    for (int j = 0; j < 8; j++) r[j] = (bf16)(0.25f * s[j]);
-    st8(out + (size_t)p * C + 8 * o, r);
-}
-
-// the 1x1 output layer and the scaling back to the system's units: zn = (b + w . d1) s d^-1/2;
-// z = zadd + zn and/or err = zn - e
-__global__ void __launch_bounds__(NTH) k_out(int n, const bf16 *__restrict__ d1, const float *__restrict__ wout,
-                                             const float *scal, const float *__restrict__ dis,
-                                             const float *__restrict__ zadd, float *__restrict__ z,
-                                             const float *__restrict__ e, float *__restrict__ err) {
-    const float s = scal[0];
-    float wv[17];
-#pragma unroll
-    for (int c = 0; c < 17; c++) wv[c] = wout[c];
-    for (int i = blockIdx.x * NTH + threadIdx.x; i < n; i += gridDim.x * NTH) {
-        const bf16x8 a = ld8(d1 + (size_t)16 * i), b = ld8(d1 + (size_t)16 * i + 8);
-        float o = wv[16];
-#pragma unroll
-        for (int j = 0; j < 8; j++) o += wv[j] * (float)a[j] + wv[8 + j] * (float)b[j];
-        const float zn = o * s * dis[i];
-        if (err) err[i] = zn - e[i];
-        if (z) z[i] = (zadd ? zadd[i] : 0.0f) + zn;
     }
+    __device__ inline void store(bf16 *tile) const {
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const int t = threadIdx.x + k * NTH;
+            if (t < N) st8(tile + (t / OCT) * CP + 8 * (t % OCT), v[k]);
+        }
+    }
+    // chunk c's weights for the three row taps
+    template <int NT> static __device__ inline void weights(const bf16 *wt, int c, bf16x8 (&w)[3][NT]) {
+        const int g = (threadIdx.x & 63) >> 4, c16 = threadIdx.x & 15;
+#pragma unroll
+        for (int ty = 0; ty < 3; ty++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                w[ty][t] = ld8(wt + (size_t)(t * 16 + c16) * conv_kp(CIN) + KB + (ty * C + c) * 32 + 8 * g);
+    }
+    // every chunk's products, the wave walking its R + 2 input rows, each row's pixels read once and used by up to three
+    // output rows, the next chunk's weights loading meanwhile. Lane l of an MFMA holds A[m = l % 16][k = 8 (l / 16) + j],
+    // B[k = 8 (l / 16) + j][n = l % 16] and D[m = 4 (l / 16) + j][n = l % 16]: m the output channel, n the pixel, so a
+    // lane ends with four consecutive channels of one pixel. A padded pair reads the slab's first pair (inside the
+    // stencil) against zero weights.
+    template <int NT>
+    static __device__ inline void products(const bf16 *wt, const bf16 *tile, bf16x8 (&w)[3][NT], f32x4 (&acc)[R][NT]) {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c16 = lane & 15;
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const int pair = 4 * c + g < 3 * OCT ? 4 * c + g : 0, tx = pair / OCT, o = pair % OCT;
+            const bf16 *px = tile + (16 * wave + c16 + tx) * CP + 8 * o;
+            bf16x8 wn[3][NT];
+            if (c + 1 < C) weights<NT>(wt, c + 1, wn);
+#pragma unroll
+            for (int i = 0; i < RH; i++) {
+                const bf16x8 p = ld8(px + i * RW * CP);
+#pragma unroll
+                for (int ty = 0; ty < 3; ty++) {
+                    const int r = i - ty;
+                    if (r < 0 || r >= R) continue;
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+                        acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[ty][t], p, acc[r][t], 0, 0, 0);
+                }
+            }
+            if (c + 1 < C)
+#pragma unroll
+                for (int ty = 0; ty < 3; ty++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++) w[ty][t] = wn[ty][t];
+        }
+    }
+};
+
+template <int CIN, int R, int NT, int S>
+__device__ inline void conv_slabs(const ConvArgs &a, bf16 *tile, int x0, int y0, const ConvSlab<CIN, R, S> &slab,
+                                  f32x4 (&acc)[R][NT]) {
+    using SL = ConvSlab<CIN, R, S>;
+    bf16x8 w[3][NT];
+    SL::template weights<NT>(a.wt, 0, w);
+    slab.store(tile);
+    __syncthreads();
+    if constexpr (SL::CB + SL::SC < CIN) {
+        ConvSlab<CIN, R, S + 1> next;
+        next.load(a, x0, y0);
+        SL::template products<NT>(a.wt, tile, w, acc);
+        __syncthreads();  // the slab is read
+        conv_slabs<CIN, R, NT, S + 1>(a, tile, x0, y0, next, acc);
+    } else {
+        SL::template products<NT>(a.wt, tile, w, acc);
+    }
+}
+
+// the value of the lane beside (lane ^ 1), without the LDS unit
+__device__ __forceinline__ float beside(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
+}
+
+// a and b summed over pairs of 16-lane rows, and over the two halves: rows (a0 + a1, b0 + b1, a2 + a3, b2 + b3), and
+// halves (a.low + a.high, b.low + b.high)
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float swap16_add(float a, float b) {
+    const u32x2 r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
+                                                     false, false);
+    const unsigned lo = r[0], hi = r[1];
+    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+__device__ __forceinline__ float swap32_add(float a, float b) {
+    const u32x2 r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
+                                                     false, false);
+    const unsigned lo = r[0], hi = r[1];
+    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+
+// A block computes TW x R pixels (a wave 16 columns of every row) x all COUT channels. Measured at 2048^2 (nine tap reads
+// of LDS per product row and COUT-scattered 2-byte stores before): 48 -> 16 channels 296 -> 136 us, 96 -> 32 at 1024^2
+// 168 -> 92, 64 -> 64 at 512^2 81 -> 56; the wide-image 16-channel layers are bound by HBM (8 -> 16: 38 us, 5.3 TB/s).
+template <int CIN, int COUT, int R, int EPI>
+__global__ void __launch_bounds__(NTH) k_conv(ConvArgs a) {
+    constexpr int NT = COUT / 16, FULL = CIN / 32, REST = CIN % 32;
+    constexpr int CPM = FULL ? 40 : REST == 8 ? 8 : REST + 8;
+    constexpr int SUMMED = EPI == CONV_SPLIT ? COUT / 3 * 2 : 0;  // the concat's upsampled channels
+    static_assert(CIN % 8 == 0 && COUT % 16 == 0 && R % 2 == 0, "channel counts, rows");
+    static_assert(EPI != CONV_OUT || COUT == 16, "the output layer reads 16 channels");
+    __shared__ __attribute__((aligned(16))) bf16 tile[(R + 2) * (TW + 2) * CPM];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c16 = lane & 15;
+    const int blk = xcd_tile(), x0 = (blk % gridDim.x) * TW, y0 = (blk / gridDim.x) * R;
+    f32x4 acc[R][NT];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    {
+        ConvSlab<CIN, R, 0> first;
+        first.load(a, x0, y0);
+        conv_slabs<CIN, R, NT, 0>(a, tile, x0, y0, first, acc);
+    }
+    const int x = x0 + 16 * wave + c16, H = a.H, W = a.W;
+    if (x0 + 16 * wave >= W) return;  // the whole wave is past the image
+    float o[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) o[r] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const int co = t * 16 + 4 * g;
+        const bool summed = t * 16 < SUMMED;
+        float b[4] = {0.0f, 0.0f, 0.0f, 0.0f}, wv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (a.bias) b[j] = a.bias[co + j];
+            if (EPI == CONV_OUT) wv[j] = a.wout[co + j];
+        }
+        bf16x4 s[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const bool in = x < W && y0 + r < H;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                float v = acc[r][t][j] + b[j];
+                if (a.relu) v = fmaxf(v, 0.0f);
+                s[r][j] = (bf16)v;
+                if (EPI == CONV_OUT) o[r] += wv[j] * (float)s[r][j];
+            }
+            if (EPI == CONV_UNPOOL) {
+                if (in)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        bf16x4 *p = (bf16x4 *)(a.out + ((size_t)(2 * (y0 + r) + (q >> 1)) * (2 * W) + 2 * x + (q & 1)) * COUT + co);
+                        bf16x4 f = *p;
+#pragma unroll
+                        for (int j = 0; j < 4; j++) f[j] = (bf16)((float)f[j] + 0.25f * (float)s[r][j]);
+                        *p = f;
+                    }
+            } else if (!summed && in) {
+                *(bf16x4 *)(a.out + ((size_t)(y0 + r) * W + x) * (COUT - SUMMED) + co - SUMMED) = s[r];
+            }
+        }
+        if (EPI == CONV_POOL || summed) {
+            constexpr int HC = EPI == CONV_POOL ? COUT : SUMMED;
+            const float f = EPI == CONV_POOL ? 0.25f : 1.0f;
+#pragma unroll
+            for (int r = 0; r < R; r += 2) {
+                bf16x4 h;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float v0 = (float)s[r][j], v1 = (float)s[r + 1][j];
+                    h[j] = (bf16)(f * (((v0 + beside(v0)) + v1) + beside(v1)));
+                }
+                if (!(c16 & 1) && x < W && y0 + r < H)
+                    *(bf16x4 *)(a.half + ((size_t)((y0 + r) >> 1) * (W >> 1) + (x >> 1)) * HC + co) = h;
+            }
+        }
+    }
+    if (EPI == CONV_OUT) {
+        const float s = a.scal[0], bo = a.wout[16];
+        // the four groups' sums of two or four rows joined by lane swaps, group g ending with row g (of two: g % 2)
+        constexpr int Q = R < 4 ? 2 : 4;
+#pragma unroll
+        for (int r0 = 0; r0 < R; r0 += Q) {
+            float v = swap16_add(o[r0], o[r0 + 1]);
+            v = swap32_add(v, Q == 4 ? swap16_add(o[r0 + Q - 2], o[r0 + Q - 1]) : v);
+            const int y = y0 + r0 + g;
+            if (g < Q && x < W && y < H) {
+                const size_t i = (size_t)y * W + x;
+                const float zn = (v + bo) * s * a.dis[i];
+                if (a.err) a.err[i] = zn - a.e[i];
+                if (a.z) a.z[i] = (a.zadd ? a.zadd[i] : 0.0f) + zn;
+            }
+        }
+    }
+}
+
+// Rows per wave: the more rows, the fewer reads of LDS and of the halo per product (R + 2 for 3 R NT products), as long
+// as the launch still fills the chip; wide outputs keep four (their accumulators and weights take the registers).
+template <int CIN, int COUT, int EPI = CONV_PLAIN> static void conv(hipStream_t s, const ConvArgs &a) {
+    auto blocks = [&](int r) { return ((a.W + TW - 1) / TW) * ((a.H + r - 1) / r); };
+    auto go = [&](auto kernel, int r) {
+        hipLaunchKernelGGL(kernel, dim3((a.W + TW - 1) / TW, (a.H + r - 1) / r), dim3(NTH), 0, s, a);
+    };
+    if constexpr (COUT <= 48)
+        if (blocks(8) >= CONV_FILL) return go(k_conv<CIN, COUT, 8, EPI>, 8);
+    if (blocks(4) >= CONV_FILL) return go(k_conv<CIN, COUT, 4, EPI>, 4);
+    go(k_conv<CIN, COUT, 2, EPI>, 2);
 }
 
 // ------------------------------------------------------------------------------------------------------- training
@@ -379,48 +527,6 @@ __global__ void k_dw_reduce(const float *__restrict__ part, int nb, int cinp, in
         gb[o - nw] = (float)s;
 }
 
-// split the gradient of a concat(up(a), skip) input: g_up[Y][X][c] = sum over the 2x2 children (c < cup);
-// g_skip[p][c] = g[p][cup + c]
-__global__ void k_split_cat(const bf16 *__restrict__ g, int H, int W, int C, int cup, bf16 *__restrict__ gup,
-                            bf16 *__restrict__ gskip) {
-    const int idx = blockIdx.x * NTH + threadIdx.x;
-    const int cs = C - cup, Wo = W / 2, Ho = H / 2;
-    const int nup = Ho * Wo * (cup / 8), nsk = H * W * (cs / 8);
-    if (idx < nup) {
-        const int oc = cup / 8, o = idx % oc, p = idx / oc, Y = p / Wo, X = p - Y * Wo;
-        float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int dy = 0; dy < 2; dy++)
-#pragma unroll
-            for (int dx = 0; dx < 2; dx++) {
-                const bf16x8 v = ld8(g + ((size_t)(2 * Y + dy) * W + 2 * X + dx) * C + 8 * o);
-#pragma unroll
-                for (int j = 0; j < 8; j++) s[j] += (float)v[j];
-            }
-        bf16x8 r;
-#pragma unroll
-        for (int j = 0; j < 8; j++) r[j] = (bf16)s[j];
-        st8(gup + (size_t)p * cup + 8 * o, r);
-    } else if (idx < nup + nsk) {
-        const int k = idx - nup, oc = cs / 8, o = k % oc, p = k / oc;
-        st8(gskip + (size_t)p * cs + 8 * o, ld8(g + (size_t)p * C + cup + 8 * o));
-    }
-}
-
-// g_skip += pool_backward(g_pool): each fine pixel gets a quarter of its parent's gradient
-__global__ void k_add_pool_back(bf16 *__restrict__ gskip, const bf16 *__restrict__ gp, int H, int W, int C) {
-    const int idx = blockIdx.x * NTH + threadIdx.x;
-    const int oc = C / 8;
-    if (idx >= H * W * oc) return;
-    const int o = idx % oc, p = idx / oc, y = p / W, x = p - y * W;
-    const bf16x8 a = ld8(gskip + (size_t)p * C + 8 * o);
-    const bf16x8 b = ld8(gp + ((size_t)(y >> 1) * (W >> 1) + (x >> 1)) * C + 8 * o);
-    bf16x8 r;
-#pragma unroll
-    for (int j = 0; j < 8; j++) r[j] = (bf16)((float)a[j] + 0.25f * (float)b[j]);
-    st8(gskip + (size_t)p * C + 8 * o, r);
-}
-
 // Adam (Kingma and Ba 2015, Algorithm 1) on the FP32 master parameters
 __global__ void k_adam(int n, float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
                        float *__restrict__ v, float lr, float b1, float b2, float eps, float bc1, float bc2) {
@@ -433,20 +539,21 @@ __global__ void k_adam(int n, float *__restrict__ p, const float *__restrict__ g
     p[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
 }
 
-// the BF16 weight layouts of one layer from its FP32 (3, 3, cin, cout) master: forward (cout, kp) with
-// k = tap * cinp + ci, backward-data (cin, kpb) with k = tap' * cout + co and tap' = 8 - tap
+// the BF16 weight layouts of one layer from its FP32 (3, 3, cin, cout) master, K in k_conv's order: forward (cout, kp)
+// over the taps and input channels, backward-data (cin, kpb) over the mirrored taps and output channels
 __global__ void k_pack(const float *__restrict__ w, int cin, int cinp, int cout, int kp, int kpb, bf16 *__restrict__ wt,
                        bf16 *__restrict__ wb) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int nf = cout * kp, nbk = wb ? cin * kpb : 0;
+    int tap, c;
     if (i < nf) {
-        const int co = i / kp, k = i - co * kp, tap = k / cinp, ci = k - tap * cinp;
-        const float v = (tap < 9 && ci < cin) ? w[((size_t)tap * cin + ci) * cout + co] : 0.0f;
-        wt[i] = (bf16)v;
+        const int co = i / kp;
+        const bool in = conv_k(cinp, i - co * kp, tap, c) && c < cin;
+        wt[i] = (bf16)(in ? w[((size_t)tap * cin + c) * cout + co] : 0.0f);
     } else if (i < nf + nbk) {
-        const int j = i - nf, ci = j / kpb, k = j - ci * kpb, tb = k / cout, co = k - tb * cout;
-        const float v = tb < 9 ? w[((size_t)(8 - tb) * cin + ci) * cout + co] : 0.0f;
-        wb[j] = (bf16)v;
+        const int j = i - nf, ci = j / kpb;
+        const bool in = conv_k(cout, j - ci * kpb, tap, c);
+        wb[j] = (bf16)(in ? w[((size_t)(8 - tap) * cin + ci) * cout + c] : 0.0f);
     }
 }
 
@@ -460,8 +567,8 @@ Net::~Net() {
         if (l.wt) (void)hipFree(l.wt);
         if (l.wb) (void)hipFree(l.wb);
     }
-    void *ps[] = {params, grads, m, v, x, e1a, e1, p1, e2a, e2, p2, e3a, e3, d2a, d2, d1a, d1, g_d1, g_d1a, g_cat1,
-                  g_d2, g_d2a, g_cat2, g_e3, g_e3a, g_p2, g_e2, g_e2a, g_p1, g_e1, g_e1a, dis, err, aerr, gout, wpart,
+    void *ps[] = {params, grads, m, v, x, e1a, e1, p1, e2a, e2, p2, e3a, e3, d2a, d2, d1a, d1, g_d1, g_d1a,
+                  g_d2, g_d2a, g_e3, g_e3a, g_e2, g_e2a, g_e1, g_e1a, dis, err, aerr, gout, wpart,
                   part, lpart, opart, scal};
     for (void *q : ps)
         if (q) (void)hipFree(q);
@@ -485,8 +592,8 @@ int Net::init(int mw, int mh) {
         l.cin = LAYER_SHAPE[i][0];
         l.cout = LAYER_SHAPE[i][1];
         l.cinp = i == E1A ? 8 : l.cin;
-        l.kp = (9 * l.cinp + 31) / 32 * 32;
-        l.kpb = (9 * l.cout + 31) / 32 * 32;
+        l.kp = conv_kp(l.cinp);
+        l.kpb = conv_kp(l.cout);
         l.w_off = off;
         off += (size_t)9 * l.cin * l.cout;
         l.b_off = off;
@@ -573,7 +680,8 @@ static ConvArgs cargs(const bf16 *in, const bf16 *up, int cup, const bf16 *mask,
 
 static int grid_of(size_t n) { return (int)std::min<size_t>(NB_FEAT, (n + NTH - 1) / NTH); }
 
-int Net::forward(int w, int h, const float *own, const float *kx, const float *ky, const float *r, hipStream_t s) {
+int Net::forward(int w, int h, const float *own, const float *kx, const float *ky, const float *r, const float *zadd,
+                 float *z, const float *e, float *err, hipStream_t s) {
     if (w <= 0 || h <= 0 || w % 4 || h % 4 || w > max_w || h > max_h || (size_t)w * h > (size_t)max_w * max_h)
         return fail(SR_ERR_ARGUMENT, "network input size outside the multiples of 4 it was created for");
     if (!own || !kx || !ky || !r) return fail(SR_ERR_ARGUMENT, "network: null system array");
@@ -587,18 +695,28 @@ int Net::forward(int w, int h, const float *own, const float *kx, const float *k
     hipLaunchKernelGGL(k_feat, dim3(nb), dim3(NTH), 0, s, w, h, own, kx, ky, r, (const double *)part, nb, x, dis, scal);
     const int w2 = w / 2, h2 = h / 2, w4 = w / 4, h4 = h / 4;
     auto B = [&](int i) { return (const float *)(params + L[i].b_off); };
+    auto with_half = [](ConvArgs a, bf16 *half) {
+        a.half = half;
+        return a;
+    };
     conv<8, 16>(s, cargs(x, nullptr, 0, nullptr, L[E1A].wt, B(E1A), e1a, h, w, 1));
-    conv<16, 16>(s, cargs(e1a, nullptr, 0, nullptr, L[E1].wt, B(E1), e1, h, w, 1));
-    hipLaunchKernelGGL(k_pool, dim3((n / 4 * 2 + NTH - 1) / NTH), dim3(NTH), 0, s, e1, h, w, 16, p1);
+    conv<16, 16, CONV_POOL>(s, with_half(cargs(e1a, nullptr, 0, nullptr, L[E1].wt, B(E1), e1, h, w, 1), p1));
     conv<16, 32>(s, cargs(p1, nullptr, 0, nullptr, L[E2A].wt, B(E2A), e2a, h2, w2, 1));
-    conv<32, 32>(s, cargs(e2a, nullptr, 0, nullptr, L[E2].wt, B(E2), e2, h2, w2, 1));
-    hipLaunchKernelGGL(k_pool, dim3(((size_t)w4 * h4 * 4 + NTH - 1) / NTH), dim3(NTH), 0, s, e2, h2, w2, 32, p2);
+    conv<32, 32, CONV_POOL>(s, with_half(cargs(e2a, nullptr, 0, nullptr, L[E2].wt, B(E2), e2, h2, w2, 1), p2));
     conv<32, 64>(s, cargs(p2, nullptr, 0, nullptr, L[E3A].wt, B(E3A), e3a, h4, w4, 1));
     conv<64, 64>(s, cargs(e3a, nullptr, 0, nullptr, L[E3].wt, B(E3), e3, h4, w4, 1));
     conv<96, 32>(s, cargs(e2, e3, 64, nullptr, L[D2A].wt, B(D2A), d2a, h2, w2, 1));
     conv<32, 32>(s, cargs(d2a, nullptr, 0, nullptr, L[D2].wt, B(D2), d2, h2, w2, 1));
     conv<48, 16>(s, cargs(e1, d2, 32, nullptr, L[D1A].wt, B(D1A), d1a, h, w, 1));
-    conv<16, 16>(s, cargs(d1a, nullptr, 0, nullptr, L[D1].wt, B(D1), d1, h, w, 1));
+    ConvArgs last = cargs(d1a, nullptr, 0, nullptr, L[D1].wt, B(D1), d1, h, w, 1);
+    last.wout = params + out_off;
+    last.scal = scal;
+    last.dis = dis;
+    last.zadd = zadd;
+    last.z = z;
+    last.e = e;
+    last.err = err;
+    conv<16, 16, CONV_OUT>(s, last);
     SR_HIP(hipGetLastError());
     return SR_OK;
 }
@@ -606,13 +724,7 @@ int Net::forward(int w, int h, const float *own, const float *kx, const float *k
 int Net::apply(int w, int h, const float *own, const float *kx, const float *ky, const float *r, const float *zadd,
                float *z, hipStream_t s) {
     if (!z) return fail(SR_ERR_ARGUMENT, "network: null output");
-    SR_TRY(forward(w, h, own, kx, ky, r, s));
-    const size_t n = (size_t)w * h;
-    hipLaunchKernelGGL(k_out, dim3(grid_of(n)), dim3(NTH), 0, s, (int)n, (const bf16 *)d1,
-                       (const float *)(params + out_off), (const float *)scal, (const float *)dis, zadd, z,
-                       (const float *)nullptr, (float *)nullptr);
-    SR_HIP(hipGetLastError());
-    return SR_OK;
+    return forward(w, h, own, kx, ky, r, zadd, z, nullptr, nullptr, s);
 }
 
 template <int CIN, int COUT>
@@ -633,16 +745,12 @@ int Net::loss_grad(int w, int h, const float *own, const float *kx, const float 
         const size_t n = (size_t)max_w * max_h, n2 = n / 4, n4 = n / 16;
         SR_TRY(dalloc(&g_d1, 16 * n));
         SR_TRY(dalloc(&g_d1a, 16 * n));
-        SR_TRY(dalloc(&g_cat1, 48 * n));
         SR_TRY(dalloc(&g_d2, 32 * n2));
         SR_TRY(dalloc(&g_d2a, 32 * n2));
-        SR_TRY(dalloc(&g_cat2, 96 * n2));
         SR_TRY(dalloc(&g_e3, 64 * n4));
         SR_TRY(dalloc(&g_e3a, 64 * n4));
-        SR_TRY(dalloc(&g_p2, 32 * n4));
         SR_TRY(dalloc(&g_e2, 32 * n2));
         SR_TRY(dalloc(&g_e2a, 32 * n2));
-        SR_TRY(dalloc(&g_p1, 16 * n2));
         SR_TRY(dalloc(&g_e1, 16 * n));
         SR_TRY(dalloc(&g_e1a, 16 * n));
         SR_TRY(dalloc(&err, n));
@@ -652,12 +760,10 @@ int Net::loss_grad(int w, int h, const float *own, const float *kx, const float 
         SR_TRY(dalloc(&opart, 17 * NB_FEAT));
         SR_TRY(dalloc(&wpart, (size_t)DW_BLOCKS * (9 * 64 * 64 + 64)));
     }
-    SR_TRY(forward(w, h, own, kx, ky, r, s));
+    SR_TRY(forward(w, h, own, kx, ky, r, nullptr, nullptr, e, err, s));
     const size_t n = (size_t)w * h;
     const int nb = grid_of(n);
     const int w2 = w / 2, h2 = h / 2, w4 = w / 4, h4 = h / 4;
-    hipLaunchKernelGGL(k_out, dim3(nb), dim3(NTH), 0, s, (int)n, (const bf16 *)d1, (const float *)(params + out_off),
-                       (const float *)scal, (const float *)dis, (const float *)nullptr, (float *)nullptr, e, err);
     hipLaunchKernelGGL(k_loss, dim3(nb), dim3(NTH), 0, s, w, h, own, kx, ky, (const float *)err, e, aerr, lpart);
     hipLaunchKernelGGL(k_out_back, dim3(nb), dim3(NTH), 0, s, (int)n, (const float *)aerr, (const double *)lpart, nb,
                        (const float *)scal, (const float *)dis, (const bf16 *)d1, (const float *)(params + out_off),
@@ -667,36 +773,26 @@ int Net::loss_grad(int w, int h, const float *own, const float *kx, const float 
     dw<16, 16>(s, d1a, nullptr, 0, g_d1, d1, h, w, wpart, L[D1], grads);
     conv<16, 16>(s, cargs(g_d1, nullptr, 0, d1, L[D1].wb, nullptr, g_d1a, h, w, 0));
     dw<48, 16>(s, e1, d2, 32, g_d1a, d1a, h, w, wpart, L[D1A], grads);
-    conv<16, 48>(s, cargs(g_d1a, nullptr, 0, d1a, L[D1A].wb, nullptr, g_cat1, h, w, 0));
-    {
-        const int tot = h2 * w2 * 4 + h * w * 2;
-        hipLaunchKernelGGL(k_split_cat, dim3((tot + NTH - 1) / NTH), dim3(NTH), 0, s, (const bf16 *)g_cat1, h, w, 48,
-                           32, g_d2, g_e1);
-    }
+    ConvArgs cat = cargs(g_d1a, nullptr, 0, d1a, L[D1A].wb, nullptr, g_e1, h, w, 0);
+    cat.half = g_d2;
+    conv<16, 48, CONV_SPLIT>(s, cat);
     // decoder, level 2
     dw<32, 32>(s, d2a, nullptr, 0, g_d2, d2, h2, w2, wpart, L[D2], grads);
     conv<32, 32>(s, cargs(g_d2, nullptr, 0, d2, L[D2].wb, nullptr, g_d2a, h2, w2, 0));
     dw<96, 32>(s, e2, e3, 64, g_d2a, d2a, h2, w2, wpart, L[D2A], grads);
-    conv<32, 96>(s, cargs(g_d2a, nullptr, 0, d2a, L[D2A].wb, nullptr, g_cat2, h2, w2, 0));
-    {
-        const int tot = h4 * w4 * 8 + h2 * w2 * 4;
-        hipLaunchKernelGGL(k_split_cat, dim3((tot + NTH - 1) / NTH), dim3(NTH), 0, s, (const bf16 *)g_cat2, h2, w2, 96,
-                           64, g_e3, g_e2);
-    }
+    cat = cargs(g_d2a, nullptr, 0, d2a, L[D2A].wb, nullptr, g_e2, h2, w2, 0);
+    cat.half = g_e3;
+    conv<32, 96, CONV_SPLIT>(s, cat);
     // encoder, level 3
     dw<64, 64>(s, e3a, nullptr, 0, g_e3, e3, h4, w4, wpart, L[E3], grads);
     conv<64, 64>(s, cargs(g_e3, nullptr, 0, e3, L[E3].wb, nullptr, g_e3a, h4, w4, 0));
     dw<32, 64>(s, p2, nullptr, 0, g_e3a, e3a, h4, w4, wpart, L[E3A], grads);
-    conv<64, 32>(s, cargs(g_e3a, nullptr, 0, e3a, L[E3A].wb, nullptr, g_p2, h4, w4, 0));
-    hipLaunchKernelGGL(k_add_pool_back, dim3((h2 * w2 * 4 + NTH - 1) / NTH), dim3(NTH), 0, s, g_e2, (const bf16 *)g_p2,
-                       h2, w2, 32);
+    conv<64, 32, CONV_UNPOOL>(s, cargs(g_e3a, nullptr, 0, e3a, L[E3A].wb, nullptr, g_e2, h4, w4, 0));
     // encoder, level 2
     dw<32, 32>(s, e2a, nullptr, 0, g_e2, e2, h2, w2, wpart, L[E2], grads);
     conv<32, 32>(s, cargs(g_e2, nullptr, 0, e2, L[E2].wb, nullptr, g_e2a, h2, w2, 0));
     dw<16, 32>(s, p1, nullptr, 0, g_e2a, e2a, h2, w2, wpart, L[E2A], grads);
-    conv<32, 16>(s, cargs(g_e2a, nullptr, 0, e2a, L[E2A].wb, nullptr, g_p1, h2, w2, 0));
-    hipLaunchKernelGGL(k_add_pool_back, dim3((h * w * 2 + NTH - 1) / NTH), dim3(NTH), 0, s, g_e1, (const bf16 *)g_p1, h,
-                       w, 16);
+    conv<32, 16, CONV_UNPOOL>(s, cargs(g_e2a, nullptr, 0, e2a, L[E2A].wb, nullptr, g_e1, h2, w2, 0));
     // encoder, level 1
     dw<16, 16>(s, e1a, nullptr, 0, g_e1, e1, h, w, wpart, L[E1], grads);
     conv<16, 16>(s, cargs(g_e1, nullptr, 0, e1, L[E1].wb, nullptr, g_e1a, h, w, 0));

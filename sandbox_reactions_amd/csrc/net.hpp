@@ -13,10 +13,10 @@ typedef __bf16 bf16;
 struct NetLayer {
     int cin, cout;   // real channels
     int cinp;        // input channels as stored (the first layer's 3 features padded to 8)
-    int kp, kpb;     // forward K = 9 cinp and backward-data K = 9 cout, each rounded up to 32
+    int kp, kpb;     // forward K over cinp and backward-data K over cout, padded to the convolution's chunks
     size_t w_off, b_off;
-    bf16 *wt = nullptr;  // forward weights (cout, kp), k = tap * cinp + ci
-    bf16 *wb = nullptr;  // backward-data weights (cin, kpb), k = tap' * cout + co, taps mirrored
+    bf16 *wt = nullptr;  // forward weights (cout, kp)
+    bf16 *wb = nullptr;  // backward-data weights (cin, kpb), taps mirrored
 };
 
 struct NetStats {
@@ -44,7 +44,9 @@ class Net {
     double flops_per_apply(int w, int h) const;
 
   private:
-    int forward(int w, int h, const float *own, const float *kx, const float *ky, const float *r, hipStream_t s);
+    // the output layer's z (zadd added) and/or its difference from e, each null when not wanted
+    int forward(int w, int h, const float *own, const float *kx, const float *ky, const float *r, const float *zadd,
+                float *z, const float *e, float *err, hipStream_t s);
     int pack(hipStream_t s);
     int max_w = 0, max_h = 0;
     std::vector<NetLayer> L;
@@ -56,9 +58,8 @@ class Net {
     bf16 *x = nullptr, *e1a = nullptr, *e1 = nullptr, *p1 = nullptr, *e2a = nullptr, *e2 = nullptr, *p2 = nullptr,
          *e3a = nullptr, *e3 = nullptr, *d2a = nullptr, *d2 = nullptr, *d1a = nullptr, *d1 = nullptr;
     // gradients of the activations
-    bf16 *g_d1 = nullptr, *g_d1a = nullptr, *g_cat1 = nullptr, *g_d2 = nullptr, *g_d2a = nullptr,
-         *g_cat2 = nullptr, *g_e3 = nullptr, *g_e3a = nullptr, *g_p2 = nullptr, *g_e2 = nullptr, *g_e2a = nullptr,
-         *g_p1 = nullptr, *g_e1 = nullptr, *g_e1a = nullptr;
+    bf16 *g_d1 = nullptr, *g_d1a = nullptr, *g_d2 = nullptr, *g_d2a = nullptr, *g_e3 = nullptr, *g_e3a = nullptr,
+         *g_e2 = nullptr, *g_e2a = nullptr, *g_e1 = nullptr, *g_e1a = nullptr;
     float *dis = nullptr, *err = nullptr, *aerr = nullptr, *gout = nullptr, *wpart = nullptr;
     double *part = nullptr, *lpart = nullptr, *opart = nullptr, *host = nullptr;
     float *scal = nullptr;   // s (the residual's scale) and the mean log coupling, on the device

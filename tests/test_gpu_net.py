@@ -262,3 +262,95 @@ def test_trained_network_gains_over_the_v_cycle_alone(gpu_lib):
           f"learned without fallback {it_n}", flush=True)
     assert rel_l <= 1e-8 and rel_n <= 1e-8 and not fb_n and li_n == it_n
     assert it_l <= it_p + 20
+
+
+# Sizes at which the convolution's tiles of 64 pixels x 2, 4 or 8 rows all run, each with ragged edges: 68 x 36 (two rows
+# everywhere), 516 x 260 (four at full resolution), 2052 x 1028 (eight, eight and four).
+@pytest.mark.parametrize("w,h", [(68, 36), (516, 260), (2052, 1028)])
+def test_layers_match_over_every_tile_height(gpu_lib, w, h):
+    """Every layer, the pooled means and the output from the GPU's own inputs, in FP32 on the device: a layer's BF16
+    output is within half an ulp (2^-9 of its size, 2^-8 allowing the FP32 sums' order to tip a rounding)."""
+    import torch
+    import sandbox_reactions_amd as sr
+    print(f"net layers {w}x{h}", flush=True)
+    p = random_params(21)
+    net = sr.Net(w, h, p)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(22)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    own, kx, ky = rnd(h, w).exp(), rnd(h, w + 1).exp(), rnd(h + 1, w).exp()
+    r, z = rnd(h, w), torch.empty(h, w, device="cuda")
+    net.apply(own, kx, ky, r, z)
+    A = {k: torch.tensor(net.activation(k, w, h), device="cuda") for k in
+         ["x", "e1a", "e1", "p1", "e2a", "e2", "p2", "e3a", "e3", "d2a", "d2", "d1a", "d1"]}
+    up = lambda a: a.repeat_interleave(2, 0).repeat_interleave(2, 1)
+    for name, inp in [("e1a", A["x"][:, :, :3]), ("e1", A["e1a"]), ("e2a", A["p1"]), ("e2", A["e2a"]),
+                      ("e3a", A["p2"]), ("e3", A["e3a"]), ("d2a", torch.cat([up(A["e3"]), A["e2"]], 2)),
+                      ("d2", A["d2a"]), ("d1a", torch.cat([up(A["d2"]), A["e1"]], 2)), ("d1", A["d1a"])]:
+        wt = torch.tensor(bf16(p[name + ".w"]), device="cuda").float()
+        hh, ww, ci = inp.shape
+        padded = torch.zeros(hh + 2, ww + 2, ci, device="cuda")
+        padded[1:-1, 1:-1] = inp
+        ref = torch.tensor(p[name + ".b"], device="cuda").expand(hh * ww, -1).clone()
+        for t in range(9):
+            ref += padded[t // 3:t // 3 + hh, t % 3:t % 3 + ww].reshape(hh * ww, ci) @ wt[t // 3, t % 3]
+        ref = ref.clamp(min=0.0).reshape(hh, ww, -1)
+        err = float(((A[name] - ref).abs() - 2.0 ** -8 * ref.abs()).max()) / float(ref.max())
+        assert err <= 1e-5, (name, err)
+    for name, src in (("p1", "e1"), ("p2", "e2")):
+        a = A[src]
+        mean = 0.25 * (a[::2, ::2] + a[::2, 1::2] + a[1::2, ::2] + a[1::2, 1::2])
+        assert torch.equal(A[name], mean.bfloat16().float()), name
+    ks = kx[:, :-1] + kx[:, 1:] + ky[:-1] + ky[1:]
+    dis = (own + ks).double().rsqrt()
+    s = (r.double() * dis).square().mean().sqrt()
+    ref = (A["d1"].double() @ torch.tensor(p["out.w"], device="cuda").double() + float(p["out.b"][0])) * s * dis
+    assert float((z - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
+
+
+# one tile row, ragged tiles in both axes (32 x 4), and more tiles than blocks (each block walks five)
+@pytest.mark.parametrize("w,h", [(32, 4), (68, 36), (516, 260)])
+def test_last_layers_weight_gradient_over_ragged_tiles(gpu_lib, w, h):
+    """dW and db of the last 3x3 layer from its own input and output: ga = dL/d(out) w_out where the output is positive,
+    stored in BF16 (2^-9 of each term, so at most that of the sum of the terms' sizes)."""
+    import torch
+    import sandbox_reactions_amd as sr
+    from sandbox_reactions_amd import net as N
+    print(f"net dW {w}x{h}", flush=True)
+    p = random_params(23)
+    net = sr.Net(w, h, p)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(24)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    own, kx, ky = rnd(h, w).exp(), rnd(h, w + 1).exp(), rnd(h + 1, w).exp()
+    kx[:, 0] = kx[:, w] = 0.0
+    ky[0] = ky[h] = 0.0
+    r, e, z = rnd(h, w), rnd(h, w), torch.empty(h, w, device="cuda")
+    net.apply(own, kx, ky, r, z)
+    net.loss_grad(own, kx, ky, r, e)
+    g = N.unflatten(net.grads().astype(np.float64))
+    A = {k: torch.tensor(net.activation(k, w, h), device="cuda").double() for k in ("d1a", "d1")}
+    ks = (kx[:, :-1] + kx[:, 1:] + ky[:-1] + ky[1:]).double()
+
+    def op(v):
+        out = own.double() * v
+        dx, dy = kx[:, 1:-1].double() * (v[:, 1:] - v[:, :-1]), ky[1:-1].double() * (v[1:] - v[:-1])
+        out[:, :-1] -= dx
+        out[:, 1:] += dx
+        out[:-1] -= dy
+        out[1:] += dy
+        return out
+
+    dis = (own.double() + ks).rsqrt()
+    s = (r.double() * dis).square().mean().sqrt()
+    gout = 2.0 * op(z.double() - e.double()) / (e.double() * op(e.double())).sum() * s * dis
+    ga = gout[:, :, None] * torch.tensor(p["out.w"], device="cuda").double() * (A["d1"] > 0)
+    padded = torch.zeros(h + 2, w + 2, 16, device="cuda", dtype=torch.float64)
+    padded[1:-1, 1:-1] = A["d1a"]
+    for t in range(9):
+        x = padded[t // 3:t // 3 + h, t % 3:t % 3 + w].reshape(-1, 16)
+        ref, size = x.T @ ga.reshape(-1, 16), x.abs().T @ ga.abs().reshape(-1, 16)
+        err = (torch.tensor(g["d1.w"][t // 3, t % 3], device="cuda") - ref).abs()
+        assert bool((err <= 2.0 ** -8 * size + 1e-30).all()), (t, float((err / size).max()))
+    err = (torch.tensor(g["d1.b"], device="cuda") - ga.sum((0, 1))).abs()
+    assert bool((err <= 2.0 ** -8 * ga.abs().sum((0, 1)) + 1e-30).all())
