@@ -12,8 +12,9 @@
 //     (v_mfma_f32_16x16x32_bf16). The same kernel computes the backward-data pass with mirrored, transposed weights and
 //     the ReLU mask applied while staging; upsample + concat of the decoder is folded into the staging, the encoder's
 //     2x2 pooling and the output 1x1 layer into the epilogue;
-//   * the weight gradient (k_dw) is a reduction over pixels: FP32 on the vector units from LDS tiles, per-block
-//     partials summed in a fixed order by k_dw_reduce (deterministic, no atomics);
+//   * the weight gradient (k_dw) is a matrix product too, K the pixels: channels-last LDS tiles read transposed
+//     (ds_read_b64_tr_b16), FP32 accumulation, per-block partials summed in a fixed order by k_dw_reduce (deterministic,
+//     no atomics);
 //   * the features and the energy-norm loss are elementwise / stencil kernels.
 #include <algorithm>
 #include <cmath>
@@ -29,11 +30,14 @@ namespace sr {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 #define NTH 256
 #define NB_FEAT 1024
-#define DW_SEG 32
-#define DW_BLOCKS 256
+#define DW_FLOATS (1 << 22)  // a layer's weight-gradient partials: so many, and 256 to 1024 blocks
+#define DW_TW 32         // its tile
+#define DW_TH 4
 #define LOG_CLAMP 20.0f
 #define CONV_FILL 512  // blocks that a convolution's launch keeps the chip busy with
 
@@ -433,98 +437,149 @@ __global__ void __launch_bounds__(NTH) k_out_back(int n, const float *__restrict
     block_partials<17>(v, part, gridDim.x);
 }
 
-// out[k] = sum of part[k nb .. k nb + nb) for k < K (fixed order)
-__global__ void k_reduce_rows(const double *part, int nb, int K, float *out) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= K) return;
-    double s = 0.0;
-    for (int i = 0; i < nb; i++) s += part[(size_t)k * nb + i];
-    out[k] = (float)s;
+// out[k] = sum of part[k nb .. k nb + nb), one block per k (a fixed order)
+__global__ void __launch_bounds__(NTH) k_reduce_rows(const double *part, int nb, float *out) {
+    const double s = sum_partials(part + (size_t)blockIdx.x * nb, nb);
+    if (threadIdx.x == 0) out[blockIdx.x] = (float)s;
 }
 
-// Weight and bias gradients of one layer: dW[tap][ci][co] = sum_p x[p + tap][ci] ga[p][co], ga = gy (y > 0).
-// A block takes 32-pixel row segments in turn; thread (gi, co) accumulates every tap of input channels gi, gi + NG,
-// ... for output channel co, reading the staged tiles from LDS (x broadcast across the wave, ga conflict-free).
+// Weight and bias gradients of one layer: dW[tap][ci][co] = sum_p x[p + tap][ci] ga[p][co], ga = gy (y > 0): per tap a
+// (CIN x pixels) (pixels x COUT) product on the matrix cores, FP32 accumulation of BF16 products (each exact in FP32).
+// A block walks 32 x 4 pixel tiles; the x tile (with its one-pixel rim) and ga lie channels-last in LDS and both operands
+// are read transposed (ds_read_b64_tr_b16: of four pixels x 16 channels over 16 lanes, lane i gets channel i of the four
+// pixels), so a lane's eight K values are eight consecutive pixels of one channel. The (tap, 16 input channels) pairs are
+// dealt to the four waves, each holding its pairs' accumulators for every output channel over all tiles; the last wave
+// also sums the biases' gradients (a row of ones). The pixel stride is an odd number of 32-byte slots: the eight pixels
+// that half a wave reads take eight slots. At 512^2 the ten layers' launches take 0.19 ms (vector FMAs from FP32 tiles:
+// 1.87 ms).
 template <int CIN, int COUT>
 __global__ void __launch_bounds__(NTH) k_dw(const bf16 *__restrict__ in, const bf16 *__restrict__ up, int cup,
                                             const bf16 *__restrict__ gy, const bf16 *__restrict__ y, int H, int W,
                                             float *__restrict__ part) {
-    constexpr int NG = NTH / COUT;
-    constexpr int CPT = CIN >= NG ? CIN / NG : 1;  // input channels per thread
-    static_assert(CIN < NG || CIN % NG == 0, "channel split");
-    __shared__ float xs[3][DW_SEG + 2][CIN];
-    __shared__ float gs[DW_SEG][COUT];
-    const int co = threadIdx.x % COUT, gi = threadIdx.x / COUT;
-    const bool active = gi < CIN;
-    float acc[9][CPT];
+    constexpr int CI = CIN < 16 ? 16 : CIN, MB = CI / 16, NBK = COUT / 16, PAIRS = 9 * MB, PPW = (PAIRS + 3) / 4;
+    constexpr int XP = MB % 2 ? CI : CI + 16, GP = NBK % 2 ? COUT : COUT + 16;  // pixel strides
+    constexpr int RW = DW_TW + 2, OX = CI / 8, OG = COUT / 8;
+    __shared__ __attribute__((aligned(16))) bf16 xs[(DW_TH + 2) * RW * XP];
+    __shared__ __attribute__((aligned(16))) bf16 gs[DW_TH * DW_TW * GP];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, i16 = lane & 15;
+    f32x4 acc[PPW][NBK], bacc[NBK];
 #pragma unroll
-    for (int t = 0; t < 9; t++)
+    for (int t = 0; t < NBK; t++) {
+        bacc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < CPT; c++) acc[t][c] = 0.0f;
-    float bacc = 0.0f;
-    const int cs = CIN - cup, spr = (W + DW_SEG - 1) / DW_SEG, nseg = H * spr;
-    for (int sg = blockIdx.x; sg < nseg; sg += gridDim.x) {
-        const int yr = sg / spr, x0 = (sg - yr * spr) * DW_SEG;
+        for (int q = 0; q < PPW; q++) acc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    bf16x8 ones;
+#pragma unroll
+    for (int j = 0; j < 8; j++) ones[j] = (bf16)1.0f;
+    // eight pixels from p on of 16 channels: pixels 8 g .. 8 g + 7 of the lane's group
+    auto tr8 = [&](const bf16 *p, int stride) {
+        const bf16 *q = p + (8 * g + (i16 >> 2)) * stride + 4 * (i16 & 3);
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)q);
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(q + 4 * stride));
+        return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    const int cs = CIN - cup, spr = (W + DW_TW - 1) / DW_TW, ntile = spr * ((H + DW_TH - 1) / DW_TH);
+    for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+        const int y0 = tile / spr * DW_TH, x0 = tile % spr * DW_TW;
         __syncthreads();
-        for (int t = threadIdx.x; t < 3 * (DW_SEG + 2) * CIN; t += NTH) {
-            const int c = t % CIN, rest = t / CIN, px = rest % (DW_SEG + 2), ry = rest / (DW_SEG + 2);
-            const int yy = yr + ry - 1, xx = x0 + px - 1;
-            float val = 0.0f;
-            if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-                val = c < cup ? (float)up[((size_t)(yy >> 1) * (W >> 1) + (xx >> 1)) * cup + c]
-                              : (float)in[((size_t)yy * W + xx) * cs + (c - cup)];
-            xs[ry][px][c] = val;
+        for (int t = threadIdx.x; t < (DW_TH + 2) * RW * OX; t += NTH) {
+            const int o = t % OX, px = t / OX, lx = px % RW, ly = px / RW, ci = 8 * o;
+            const int xx = x0 + lx - 1, yy = y0 + ly - 1;
+            bf16x8 v = {};
+            if (ci < CIN && xx >= 0 && xx < W && yy >= 0 && yy < H)
+                v = ci < cup ? ld8(up + ((size_t)(yy >> 1) * (W >> 1) + (xx >> 1)) * cup + ci)
+                             : ld8(in + ((size_t)yy * W + xx) * cs + (ci - cup));
+            st8(xs + px * XP + ci, v);
         }
-        for (int t = threadIdx.x; t < DW_SEG * COUT; t += NTH) {
-            const int c = t % COUT, px = t / COUT, xx = x0 + px;
-            float gv = 0.0f;
-            if (xx < W) {
-                const size_t i = ((size_t)yr * W + xx) * COUT + c;
-                gv = (float)y[i] > 0.0f ? (float)gy[i] : 0.0f;
+        for (int t = threadIdx.x; t < DW_TH * DW_TW * OG; t += NTH) {
+            const int o = t % OG, px = t / OG, xx = x0 + px % DW_TW, yy = y0 + px / DW_TW;
+            bf16x8 v = {};
+            if (xx < W && yy < H) {
+                const size_t i = ((size_t)yy * W + xx) * COUT + 8 * o;
+                v = ld8(gy + i);
+                const bf16x8 yv = ld8(y + i);
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    if (!((float)yv[j] > 0.0f)) v[j] = (bf16)0.0f;
             }
-            gs[px][c] = gv;
+            st8(gs + px * GP + 8 * o, v);
         }
         __syncthreads();
-        if (active) {
-            for (int p = 0; p < DW_SEG; p++) {
-                const float gv = gs[p][co];
-                bacc += gv;
+#pragma unroll 1
+        for (int r = 0; r < DW_TH; r++) {
+            bf16x8 gv[NBK];
 #pragma unroll
-                for (int t = 0; t < 9; t++)
+            for (int t = 0; t < NBK; t++) gv[t] = tr8(gs + r * DW_TW * GP + 16 * t, GP);
 #pragma unroll
-                    for (int c = 0; c < CPT; c++) acc[t][c] += xs[t / 3][p + t % 3][gi + c * NG] * gv;
+            for (int q = 0; q < PPW; q++) {
+                const int pr = wave + 4 * q, tap = pr / MB, mb = pr - tap * MB;
+                if (pr >= PAIRS) continue;
+                const bf16x8 xv = tr8(xs + ((r + tap / 3) * RW + tap % 3) * XP + 16 * mb, XP);
+#pragma unroll
+                for (int t = 0; t < NBK; t++)
+                    acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, gv[t], acc[q][t], 0, 0, 0);
             }
+            if (wave == 3)
+#pragma unroll
+                for (int t = 0; t < NBK; t++)
+                    bacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, gv[t], bacc[t], 0, 0, 0);
         }
     }
     float *pb = part + (size_t)blockIdx.x * (9 * CIN * COUT + COUT);
-    if (active) {
 #pragma unroll
-        for (int t = 0; t < 9; t++)
+    for (int q = 0; q < PPW; q++) {
+        const int pr = wave + 4 * q, tap = pr / MB, mb = pr - tap * MB;
+        if (pr >= PAIRS) continue;
 #pragma unroll
-            for (int c = 0; c < CPT; c++) pb[((size_t)t * CIN + gi + c * NG) * COUT + co] = acc[t][c];
-        if (gi == 0) pb[9 * CIN * COUT + co] = bacc;
+        for (int t = 0; t < NBK; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int ci = 16 * mb + 4 * g + j;
+                if (ci < CIN) pb[((size_t)tap * CIN + ci) * COUT + 16 * t + i16] = acc[q][t][j];
+            }
     }
+    if (wave == 3 && g == 0)
+#pragma unroll
+        for (int t = 0; t < NBK; t++) pb[9 * CIN * COUT + 16 * t + i16] = bacc[t][0];
 }
 
-// sums the k_dw partials of nb blocks into a layer's gradients in the (3, 3, cin, cout) + (cout) layout
-__global__ void k_dw_reduce(const float *__restrict__ part, int nb, int cinp, int cin, int cout, float *gw, float *gb) {
-    const int o = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nw = 9 * cin * cout;
-    if (o >= nw + cout) return;
+// Every layer's k_dw partials summed into the gradients in one launch: a block takes 32 consecutive values of one
+// layer's (3, 3, cin, cout) + (cout), eight threads a value, each a strided run of the layer's blocks (in FP64), the runs
+// joined in order. (One thread a value walking all blocks took 63 us a layer: a chain of 256 loads.)
+struct DwTable {
+    int n;
+    int start[10], nb[10], cinp[10], cin[10], cout[10];  // first block, k_dw blocks, the layer's shape
+    size_t part[10], w[10], b[10];                       // offsets of the partials and of the gradients
+};
+
+__global__ void __launch_bounds__(NTH) k_dw_reduce(DwTable T, const float *__restrict__ part, float *__restrict__ grads) {
+    int l = 0;
+    while (l + 1 < T.n && (int)blockIdx.x >= T.start[l + 1]) l++;
+    const int cin = T.cin[l], cout = T.cout[l], cinp = T.cinp[l], nw = 9 * cin * cout, nb = T.nb[l];
+    const int v = threadIdx.x & 31, run = threadIdx.x >> 5, o = ((int)blockIdx.x - T.start[l]) * 32 + v;
     const size_t stride = (size_t)9 * cinp * cout + cout;
-    size_t src;
-    if (o < nw) {
-        const int co = o % cout, rest = o / cout, ci = rest % cin, tap = rest / cin;
-        src = ((size_t)tap * cinp + ci) * cout + co;
-    } else {
-        src = (size_t)9 * cinp * cout + (o - nw);
-    }
+    __shared__ double sh[NTH / 32][32];
     double s = 0.0;
-    for (int b = 0; b < nb; b++) s += part[(size_t)b * stride + src];
-    if (o < nw)
-        gw[o] = (float)s;
-    else
-        gb[o - nw] = (float)s;
+    if (o < nw + cout) {
+        size_t src = (size_t)9 * cinp * cout + (o - nw);
+        if (o < nw) {
+            const int co = o % cout, rest = o / cout, ci = rest % cin, tap = rest / cin;
+            src = ((size_t)tap * cinp + ci) * cout + co;
+        }
+        const float *p = part + T.part[l] + src;
+#pragma unroll 8
+        for (int b = run; b < nb; b += NTH / 32) s += p[(size_t)b * stride];
+    }
+    sh[run][v] = s;
+    __syncthreads();
+    if (run == 0 && o < nw + cout) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < NTH / 32; k++) t += sh[k][v];
+        grads[o < nw ? T.w[l] + o : T.b[l] + (o - nw)] = (float)t;
+    }
 }
 
 // Adam (Kingma and Ba 2015, Algorithm 1) on the FP32 master parameters
@@ -539,21 +594,32 @@ __global__ void k_adam(int n, float *__restrict__ p, const float *__restrict__ g
     p[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
 }
 
-// the BF16 weight layouts of one layer from its FP32 (3, 3, cin, cout) master, K in k_conv's order: forward (cout, kp)
-// over the taps and input channels, backward-data (cin, kpb) over the mirrored taps and output channels
-__global__ void k_pack(const float *__restrict__ w, int cin, int cinp, int cout, int kp, int kpb, bf16 *__restrict__ wt,
-                       bf16 *__restrict__ wb) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nf = cout * kp, nbk = wb ? cin * kpb : 0;
+// The BF16 weight layouts of every layer from the FP32 (3, 3, cin, cout) masters, K in k_conv's order: forward (cout, kp)
+// over the taps and input channels, backward-data (cin, kpb) over the mirrored taps and output channels (wb null: none).
+// One launch for all layers (a launch each, ten of them, cost a training step 45 us).
+struct PackTable {
+    int start[11];  // first value of each layer's two layouts, the total last
+    int cin[10], cinp[10], cout[10], kp[10], kpb[10];
+    size_t w[10];
+    bf16 *wt[10], *wb[10];
+};
+
+__global__ void k_pack(PackTable T, const float *__restrict__ params) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x, l = 0;
+    if (i >= T.start[10]) return;
+    while (i >= T.start[l + 1]) l++;
+    i -= T.start[l];
+    const int cin = T.cin[l], cout = T.cout[l], kp = T.kp[l], kpb = T.kpb[l], nf = cout * kp;
+    const float *w = params + T.w[l];
     int tap, c;
     if (i < nf) {
         const int co = i / kp;
-        const bool in = conv_k(cinp, i - co * kp, tap, c) && c < cin;
-        wt[i] = (bf16)(in ? w[((size_t)tap * cin + c) * cout + co] : 0.0f);
-    } else if (i < nf + nbk) {
+        const bool in = conv_k(T.cinp[l], i - co * kp, tap, c) && c < cin;
+        T.wt[l][i] = (bf16)(in ? w[((size_t)tap * cin + c) * cout + co] : 0.0f);
+    } else {
         const int j = i - nf, ci = j / kpb;
         const bool in = conv_k(cout, j - ci * kpb, tap, c);
-        wb[j] = (bf16)(in ? w[((size_t)(8 - tap) * cin + ci) * cout + c] : 0.0f);
+        T.wb[l][j] = (bf16)(in ? w[((size_t)(8 - tap) * cin + ci) * cout + c] : 0.0f);
     }
 }
 
@@ -652,11 +718,21 @@ int Net::get_grads(float *h, size_t n) {
 }
 
 int Net::pack(hipStream_t s) {
-    for (auto &l : L) {
-        const int total = l.cout * l.kp + (l.wb ? l.cin * l.kpb : 0);
-        hipLaunchKernelGGL(k_pack, dim3((total + 255) / 256), dim3(256), 0, s, params + l.w_off, l.cin, l.cinp, l.cout,
-                           l.kp, l.kpb, l.wt, l.wb);
+    PackTable T;
+    T.start[0] = 0;
+    for (int i = 0; i < 10; i++) {
+        const NetLayer &l = L[i];
+        T.cin[i] = l.cin;
+        T.cinp[i] = l.cinp;
+        T.cout[i] = l.cout;
+        T.kp[i] = l.kp;
+        T.kpb[i] = l.kpb;
+        T.w[i] = l.w_off;
+        T.wt[i] = l.wt;
+        T.wb[i] = l.wb;
+        T.start[i + 1] = T.start[i] + l.cout * l.kp + (l.wb ? l.cin * l.kpb : 0);
     }
+    hipLaunchKernelGGL(k_pack, dim3((T.start[10] + 255) / 256), dim3(256), 0, s, T, (const float *)params);
     SR_HIP(hipGetLastError());
     packed = true;
     return SR_OK;
@@ -727,15 +803,35 @@ int Net::apply(int w, int h, const float *own, const float *kx, const float *ky,
     return forward(w, h, own, kx, ky, r, zadd, z, nullptr, nullptr, s);
 }
 
+// The weight gradient's blocks for an image: a tile each up to as many as the partials' size allows (four to a CU where
+// the layer is small: a block waits on its tile's loads before it computes; one where every block's partials are 100 KB),
+// then as few as take the same number of turns.
+static int dw_blocks_most(int size) { return std::max(256, std::min(1024, DW_FLOATS / size)); }
+static int dw_tiles(int H, int W) { return ((W + DW_TW - 1) / DW_TW) * ((H + DW_TH - 1) / DW_TH); }
+static int dw_blocks(int H, int W, int size) {
+    const int nt = dw_tiles(H, W), most = dw_blocks_most(size), turns = (nt + most - 1) / most;
+    return (nt + turns - 1) / turns;
+}
+
 template <int CIN, int COUT>
 static void dw(hipStream_t s, const bf16 *in, const bf16 *up, int cup, const bf16 *gy, const bf16 *y, int H, int W,
-               float *wpart, const NetLayer &l, float *grads) {
-    const int nseg = H * ((W + DW_SEG - 1) / DW_SEG);
-    const int nb = std::min(DW_BLOCKS, nseg);
-    hipLaunchKernelGGL((k_dw<CIN, COUT>), dim3(nb), dim3(NTH), 0, s, in, up, cup, gy, y, H, W, wpart);
-    const int nout = 9 * l.cin * l.cout + l.cout;
-    hipLaunchKernelGGL(k_dw_reduce, dim3((nout + 255) / 256), dim3(256), 0, s, (const float *)wpart, nb, l.cinp,
-                       l.cin, l.cout, grads + l.w_off, grads + l.b_off);
+               float *wpart, const NetLayer &l, DwTable &T) {
+    const int nb = dw_blocks(H, W, 9 * CIN * COUT + COUT), k = T.n++, nout = 9 * l.cin * l.cout + l.cout;
+    T.nb[k] = nb;
+    T.cinp[k] = l.cinp;
+    T.cin[k] = l.cin;
+    T.cout[k] = l.cout;
+    T.w[k] = l.w_off;
+    T.b[k] = l.b_off;
+    if (k == 0) {
+        T.start[0] = 0;
+        T.part[0] = 0;
+    }
+    hipLaunchKernelGGL((k_dw<CIN, COUT>), dim3(nb), dim3(NTH), 0, s, in, up, cup, gy, y, H, W, wpart + T.part[k]);
+    if (k + 1 < 10) {
+        T.start[k + 1] = T.start[k] + (nout + 31) / 32;
+        T.part[k + 1] = T.part[k] + (size_t)nb * (9 * l.cinp * l.cout + l.cout);
+    }
 }
 
 int Net::loss_grad(int w, int h, const float *own, const float *kx, const float *ky, const float *r, const float *e,
@@ -758,45 +854,57 @@ int Net::loss_grad(int w, int h, const float *own, const float *kx, const float 
         SR_TRY(dalloc(&gout, n));
         SR_TRY(dalloc(&lpart, 2 * NB_FEAT));
         SR_TRY(dalloc(&opart, 17 * NB_FEAT));
-        SR_TRY(dalloc(&wpart, (size_t)DW_BLOCKS * (9 * 64 * 64 + 64)));
+        // every layer's weight-gradient partials, each layer's at its own resolution
+        const int shift[10] = {0, 0, 1, 1, 2, 2, 1, 1, 0, 0};
+        size_t parts = 0;
+        for (int i = 0; i < 10; i++) {
+            const int size = 9 * L[i].cinp * L[i].cout + L[i].cout;
+            parts += (size_t)std::min(dw_blocks_most(size), dw_tiles(max_h >> shift[i], max_w >> shift[i])) * size;
+        }
+        SR_TRY(dalloc(&wpart, parts));
     }
     SR_TRY(forward(w, h, own, kx, ky, r, nullptr, nullptr, e, err, s));
     const size_t n = (size_t)w * h;
     const int nb = grid_of(n);
     const int w2 = w / 2, h2 = h / 2, w4 = w / 4, h4 = h / 4;
+    DwTable T;
+    T.n = 0;
     hipLaunchKernelGGL(k_loss, dim3(nb), dim3(NTH), 0, s, w, h, own, kx, ky, (const float *)err, e, aerr, lpart);
     hipLaunchKernelGGL(k_out_back, dim3(nb), dim3(NTH), 0, s, (int)n, (const float *)aerr, (const double *)lpart, nb,
                        (const float *)scal, (const float *)dis, (const bf16 *)d1, (const float *)(params + out_off),
                        gout, g_d1, opart);
-    hipLaunchKernelGGL(k_reduce_rows, dim3(1), dim3(64), 0, s, (const double *)opart, nb, 17, grads + out_off);
+    hipLaunchKernelGGL(k_reduce_rows, dim3(17), dim3(NTH), 0, s, (const double *)opart, nb, grads + out_off);
     // decoder, level 1
-    dw<16, 16>(s, d1a, nullptr, 0, g_d1, d1, h, w, wpart, L[D1], grads);
+    dw<16, 16>(s, d1a, nullptr, 0, g_d1, d1, h, w, wpart, L[D1], T);
     conv<16, 16>(s, cargs(g_d1, nullptr, 0, d1, L[D1].wb, nullptr, g_d1a, h, w, 0));
-    dw<48, 16>(s, e1, d2, 32, g_d1a, d1a, h, w, wpart, L[D1A], grads);
+    dw<48, 16>(s, e1, d2, 32, g_d1a, d1a, h, w, wpart, L[D1A], T);
     ConvArgs cat = cargs(g_d1a, nullptr, 0, d1a, L[D1A].wb, nullptr, g_e1, h, w, 0);
     cat.half = g_d2;
     conv<16, 48, CONV_SPLIT>(s, cat);
     // decoder, level 2
-    dw<32, 32>(s, d2a, nullptr, 0, g_d2, d2, h2, w2, wpart, L[D2], grads);
+    dw<32, 32>(s, d2a, nullptr, 0, g_d2, d2, h2, w2, wpart, L[D2], T);
     conv<32, 32>(s, cargs(g_d2, nullptr, 0, d2, L[D2].wb, nullptr, g_d2a, h2, w2, 0));
-    dw<96, 32>(s, e2, e3, 64, g_d2a, d2a, h2, w2, wpart, L[D2A], grads);
+    dw<96, 32>(s, e2, e3, 64, g_d2a, d2a, h2, w2, wpart, L[D2A], T);
     cat = cargs(g_d2a, nullptr, 0, d2a, L[D2A].wb, nullptr, g_e2, h2, w2, 0);
     cat.half = g_e3;
     conv<32, 96, CONV_SPLIT>(s, cat);
     // encoder, level 3
-    dw<64, 64>(s, e3a, nullptr, 0, g_e3, e3, h4, w4, wpart, L[E3], grads);
+    dw<64, 64>(s, e3a, nullptr, 0, g_e3, e3, h4, w4, wpart, L[E3], T);
     conv<64, 64>(s, cargs(g_e3, nullptr, 0, e3, L[E3].wb, nullptr, g_e3a, h4, w4, 0));
-    dw<32, 64>(s, p2, nullptr, 0, g_e3a, e3a, h4, w4, wpart, L[E3A], grads);
+    dw<32, 64>(s, p2, nullptr, 0, g_e3a, e3a, h4, w4, wpart, L[E3A], T);
     conv<64, 32, CONV_UNPOOL>(s, cargs(g_e3a, nullptr, 0, e3a, L[E3A].wb, nullptr, g_e2, h4, w4, 0));
     // encoder, level 2
-    dw<32, 32>(s, e2a, nullptr, 0, g_e2, e2, h2, w2, wpart, L[E2], grads);
+    dw<32, 32>(s, e2a, nullptr, 0, g_e2, e2, h2, w2, wpart, L[E2], T);
     conv<32, 32>(s, cargs(g_e2, nullptr, 0, e2, L[E2].wb, nullptr, g_e2a, h2, w2, 0));
-    dw<16, 32>(s, p1, nullptr, 0, g_e2a, e2a, h2, w2, wpart, L[E2A], grads);
+    dw<16, 32>(s, p1, nullptr, 0, g_e2a, e2a, h2, w2, wpart, L[E2A], T);
     conv<32, 16, CONV_UNPOOL>(s, cargs(g_e2a, nullptr, 0, e2a, L[E2A].wb, nullptr, g_e1, h2, w2, 0));
     // encoder, level 1
-    dw<16, 16>(s, e1a, nullptr, 0, g_e1, e1, h, w, wpart, L[E1], grads);
+    dw<16, 16>(s, e1a, nullptr, 0, g_e1, e1, h, w, wpart, L[E1], T);
     conv<16, 16>(s, cargs(g_e1, nullptr, 0, e1, L[E1].wb, nullptr, g_e1a, h, w, 0));
-    dw<8, 16>(s, x, nullptr, 0, g_e1a, e1a, h, w, wpart, L[E1A], grads);
+    dw<8, 16>(s, x, nullptr, 0, g_e1a, e1a, h, w, wpart, L[E1A], T);
+    const NetLayer &l0 = L[E1A];  // the last in the table
+    const int rblocks = T.start[9] + (9 * l0.cin * l0.cout + l0.cout + 31) / 32;
+    hipLaunchKernelGGL(k_dw_reduce, dim3(rblocks), dim3(NTH), 0, s, T, (const float *)wpart, grads);
     SR_HIP(hipGetLastError());
     if (loss) {
         SR_HIP(hipMemcpyAsync(host, lpart, sizeof(double) * 2 * nb, hipMemcpyDeviceToHost, s));
