@@ -75,10 +75,51 @@ void react_build(const sr_react_params *p, const sr_physics &ph, ReactDev *out) 
         const sr_react_record &c = p->rec[r];
         for (int k = 0; k < c.n_out; k++) out->nu[r][c.out_species[k]] += c.out_share[k];
         for (int k = 0; k < c.n_in; k++) out->nu[r][c.in_species[k]] -= c.in_share[k];
-        if (c.n_terms > 0)  // rates.rs:62-71: log-spaced nodes from T_thr over the span
-            for (int i = 0; i < REACT_TABLE; i++)
-                out->ln_f[r][i] =
-                    std::log(f_sum(c, c.t_thr * std::exp(std::log(2.5) * (double)i / (double)(REACT_TABLE - 1))));
+        // rates.rs:62-71: log-spaced nodes from T_thr over the span; a record of the same law as an earlier one reads its
+        out->f_of[r] = -1;
+        if (c.n_terms == 0) continue;
+        out->ln_thr[r] = std::log(c.t_thr);
+        for (int q = 0; q < r && out->f_of[r] < 0; q++) {
+            const sr_react_record &o = p->rec[q];
+            bool same = o.n_terms == c.n_terms && o.t_thr == c.t_thr;
+            for (int k = 0; same && k < c.n_terms; k++)
+                same = o.t_k[k] == c.t_k[k] && o.nu[k] == c.nu[k] && o.w[k] == c.w[k];
+            if (same) out->f_of[r] = out->f_of[q];
+        }
+        if (out->f_of[r] >= 0) continue;
+        out->f_of[r] = out->tables++;
+        for (int i = 0; i < REACT_TABLE; i++)
+            out->ln_f[out->f_of[r]][i] =
+                std::log(f_sum(c, c.t_thr * std::exp(std::log(2.5) * (double)i / (double)(REACT_TABLE - 1))));
+    }
+    // the linear system's entries, items and elimination pattern
+    for (int r = 0; r < p->n_records; r++) {
+        out->ent0[r] = out->entries;
+        out->slot[r] = out->slots;
+        if (r == p->nfe) continue;
+        out->entries += p->rec[r].n_in;
+        out->slots++;
+    }
+    out->ent0[p->n_records] = out->entries;
+    unsigned reach[NS];  // the columns a row can hold a value in
+    for (int i = 0; i < NS; i++) {
+        reach[i] = 1u << i;
+        for (int j = 0; j < NS; j++) {
+            const int first = out->items;
+            for (int r = 0; r < p->n_records; r++) {
+                if (r == p->nfe || out->nu[r][i] == 0.0) continue;
+                for (int k = 0; k < p->rec[r].n_in; k++)
+                    if (p->rec[r].in_species[k] == j)
+                        out->item[out->items++] = {out->nu[r][i], out->ent0[r] + k, 0};
+            }
+            if (out->items == first) continue;
+            out->item[out->items - 1].last = 1;
+            out->row[i] |= 1u << j;
+            reach[i] |= 1u << j;
+        }
+        for (int j = 0; j < i; j++)
+            if (reach[i] >> j & 1) reach[i] |= reach[j] >> j << j;
+        out->row[i] |= (reach[i] & ((1u << i) - 1)) << 16;
     }
     out->sigma_vac = ph.sigma_vac;
     out->t_floor = ph.t_floor;
@@ -105,6 +146,17 @@ __device__ inline void comp(const double *x, double *mu, double *y_e) {
     *y_e = ye;
 }
 
+// The tables and the threads' private arrays in LDS: the cold pairs' ln u, f's tables, then per thread a value by species
+// (x while the rates are formed, dX after a solve), omega by record and the derivatives by entry. A species or record
+// index is the wave's own but not the compiler's, so such an array in registers would go to scratch memory (as the whole
+// pass's did: 587 us a pass at 512^2, 105 now). A thread's element k lies NT values from its element
+// k - 1: no bank conflicts. NT = 256 threads share the tables, so that two blocks (two waves a SIMD) fit a CU; with so many
+// inputs that they would not (the shipped records: 78 KB), 64.
+struct Lds {
+    const double *cold, *ln_f;
+    double *v, *omega, *grad;  // the thread's own: element k at [k * NT]
+};
+
 // u(x) of one pair from its FP64 table: linear in (ln x, ln u), the K1 x^2 power law below the first node
 __device__ inline double cold_u_d(const ReactDev &D, const double *lnu, double x) {
     if (x <= 0.0) return 0.0;
@@ -116,10 +168,10 @@ __device__ inline double cold_u_d(const ReactDev &D, const double *lnu, double x
     return exp(lnu[i] + frac * (lnu[i + 1] - lnu[i]));
 }
 
-__device__ inline double eps_cold_d(const ReactDev &D, double sigma, double y_e, double x_n) {
+__device__ inline double eps_cold_d(const ReactDev &D, const Lds &M, double sigma, double y_e, double x_n) {
     double u = 0.0;
-    if (D.cold_pair[0]) u += cold_u_d(D, D.cold_lnu[0], y_e * sigma);
-    if (D.cold_pair[1]) u += cold_u_d(D, D.cold_lnu[1], x_n * sigma);
+    if (D.cold_pair[0]) u += cold_u_d(D, M.cold, y_e * sigma);
+    if (D.cold_pair[1]) u += cold_u_d(D, M.cold + COLD_POINTS, x_n * sigma);
     return u / sigma;
 }
 
@@ -132,17 +184,18 @@ __device__ __forceinline__ double ipow(double x, double n) {
     return pow(x, n);
 }
 
-// f(T) through the table (rates.rs:98-118): 0 below T_thr, the direct sum past the table's span
-__device__ inline double temp_factor(const ReactDev &D, int r, double t) {
+// f(T) through the table (rates.rs:98-118) from T and ln T: 0 below T_thr, the direct sum past the table's span
+__device__ inline double temp_factor(const ReactDev &D, const Lds &M, int r, double t, double ln_t) {
     const sr_react_record &c = D.P.rec[r];
     if (c.n_terms == 0) return 1.0;
     if (t < c.t_thr) return 0.0;
     const double step = log(2.5) / (double)(REACT_TABLE - 1);
-    const double pos = log(t / c.t_thr) / step;
+    const double pos = fmax(ln_t - D.ln_thr[r], 0.0) / step;
     if (pos >= (double)(REACT_TABLE - 1)) return f_sum(c, t);
     const int i = (int)floor(pos);
     const double frac = pos - (double)i;
-    return exp(D.ln_f[r][i] + frac * (D.ln_f[r][i + 1] - D.ln_f[r][i]));
+    const double *ln_f = M.ln_f + D.f_of[r] * REACT_TABLE;
+    return exp(ln_f[i] + frac * (ln_f[i + 1] - ln_f[i]));
 }
 
 // the gate g(Y_e Sigma) (rates.rs:119-125)
@@ -150,16 +203,6 @@ __device__ inline double gate(const sr_react_record &c, double sigma, double y_e
     if (!c.gated) return 1.0;
     const double yes = y_e * sigma;
     return yes > c.sigma_g ? pow(yes / c.sigma_g - 1.0, c.gate_p) : 0.0;
-}
-
-// omega = A Sigma^a prod X^n f(T) g(Y_e Sigma) (rates.rs:121-131)
-__device__ inline double omega(const ReactDev &D, int r, double sigma, const double *x, double t, double y_e) {
-    const sr_react_record &c = D.P.rec[r];
-    const double f = temp_factor(D, r, t);
-    double orders = 1.0;
-    for (int k = 0; k < c.n_in; k++) orders *= ipow(x[c.in_species[k]], c.in_order[k]);
-    const double g = gate(c, sigma, y_e);
-    return c.a_coef * ipow(sigma, c.a_sigma) * orders * f * g;
 }
 
 // N_Fe over dt in closed form (react.rs:470-513)
@@ -207,18 +250,20 @@ __device__ double nfe_exact(const ReactDev &D, double sigma, double *x, double d
     return dm;
 }
 
-// (I - h J) dX = h S, Gaussian elimination with partial pivoting, the last of equal pivots (react.rs:515-560)
-__device__ void solve(const ReactDev &D, const double (*grad)[NS], const double *s, double h, double *dx) {
+// (I - h J) dX = h S, Gaussian elimination with partial pivoting, the last of equal pivots (react.rs:515-560): the form
+// for a system that needs a row exchange, its matrix in scratch memory
+template <int NT>
+__device__ __noinline__ void solve_pivoted(const ReactDev &D, const Lds &M, const double *s, double h, double *dx) {
     double a[NS][NS + 1];
-    const int nr = D.P.n_records;
+    int q = 0;
     for (int i = 0; i < NS; i++) {
-        for (int j = 0; j <= NS; j++) a[i][j] = 0.0;
-        a[i][i] = 1.0;
-        a[i][NS] = h * s[i];
-        for (int r = 0; r < nr; r++) {
-            if (D.nu[r][i] == 0.0) continue;
-            for (int j = 0; j < NS; j++) a[i][j] -= h * D.nu[r][i] * grad[r][j];
+        for (int j = 0; j < NS; j++) {
+            a[i][j] = i == j ? 1.0 : 0.0;
+            if (D.row[i] >> j & 1) do {
+                    a[i][j] -= h * D.item[q].nu * M.grad[D.item[q].e * NT];
+                } while (!D.item[q++].last);
         }
+        a[i][NS] = h * s[i];
     }
     for (int col = 0; col < NS; col++) {
         int piv = col;
@@ -245,81 +290,156 @@ __device__ void solve(const ReactDev &D, const double (*grad)[NS], const double 
     }
 }
 
+// The same system by rows in registers: each row is built and reduced by the rows above it (the columns it can hold a
+// value in, `lower`), the same operations in the same order on every element as by columns. Where the pivoted form would
+// exchange rows (an element at least as large as its pivot) the pivoted form solves the system instead; the consumed
+// species' diagonal 1 + h sum of its losses exceeds what any product's row holds, so no physical system is. NA: the
+// species to solve for (9 where the last, the neutrons, has no items, as with N_Fe in closed form: dX = 0).
+template <int NA, int NT>
+__device__ inline void solve(const ReactDev &D, const Lds &M, const double (&s)[NS], double h, double (&dx)[NS]) {
+    double u[NA][NA];
+    bool exchange = false;
+    int q = 0;
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+        double b = h * s[i];
+        const unsigned shape = D.row[i];
+#pragma unroll
+        for (int j = 0; j < NA; j++) {
+            u[i][j] = i == j ? 1.0 : 0.0;
+            if (shape >> j & 1) do {
+                    u[i][j] -= h * D.item[q].nu * M.grad[D.item[q].e * NT];
+                } while (!D.item[q++].last);
+        }
+#pragma unroll
+        for (int col = 0; col < i; col++) {
+            if (!(shape >> (16 + col) & 1)) continue;
+            const double d = u[col][col];
+            exchange |= fabs(u[i][col]) >= fabs(d);
+            const double f = u[i][col] / d;
+#pragma unroll
+            for (int j = col + 1; j < NS; j++) u[i][j] -= f * u[col][j];
+            b -= f * dx[col];
+        }
+        dx[i] = b;
+    }
+#pragma unroll
+    for (int i = NA - 1; i >= 0; i--) {
+        double v = dx[i];
+#pragma unroll
+        for (int j = i + 1; j < NA; j++) v -= u[i][j] * dx[j];
+        exchange |= u[i][i] == 0.0;
+        dx[i] = v / u[i][i];
+    }
+#pragma unroll
+    for (int i = NA; i < NS; i++) dx[i] = 0.0;
+    if (exchange) {
+        double sv[NS], dv[NS];
+        for (int i = 0; i < NS; i++) sv[i] = s[i];
+        solve_pivoted<NT>(D, M, sv, h, dv);
+#pragma unroll
+        for (int i = 0; i < NS; i++) dx[i] = dv[i];
+    }
+}
+
 struct CellOut {
-    double x[NS], de, lost, booked[NG], pinned_e;
+    double de, lost, booked[NG], pinned_e;
     int nfe, pinned, unfinished, changed;
     double substeps, retried, max_dx, max_dt_rel;
 };
 
-// one cell over dt (react.rs:272-449)
-__device__ void burn(const ReactDev &D, double sigma, const double *x0, double e_tot0, double dt, CellOut &cell) {
+// one cell over dt (react.rs:272-449), its fractions in x; the composition, the cold energy and T of a state are formed
+// once, with the sub-step that reaches it
+template <int NA, int NT>
+__device__ inline void burn(const ReactDev &D, const Lds &M, double sigma, double (&x)[NS], double e_tot, double dt,
+                            CellOut &cell) {
     const sr_react_params &P = D.P;
     const int nr = P.n_records, pin = P.pin_temperature;
-    double x[NS];
-    for (int s = 0; s < NS; s++) x[s] = x0[s];
-    double e_tot = e_tot0;
     cell.de = cell.lost = cell.pinned_e = cell.substeps = cell.retried = cell.max_dx = cell.max_dt_rel = 0.0;
+#pragma unroll
     for (int g = 0; g < NG; g++) cell.booked[g] = 0.0;
     cell.nfe = cell.pinned = cell.unfinished = cell.changed = 0;
-    double mu0, y_e0;
-    comp(x, &mu0, &y_e0);
-    const double eps_th0 = fmax(e_tot0 - eps_cold_d(D, sigma, y_e0, x0[ID_N]), D.t_floor / mu0);
-    const double t0 = mu0 * eps_th0;
+    double mu, y_e;
+    comp(x, &mu, &y_e);
+    double t = mu * fmax(e_tot - eps_cold_d(D, M, sigma, y_e, x[ID_N]), D.t_floor / mu);
+    const double t0 = t;
     if (P.nfe >= 0) {
-        const double w_nfe = omega(D, P.nfe, sigma, x, t0, y_e0);
+        // N_Fe's rate at the start (no temperature law: f = 1)
+        const sr_react_record &c = P.rec[P.nfe];
+        const double g = gate(c, sigma, y_e);
+        double x_in = 0.0;
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+            if (s == c.in_species[0]) x_in = x[s];
+        const double w_nfe = g > 0.0 ? c.a_coef * ipow(sigma, c.a_sigma) * x_in * g : 0.0;
         cell.nfe = w_nfe > 0.0;
         if (cell.nfe) {
-            const double dm = nfe_exact(D, sigma, x, dt);
-            const double heat = P.rec[P.nfe].q * dm;
+            double xn[NS];
+            for (int s = 0; s < NS; s++) xn[s] = x[s];
+            const double dm = nfe_exact(D, sigma, xn, dt);
+            const double heat = c.q * dm;
             if (!pin) e_tot += heat;
             cell.de += heat;
-            cell.booked[P.rec[P.nfe].group] += heat;
+#pragma unroll
+            for (int q = 0; q < NG; q++)
+                if (q == c.group) cell.booked[q] += heat;
             cell.changed |= dm > 0.0;
+#pragma unroll
+            for (int s = 0; s < NS; s++) x[s] = xn[s];
+            comp(x, &mu, &y_e);
+            if (!pin) t = mu * fmax(e_tot - eps_cold_d(D, M, sigma, y_e, x[ID_N]), D.t_floor / mu);
         }
     }
     double t_done = 0.0, h_try = HUGE_VAL;
     unsigned long long attempts = 0;
     while (t_done < dt) {
         double t_rem = dt - t_done;
-        double mu, y_e;
-        comp(x, &mu, &y_e);
-        const double t = pin ? t0 : mu * fmax(e_tot - eps_cold_d(D, sigma, y_e, x[ID_N]), D.t_floor / mu);
-        double omegas[NR], grad[NR][NS], s[NS], qdot = 0.0;
-        for (int i = 0; i < NS; i++) s[i] = 0.0;
+        double s[NS], qdot = 0.0;
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+            s[i] = 0.0;
+            M.v[i * NT] = x[i];
+        }
         double enu = P.neutrinos && t >= P.t_nu ? P.a_nu * pow(t / P.t_nu, P.m_nu) : 0.0;
-        int any = 0;
+        int any = 0, f_last = -1;
+        const double ln_t = log(t);
+        double f_val = 1.0;
         for (int r = 0; r < nr; r++) {
-            omegas[r] = 0.0;
-            for (int j = 0; j < NS; j++) grad[r][j] = 0.0;
             if (r == P.nfe) continue;
             const sr_react_record &c = P.rec[r];
             // omega at X and, for each input j, at X with X_j = 1 (whose factor 1^n is exactly 1): f, g and A Sigma^a
-            // once, each input's power once, the products in omega()'s order
-            const double f = temp_factor(D, r, t), g = gate(c, sigma, y_e);
+            // once (f kept for a next record of the same law), each input's power once, the products in their order
+            if (c.n_terms == 0 || D.f_of[r] != f_last) f_val = temp_factor(D, M, r, t, ln_t);
+            f_last = D.f_of[r];
+            const double f = f_val, g = gate(c, sigma, y_e);
             const double ap = c.a_coef * ipow(sigma, c.a_sigma);
             const int n_in = c.n_in;
-            double pw[4];
+            double xk[4], pw[4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) pw[k] = k < n_in ? ipow(x[c.in_species[k]], c.in_order[k]) : 1.0;
+            for (int k = 0; k < 4; k++) {
+                xk[k] = k < n_in ? M.v[c.in_species[k] * NT] : 1.0;
+                pw[k] = k < n_in ? ipow(xk[k], c.in_order[k]) : 1.0;
+            }
             double orders = 1.0;
 #pragma unroll
             for (int k = 0; k < 4; k++)
                 if (k < n_in) orders *= pw[k];
             const double w = ap * orders * f * g;
-            omegas[r] = w;
+            M.omega[D.slot[r] * NT] = w;
             cell.nfe |= c.latch && w > 0.0;
+            double *grad = M.grad + D.ent0[r] * NT;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 if (k >= n_in) break;
                 const int j = c.in_species[k];
                 const double n = c.in_order[k];
-                if (n == 0.0) continue;
                 double oj = 1.0;
 #pragma unroll
                 for (int q = 0; q < 4; q++)
                     if (q < n_in) oj *= c.in_species[q] == j ? 1.0 : pw[q];
-                grad[r][j] += n * ipow(x[j], n - 1.0) * (ap * oj * f * g);
+                grad[k * NT] = n * ipow(xk[k], n - 1.0) * (ap * oj * f * g);
             }
+#pragma unroll
             for (int i = 0; i < NS; i++) s[i] += D.nu[r][i] * w;
             qdot += c.q * w;
             any |= w != 0.0;
@@ -336,11 +456,13 @@ __device__ void burn(const ReactDev &D, double sigma, const double *x0, double e
             enu = enu * k;
         }
         double s_max = 0.0;
+#pragma unroll
         for (int i = 0; i < NS; i++) s_max = fmax(s_max, fabs(s[i]));
         double h = t_rem;
         if (s_max > 0.0) h = fmin(h, P.burn_dx / s_max);
         if (!pin) {
             double dinv_mu = 0.0;
+#pragma unroll
             for (int i = 0; i < NS; i++) dinv_mu += s[i] * r_zp1_a[i];
             const double dt_dt = mu * (qdot - enu) - t * mu * dinv_mu;
             if (dt_dt != 0.0) h = fmin(h, P.burn_dt * t / fabs(dt_dt));
@@ -354,39 +476,46 @@ __device__ void burn(const ReactDev &D, double sigma, const double *x0, double e
             }
             const int last = h >= t_rem;
             const double h_use = fmin(h, t_rem);
-            double dx[NS], x_new[NS];
-            solve(D, grad, s, h_use, dx);
+            double dx[NS];
+            solve<NA, NT>(D, M, s, h_use, dx);
             double worst = 0.0;
             int negative = 0;
+#pragma unroll
             for (int i = 0; i < NS; i++) {
-                x_new[i] = x[i] + dx[i];
+                M.v[i * NT] = dx[i];
                 worst = fmax(worst, fabs(dx[i]));
-                if (x_new[i] < -1e-12) negative = 1;
+                dx[i] += x[i];  // the new fractions from here
+                if (dx[i] < -1e-12) negative = 1;
             }
             double de = 0.0, by_group[NG];
+#pragma unroll
             for (int g = 0; g < NG; g++) by_group[g] = 0.0;
             for (int r = 0; r < nr; r++) {
+                if (r == P.nfe) continue;
+                const sr_react_record &c = P.rec[r];
                 double lin = 0.0;
-                for (int j = 0; j < NS; j++) lin += grad[r][j] * dx[j];
-                const double xi = h_use * (omegas[r] + lin);
-                de += P.rec[r].q * xi;
-                by_group[P.rec[r].group] += P.rec[r].q * xi;
+                for (int q = 0; q < c.n_in; q++)
+                    lin += M.grad[(D.ent0[r] + q) * NT] * M.v[c.in_species[q] * NT];
+                const double e = c.q * (h_use * (M.omega[D.slot[r] * NT] + lin));
+                de += e;
+#pragma unroll
+                for (int g = 0; g < NG; g++)
+                    if (g == c.group) by_group[g] += e;
             }
             const double lost = enu * h_use;
             double sum = 0.0;
+#pragma unroll
             for (int i = 0; i < NS; i++) {
-                x_new[i] = fmax(x_new[i], 0.0);
-                sum += x_new[i];
+                dx[i] = fmax(dx[i], 0.0);
+                sum += dx[i];
             }
-            for (int i = 0; i < NS; i++) x_new[i] /= sum;
-            double mu_new, y_e_new, e_new, t_new;
-            comp(x_new, &mu_new, &y_e_new);
-            if (pin) {
-                e_new = e_tot;
-                t_new = t0;
-            } else {
+#pragma unroll
+            for (int i = 0; i < NS; i++) dx[i] /= sum;
+            double mu_new, y_e_new, e_new = e_tot, t_new = t0;
+            comp(dx, &mu_new, &y_e_new);
+            if (!pin) {
                 e_new = e_tot + de - lost;
-                t_new = mu_new * fmax(e_new - eps_cold_d(D, sigma, y_e_new, x_new[ID_N]), D.t_floor / mu_new);
+                t_new = mu_new * fmax(e_new - eps_cold_d(D, M, sigma, y_e_new, dx[ID_N]), D.t_floor / mu_new);
             }
             const double dt_rel = pin ? 0.0 : fabs(t_new - t) / t;
             const int bad = worst > P.burn_dx * (1.0 + 1e-12) || dt_rel > P.burn_dt * (1.0 + 1e-12) || negative;
@@ -395,10 +524,15 @@ __device__ void burn(const ReactDev &D, double sigma, const double *x0, double e
                 cell.retried += 1.0;
                 continue;
             }
-            for (int i = 0; i < NS; i++) x[i] = x_new[i];
+#pragma unroll
+            for (int i = 0; i < NS; i++) x[i] = dx[i];
             e_tot = e_new;
+            mu = mu_new;
+            y_e = y_e_new;
+            t = t_new;
             cell.de += de - lost;
             cell.lost += lost;
+#pragma unroll
             for (int g = 0; g < NG; g++) cell.booked[g] += by_group[g];
             cell.substeps += 1.0;
             cell.changed = 1;
@@ -410,64 +544,92 @@ __device__ void burn(const ReactDev &D, double sigma, const double *x0, double e
         }
         if (cell.unfinished) break;
     }
-    for (int s = 0; s < NS; s++) cell.x[s] = x[s];
     if (pin && cell.changed) {
-        double mu, y_e;
-        comp(x, &mu, &y_e);
         cell.pinned = 1;
-        cell.pinned_e = t0 / mu + eps_cold_d(D, sigma, y_e, x[ID_N]);
+        cell.pinned_e = t0 / mu + eps_cold_d(D, M, sigma, y_e, x[ID_N]);
     }
 }
 
-__global__ void __launch_bounds__(REACT_NT) k_react(const ReactDev *__restrict__ Dp, HydroState st, int n, double dt_arg,
-                                                   const double *__restrict__ scal, double *__restrict__ nuclear,
-                                                   double *__restrict__ lost, double *__restrict__ snu, double *psum,
-                                                   double *pmax) {
+// one thread per cell (a sum carried over more would hold 30 registers through the solve)
+template <int NA, int NT>
+__global__ void __launch_bounds__(NT, 2) k_react(const ReactDev *__restrict__ Dp, HydroState st, int n, double dt_arg,
+                                                      const double *__restrict__ scal, double *__restrict__ nuclear,
+                                                      double *__restrict__ lost, double *__restrict__ snu, double *psum,
+                                                      double *pmax) {
+    extern __shared__ double mem[];
     const ReactDev &D = *Dp;
+    const int nt = D.tables * REACT_TABLE, i = blockIdx.x * NT + threadIdx.x;
+    for (int k = threadIdx.x; k < 2 * COLD_POINTS; k += NT) mem[k] = (&D.cold_lnu[0][0])[k];
+    for (int k = threadIdx.x; k < nt; k += NT) mem[2 * COLD_POINTS + k] = (&D.ln_f[0][0])[k];
+    __syncthreads();
+    Lds M;
+    M.cold = mem;
+    M.ln_f = mem + 2 * COLD_POINTS;
+    M.v = mem + 2 * COLD_POINTS + nt + threadIdx.x;
+    M.omega = M.v + NS * NT;
+    M.grad = M.omega + D.slots * NT;
     const double dt = dt_arg >= 0.0 ? dt_arg : scal[0];
     double vs[REACT_SUMS], vm[REACT_MAXES];
     for (int k = 0; k < REACT_SUMS; k++) vs[k] = 0.0;
     for (int k = 0; k < REACT_MAXES; k++) vm[k] = 0.0;
-    for (int i = blockIdx.x * REACT_NT + threadIdx.x; i < n; i += gridDim.x * REACT_NT) {
-        for (int g = 0; g < NG; g++) nuclear[(size_t)g * n + i] = 0.0;
-        lost[i] = 0.0;
-        snu[i] = 0.0;
+    if (i < n) {
         const double sigma = st.sigma[i];
-        if (sigma < D.sigma_vac) continue;
         double x[NS];
+#pragma unroll
         for (int s = 0; s < NS; s++) x[s] = (double)st.x[(size_t)s * n + i];
-        const double mx = st.mx[i], my = st.my[i], e = st.e[i];
-        const double kinetic = 0.5 * (mx * mx + my * my) / (sigma * sigma);
-        const double e_tot = e / sigma - kinetic;
-        CellOut c;
-        burn(D, sigma, x, e_tot, dt, c);
-        vs[0] += c.substeps;
-        vs[1] += c.retried;
-        vs[2] += (double)c.unfinished;
-        vm[0] = fmax(vm[0], c.substeps);
-        vm[1] = fmax(vm[1], c.max_dx);
-        vm[2] = fmax(vm[2], c.max_dt_rel);
-        vm[3] = fmax(vm[3], (double)c.nfe);
-        if (!c.changed) continue;
-        for (int s = 0; s < NS; s++) st.x[(size_t)s * n + i] = (float)c.x[s];
-        st.e[i] = (float)(c.pinned ? sigma * (c.pinned_e + kinetic) : e + sigma * c.de);
-        for (int g = 0; g < NG; g++) {
-            const double b = sigma * c.booked[g];
-            nuclear[(size_t)g * n + i] = b;
-            vs[3 + g] += b;
+        CellOut c{};
+        if (!(sigma < D.sigma_vac)) {
+            const double mx = st.mx[i], my = st.my[i];
+            const double kinetic = 0.5 * (mx * mx + my * my) / (sigma * sigma);
+            burn<NA, NT>(D, M, sigma, x, st.e[i] / sigma - kinetic, dt, c);
+            vs[0] = c.substeps;
+            vs[1] = c.retried;
+            vs[2] = (double)c.unfinished;
+            vm[0] = c.substeps;
+            vm[1] = c.max_dx;
+            vm[2] = c.max_dt_rel;
+            vm[3] = (double)c.nfe;
+            if (c.changed) {
+#pragma unroll
+                for (int s = 0; s < NS; s++) st.x[(size_t)s * n + i] = (float)x[s];
+                st.e[i] = (float)(c.pinned ? sigma * (c.pinned_e + kinetic) : st.e[i] + sigma * c.de);
+            }
         }
-        lost[i] = sigma * c.lost;
-        vs[3 + NG] += sigma * c.lost;
-        if (c.x[ID_N] >= X_N_STAR && dt > 0.0) snu[i] = sigma * c.lost / dt;
+        // booked as the cell changed, zero elsewhere
+        const double on = c.changed ? sigma : 0.0;
+#pragma unroll
+        for (int g = 0; g < NG; g++) nuclear[(size_t)g * n + i] = vs[3 + g] = on * c.booked[g];
+        lost[i] = vs[3 + NG] = on * c.lost;
+        snu[i] = c.changed && x[ID_N] >= X_N_STAR && dt > 0.0 ? sigma * c.lost / dt : 0.0;
     }
     block_partials<REACT_SUMS>(vs, psum, gridDim.x);
     block_partials<REACT_MAXES, 1>(vm, pmax, gridDim.x);
 }
 
-int react_launch(const ReactDev *D, const HydroState &st, int n, double dt, const double *scal, double *nuclear,
-                 double *lost, double *snu, double *psum, double *pmax, int *nblocks, hipStream_t s) {
-    const int nb = std::max(1, std::min(REACT_BLOCKS, (n + REACT_NT - 1) / REACT_NT));
-    hipLaunchKernelGGL(k_react, dim3(nb), dim3(REACT_NT), 0, s, D, st, n, dt, scal, nuclear, lost, snu, psum, pmax);
+// whether the records' system leaves the neutrons out
+static bool react_neutrons(const ReactDev &h) {
+    unsigned any = h.row[ID_N];
+    for (int i = 0; i < NS; i++) any |= h.row[i] >> ID_N & 1;
+    for (int r = 0; r < h.P.n_records; r++)
+        if (r != h.P.nfe) any |= h.nu[r][ID_N] != 0.0;
+    return any != 0;
+}
+
+ReactLaunch react_plan(const ReactDev &h) {
+    auto lds = [&](int nt) {
+        return (int)sizeof(double) * (2 * COLD_POINTS + h.tables * REACT_TABLE + nt * (NS + h.slots + h.entries));
+    };
+    const int nt = lds(256) <= 78 * 1024 ? 256 : REACT_NT_LEAST;  // and 2 KB of partial sums
+    return {nt, lds(nt), react_neutrons(h)};
+}
+
+int react_launch(const ReactDev *D, const ReactLaunch &plan, const HydroState &st, int n, double dt, const double *scal,
+                 double *nuclear, double *lost, double *snu, double *psum, double *pmax, int *nblocks, hipStream_t s) {
+    const int nb = plan.blocks(n);
+    auto kernel = plan.nt == 256 ? (plan.neutrons ? k_react<NS, 256> : k_react<NS - 1, 256>)
+                                 : (plan.neutrons ? k_react<NS, REACT_NT_LEAST> : k_react<NS - 1, REACT_NT_LEAST>);
+    SR_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, plan.lds));
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(plan.nt), plan.lds, s, D, st, n, dt, scal, nuclear, lost, snu, psum, pmax);
     if (nblocks) *nblocks = nb;
     SR_HIP(hipGetLastError());
     return SR_OK;

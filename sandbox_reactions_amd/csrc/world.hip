@@ -399,6 +399,7 @@ struct sr_world {
     double *react_nuc = nullptr, *react_lost = nullptr, *react_snu = nullptr, *react_psum = nullptr,
            *react_pmax = nullptr;
     int react_nb = 0;
+    ReactLaunch react_plan{};
     bool sinks_on = false;  // P3 in the step
     SinkParams sk_par{};
     SinkBufs sk{};
@@ -849,7 +850,7 @@ static int one_step(sr_world *wd) {
     mark(wd, 12);
     if (wd->react) {  // P6 at the step's dt
         HydroState &st = wd->st[wd->cur];
-        SR_TRY(react_launch(wd->react, st, (int)wd->n, -1.0, wd->scal, wd->react_nuc, wd->react_lost, wd->react_snu,
+        SR_TRY(react_launch(wd->react, wd->react_plan, st, (int)wd->n, -1.0, wd->scal, wd->react_nuc, wd->react_lost, wd->react_snu,
                             wd->react_psum, wd->react_pmax, &wd->react_nb, s));
     }
     mark(wd, 4);
@@ -1073,16 +1074,19 @@ extern "C" int sr_set_reactions(sr_world *wd, const sr_react_params *p) {
         SR_TRY(world_alloc(wd, (void **)&wd->react_nuc, sizeof(double) * SR_REACT_GROUPS * n));
         SR_TRY(world_alloc(wd, (void **)&wd->react_lost, sizeof(double) * n));
         SR_TRY(world_alloc(wd, (void **)&wd->react_snu, sizeof(double) * n));
-        SR_TRY(world_alloc(wd, (void **)&wd->react_psum, sizeof(double) * REACT_SUMS * REACT_BLOCKS));
-        SR_TRY(world_alloc(wd, (void **)&wd->react_pmax, sizeof(double) * REACT_MAXES * REACT_BLOCKS));
+        const size_t most = (n + REACT_NT_LEAST - 1) / REACT_NT_LEAST;  // blocks
+        SR_TRY(world_alloc(wd, (void **)&wd->react_psum, sizeof(double) * REACT_SUMS * most));
+        SR_TRY(world_alloc(wd, (void **)&wd->react_pmax, sizeof(double) * REACT_MAXES * most));
     }
     ReactDev *h = new ReactDev;
     react_build(p, wd->ph, h);
+    const ReactLaunch plan = react_plan(*h);
     const hipError_t e = hipMemcpyAsync(wd->react_dev_mem, h, sizeof(ReactDev), hipMemcpyHostToDevice, wd->s);
     const hipError_t e2 = e == hipSuccess ? hipStreamSynchronize(wd->s) : e;
     delete h;
     if (e2 != hipSuccess) return fail(SR_ERR_DEVICE, std::string("sr_set_reactions: ") + hipGetErrorString(e2));
     wd->react = wd->react_dev_mem;
+    wd->react_plan = plan;
     return SR_OK;
 }
 
@@ -1090,7 +1094,7 @@ extern "C" int sr_react_apply(sr_world *wd, double dt) {
     if (!wd) return fail(SR_ERR_ARGUMENT, "null world");
     if (!wd->react) return fail(SR_ERR_ARGUMENT, "sr_react_apply: no reactions (sr_set_reactions)");
     if (!(dt >= 0.0) || !std::isfinite(dt)) return fail(SR_ERR_ARGUMENT, "sr_react_apply: dt >= 0 is required");
-    SR_TRY(react_launch(wd->react, wd->st[wd->cur], (int)wd->n, dt, wd->scal, wd->react_nuc, wd->react_lost,
+    SR_TRY(react_launch(wd->react, wd->react_plan, wd->st[wd->cur], (int)wd->n, dt, wd->scal, wd->react_nuc, wd->react_lost,
                         wd->react_snu, wd->react_psum, wd->react_pmax, &wd->react_nb, wd->s));
     SR_HIP(hipStreamSynchronize(wd->s));
     return SR_OK;

@@ -317,3 +317,47 @@ def test_the_burning_field_is_the_oracles(gpu_lib, dt):
     assert (np.abs(p[3] - o[3]) / np.abs(o[3])).max() <= 1e-5
     assert np.abs(nuc - onuc).sum() <= 1e-5 * np.abs(onuc).sum()
     assert abs(rep.substeps - orep.substeps) <= 1e-3 * orep.substeps
+
+
+def plain_record(rec, ins, outs, a):
+    """A record of no temperature law: (species, share, order) in, (species, share) out, omega = a prod X^n."""
+    rec.n_in, rec.n_out, rec.n_terms, rec.gated, rec.latch, rec.group = len(ins), len(outs), 0, 0, 0, 1
+    rec.q, rec.a_coef, rec.a_sigma, rec.t_thr = 10.0, a, 0.0, 0.0
+    for k, (sp, share, order) in enumerate(ins):
+        rec.in_species[k], rec.in_share[k], rec.in_order[k] = SP.index(sp), share, order
+    for k, (sp, share) in enumerate(outs):
+        rec.out_species[k], rec.out_share[k] = SP.index(sp), share
+
+
+# a catalyst (H + 0.5 He -> 0.5 He + C: helium's row is the identity while carbon's holds -h A X_H = -7, so the linear
+# system needs a row exchange); a system that holds the neutrons (iron to neutrons at order 2, not N_Fe's closed form);
+# the most inputs that the records allow (16 records of four), which take the smaller block
+@pytest.mark.parametrize("kind", ["catalyst", "neutrons", "many"])
+def test_general_records_are_the_oracles(gpu_lib, kind):
+    p = react.params(only=[])
+    if kind == "catalyst":
+        p.n_records = 1
+        plain_record(p.rec[0], [("H", 1.0, 1.0), ("He", 0.5, 1.0)], [("He", 0.5), ("C", 1.0)], 20.0)
+    elif kind == "neutrons":
+        p.n_records = 2
+        plain_record(p.rec[0], [("Fe", 1.0, 2.0)], [("n", 1.0)], 0.5)
+        plain_record(p.rec[1], [("n", 0.5, 1.0), ("H", 0.5, 1.0)], [("He", 1.0)], 0.7)
+    else:
+        p.n_records = 16
+        for k in range(16):
+            plain_record(p.rec[k], [(sp, 0.25, 1.0 + (k + j) % 2) for j, sp in enumerate(("H", "He", "C", "O"))],
+                         [("Ne", 0.5), ("Mg", 0.25), ("Si", 0.25)], 0.3 * (k + 1))
+    fractions = {"catalyst": [("H", 0.7), ("He", 0.005), ("O", 0.295)],
+                 "neutrons": [("H", 0.3), ("Fe", 0.5), ("n", 0.2)],
+                 "many": [("H", 0.3), ("He", 0.2), ("C", 0.3), ("O", 0.2)]}[kind]
+    cells = [(1.0 + 0.3 * i, 100.0, x_of(fractions)) for i in range(40)]
+    r = Rig(gpu_lib, p, cells)
+    o = np.ascontiguousarray(r.planes())
+    rep = r.run(0.5)
+    orep, onuc, _, _ = oracle.react_step(oracle.reference_physics(), p, o, 0.5)
+    got = r.planes()
+    assert rep.substeps == orep.substeps and rep.retried == orep.retried and rep.unfinished == 0
+    assert np.abs(got[4:] - o[4:]).max() <= 1e-6  # f32 planes of f64 steps
+    assert (np.abs(got[3] - o[3]) <= 1e-6 * np.maximum(np.abs(o[3]), 1e-30)).all()
+    nuc, _, _ = r.world.read_react_planes()
+    assert np.abs(nuc - onuc.reshape(nuc.shape)).max() <= 1e-9 * np.abs(onuc).max()
