@@ -12,6 +12,7 @@
 #include <mutex>
 #include <thread>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -21,46 +22,155 @@ namespace sr {
 
 // -------------------------------------------------------------------------------------------------------- kernels
 
-// Rows y in [0, h) of sigma (masked at sigma_vac), zero-padded to px reals, forward real FFT; spectrum bins
-// k in [0, px/2] written column-major: spec[k * ld + y].
-template <typename TIn>
-__global__ void __launch_bounds__(256) k_rows_r2c(const TIn *__restrict__ sigma, int w, int h, TIn sigma_vac,
-                                                  int px, int logL, int rb, const float2 *__restrict__ tw,
-                                                  int tw_stride_half, int tw_stride_full, float2 *__restrict__ spec,
-                                                  int ld) {
-    extern __shared__ float2 lds[];
-    const int L = 1 << logL;
-    float2 *a = lds, *b = lds + rb * L;
-    // row groups remapped so that each XCD takes one contiguous run of them: the groups that share a bin's cache
-    // line of the column-major spectrum then write it through the same L2
-    const int y0 = xcd_tile() * rb;
-    for (int t = threadIdx.x; t < rb * L; t += blockDim.x) {
-        const int r = t >> logL, m = t & (L - 1), y = y0 + r;
-        float2 v = make_float2(0.f, 0.f);
-        if (y < h) {
-            const int x0 = 2 * m, x1 = 2 * m + 1;
-            if (x0 < w) {
-                const TIn s = sigma[(size_t)y * w + x0];
-                v.x = s >= sigma_vac ? (float)s : 0.f;
-            }
-            if (x1 < w) {
-                const TIn s = sigma[(size_t)y * w + x1];
-                v.y = s >= sigma_vac ? (float)s : 0.f;
+// ---- The convolution's transforms: a sequence of N = 2^LOGN points lies in the registers of T = N / E threads, E = 16 (8
+// below 1024, 4 below 64) to a thread: thread t holds the points t + i T, before and after the transform alike, so that a
+// forward transform's result is an inverse's input in place. Stockham passes of radix E (the last of what is left) between
+// which the points cross through LDS: three passes and two crossings at 4096 points, where radix 4 from LDS to LDS took
+// six passes. One buffer a sequence, an entry of padding every 16: a wave's reads and writes spread over the banks.
+template <int LOGN> struct Fft {
+    static constexpr int N = 1 << LOGN, E = LOGN >= 10 ? 16 : LOGN >= 6 ? 8 : 4, T = N / E;
+    static constexpr int LDS = N + N / 16;  // a sequence's entries
+};
+__device__ __forceinline__ int fft_at(int i) { return i + (i >> 4); }
+
+template <bool INV> __device__ __forceinline__ void dft2(float2 &a, float2 &b) {
+    const float2 t = a;
+    a = cadd(t, b);
+    b = csub(t, b);
+}
+template <bool INV> __device__ __forceinline__ void dft4(float2 &a, float2 &b, float2 &c, float2 &d) {
+    const float2 s0 = cadd(a, c), s1 = csub(a, c), s2 = cadd(b, d), s3 = crot(csub(b, d), INV);
+    a = cadd(s0, s2);
+    b = cadd(s1, s3);
+    c = csub(s0, s2);
+    d = csub(s1, s3);
+}
+// the DFT of v[0], v[S], ... v[(R - 1) S] in place, natural order
+template <int R, int S, bool INV> __device__ __forceinline__ void dft(float2 *v) {
+    constexpr float C8 = 0.70710678118654752f, C1 = 0.92387953251128674f, S1 = 0.38268343236508977f;
+    if constexpr (R == 2) {
+        dft2<INV>(v[0], v[S]);
+    } else if constexpr (R == 4) {
+        dft4<INV>(v[0], v[S], v[2 * S], v[3 * S]);
+    } else if constexpr (R == 8) {
+        float2 e[4] = {v[0], v[2 * S], v[4 * S], v[6 * S]}, o[4] = {v[S], v[3 * S], v[5 * S], v[7 * S]};
+        dft4<INV>(e[0], e[1], e[2], e[3]);
+        dft4<INV>(o[0], o[1], o[2], o[3]);
+        o[1] = cmul(o[1], make_float2(C8, INV ? C8 : -C8));
+        o[2] = crot(o[2], INV);
+        o[3] = cmul(o[3], make_float2(-C8, INV ? C8 : -C8));
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            v[k * S] = cadd(e[k], o[k]);
+            v[(k + 4) * S] = csub(e[k], o[k]);
+        }
+    } else {
+        static_assert(R == 16, "radices 2, 4, 8, 16");
+        // index 4 m1 + m0 in, q0 + 4 q1 out: columns m0 over m1, the twiddles W16^(m0 q0), rows over m0
+        float2 c[4][4];
+#pragma unroll
+        for (int m0 = 0; m0 < 4; m0++) {
+#pragma unroll
+            for (int m1 = 0; m1 < 4; m1++) c[m0][m1] = v[(4 * m1 + m0) * S];
+            dft4<INV>(c[m0][0], c[m0][1], c[m0][2], c[m0][3]);
+        }
+        const float sg = INV ? 1.0f : -1.0f;
+        c[1][1] = cmul(c[1][1], make_float2(C1, sg * S1));
+        c[1][2] = cmul(c[1][2], make_float2(C8, sg * C8));
+        c[1][3] = cmul(c[1][3], make_float2(S1, sg * C1));
+        c[2][1] = cmul(c[2][1], make_float2(C8, sg * C8));
+        c[2][2] = crot(c[2][2], INV);
+        c[2][3] = cmul(c[2][3], make_float2(-C8, sg * C8));
+        c[3][1] = cmul(c[3][1], make_float2(S1, sg * C1));
+        c[3][2] = cmul(c[3][2], make_float2(-C8, sg * C8));
+        c[3][3] = cmul(c[3][3], make_float2(-C1, -sg * S1));
+#pragma unroll
+        for (int q0 = 0; q0 < 4; q0++) {
+            dft4<INV>(c[0][q0], c[1][q0], c[2][q0], c[3][q0]);
+#pragma unroll
+            for (int q1 = 0; q1 < 4; q1++) v[(q0 + 4 * q1) * S] = c[q1][q0];
+        }
+    }
+}
+
+// the passes from stride NS on (NS points already combined); every thread of the block takes part (barriers)
+template <int LOGN, int LOGNS, bool INV>
+__device__ __forceinline__ void fft_passes(float2 *v, float2 *lds, int t, const float2 *__restrict__ tw, int tw_stride) {
+    using F = Fft<LOGN>;
+    constexpr int NS = 1 << LOGNS, R = F::N / NS < F::E ? F::N / NS : F::E, B = F::E / R;
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+        const int k = (t + b * F::T) & (NS - 1);
+        if constexpr (NS > 1) {
+#pragma unroll
+            for (int m = 1; m < R; m++) {
+                float2 w = tw[(k * m * (F::N / (NS * R))) * tw_stride];
+                if (INV) w = cconj(w);
+                v[b + m * B] = cmul(v[b + m * B], w);
             }
         }
-        a[t] = v;
+        dft<R, B, INV>(v + b);
     }
-    __syncthreads();
-    float2 *Z = lds_fft(a, b, L, logL, rb, tw, tw_stride_half, false);
+    if constexpr (NS * R < F::N) {
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            const int j = t + b * F::T, k = j & (NS - 1);
+#pragma unroll
+            for (int q = 0; q < R; q++) lds[fft_at((j - k) * R + k + q * NS)] = v[b + q * B];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < F::E; i++) v[i] = lds[fft_at(t + i * F::T)];
+        constexpr int NEXT = LOGNS + (R == 16 ? 4 : R == 8 ? 3 : R == 4 ? 2 : 1);
+        fft_passes<LOGN, NEXT, INV>(v, lds, t, tw, tw_stride);
+    }
+}
+
+// Rows y in [0, h) of sigma (masked at sigma_vac), zero-padded to px = 2 L reals, forward real FFT; spectrum bins
+// k in [0, L] written column-major: spec[k * ld + y]. A block takes rb rows of T threads each.
+template <typename TIn, int LOGL>
+__global__ void k_rows_r2c(const TIn *__restrict__ sigma, int w, int h, TIn sigma_vac, int rb,
+                           const float2 *__restrict__ tw, int tw_stride_half, int tw_stride_full,
+                           float2 *__restrict__ spec, int ld) {
+    using F = Fft<LOGL>;
+    extern __shared__ float2 lds[];
+    constexpr int L = F::N;
+    // row groups remapped so that each XCD takes one contiguous run of them: the groups that share a bin's cache
+    // line of the column-major spectrum then write it through the same L2
+    const int y0 = xcd_tile() * rb, t = threadIdx.x % F::T;
+    {
+        const int r = threadIdx.x / F::T, y = y0 + r;
+        float2 v[F::E];
+        float2 *row = lds + r * F::LDS;
+#pragma unroll
+        for (int i = 0; i < F::E; i++) {
+            const int x = 2 * (t + i * F::T);
+            v[i] = make_float2(0.f, 0.f);
+            if (y < h && x < w) {
+                const TIn s = sigma[(size_t)y * w + x];
+                v[i].x = s >= sigma_vac ? (float)s : 0.f;
+                if (x + 1 < w) {
+                    const TIn s1 = sigma[(size_t)y * w + x + 1];
+                    v[i].y = s1 >= sigma_vac ? (float)s1 : 0.f;
+                }
+            }
+        }
+        fft_passes<LOGL, 0, false>(v, row, t, tw, tw_stride_half);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < F::E; i++) row[fft_at(t + i * F::T)] = v[i];
+        __syncthreads();
+    }
     // X[k] = (Z_k + conj Z_{L-k}) / 2 - i/2 W^k (Z_k - conj Z_{L-k}),  W = e^{-2 pi i / px}
     // Consecutive lanes take consecutive rows of one bin, so each bin's rb rows go out as one contiguous segment of
     // the column-major spectrum (rather than one 8-byte value per lane at stride ld).
-    const int nk = L + 1;
-    for (int t = threadIdx.x; t < rb * nk; t += blockDim.x) {
-        const int k = t / rb, r = t - k * rb, y = y0 + r;
+    for (int q = threadIdx.x; q < rb * (L + 1); q += blockDim.x) {
+        const int k = q / rb, r = q - k * rb, y = y0 + r;
         if (y >= h) continue;
-        const float2 zk = Z[r * L + (k & (L - 1))];
-        const float2 zc = cconj(Z[r * L + ((L - k) & (L - 1))]);
+        const float2 *Z = lds + r * F::LDS;
+        const float2 zk = Z[fft_at(k & (L - 1))];
+        const float2 zc = cconj(Z[fft_at((L - k) & (L - 1))]);
         const float2 e = make_float2(0.5f * (zk.x + zc.x), 0.5f * (zk.y + zc.y));
         const float2 d = make_float2(0.5f * (zk.x - zc.x), 0.5f * (zk.y - zc.y));
         const float2 wk = tw[k * tw_stride_full];
@@ -70,69 +180,90 @@ __global__ void __launch_bounds__(256) k_rows_r2c(const TIn *__restrict__ sigma,
     }
 }
 
-// One spectral column per block: forward FFT of length py (rows >= h are zero), multiply by the kernel spectrum
-// (real, even; quarter table with (py/2 + 1) entries per column, already divided by px * py), inverse FFT, write the
-// ring rows -1..h as out[k * ldo + j], j = y + 1.
-__global__ void __launch_bounds__(256) k_columns(const float2 *__restrict__ spec, int ld, int h, int py, int logpy,
-                                                 const float *__restrict__ khat, const float2 *__restrict__ tw,
-                                                 int tw_stride, float2 *__restrict__ out, int ldo) {
+// Spectral columns, T threads each and as many to a block as make a wave: forward FFT of length py (rows >= h are zero),
+// multiply by the kernel spectrum (real, even; quarter table with (py/2 + 1) entries per column, already divided by
+// px * py), inverse FFT, write the ring rows -1..h as out[k * ldo + j], j = y + 1. A column comes from and goes to global
+// memory through the registers. At 2048^2 (py 4096) 54 us, 154 with
+// radix-4 passes in LDS; the row transforms 31 us each way, 61 and 50.
+template <int LOGN>
+__global__ void __launch_bounds__(256) k_columns(const float2 *__restrict__ spec, int ld, int h, int ncols, const float *__restrict__ khat,
+                          const float2 *__restrict__ tw, int tw_stride, float2 *__restrict__ out, int ldo) {
+    using F = Fft<LOGN>;
     extern __shared__ float2 lds[];
-    float2 *a = lds, *b = lds + py;
-    const int k = blockIdx.x;
+    constexpr int N = F::N;
+    const int c = threadIdx.x / F::T, t = threadIdx.x % F::T;
+    const int k = min(blockIdx.x * ((int)blockDim.x / F::T) + c, ncols - 1);  // past the last: the last again
+    float2 *buf = lds + c * F::LDS;
+    float2 v[F::E];
     const float2 *col = spec + (size_t)k * ld;
-    for (int y = threadIdx.x; y < py; y += blockDim.x) a[y] = y < h ? col[y] : make_float2(0.f, 0.f);
-    __syncthreads();
-    float2 *F = lds_fft(a, b, py, logpy, 1, tw, tw_stride, false);
-    float2 *G = (F == a) ? b : a;
-    const float *kq = khat + (size_t)k * (py / 2 + 1);
-    for (int ky = threadIdx.x; ky < py; ky += blockDim.x) {
-        const float s = kq[ky <= py / 2 ? ky : py - ky];
-        const float2 f = F[ky];
-        F[ky] = make_float2(f.x * s, f.y * s);
+    const float *kq = khat + (size_t)k * (N / 2 + 1);
+    float kv[F::E];
+#pragma unroll
+    for (int i = 0; i < F::E; i++) {
+        const int y = t + i * F::T;
+        v[i] = y < h ? col[y] : make_float2(0.f, 0.f);
+        kv[i] = kq[y <= N / 2 ? y : N - y];
     }
-    __syncthreads();
-    float2 *R = lds_fft(F, G, py, logpy, 1, tw, tw_stride, true);
+    fft_passes<LOGN, 0, false>(v, buf, t, tw, tw_stride);
+#pragma unroll
+    for (int i = 0; i < F::E; i++) v[i] = make_float2(v[i].x * kv[i], v[i].y * kv[i]);
+    int ti = t;
+    asm volatile("" : "+v"(ti));  // the inverse's twiddles loaded again: kept, they would take 60 registers
+    fft_passes<LOGN, 0, true>(v, buf, ti, tw, tw_stride);
     float2 *o = out + (size_t)k * ldo;
-    for (int j = threadIdx.x; j < h + 2; j += blockDim.x) {
-        const int y = j == 0 ? py - 1 : j - 1;
-        o[j] = R[y];
+#pragma unroll
+    for (int i = 0; i < F::E; i++) {
+        const int y = t + i * F::T;
+        if (y <= h) o[y + 1] = v[i];
+        if (y == N - 1) o[0] = v[i];
     }
 }
 
-// Rows j in [0, h+2) of the ringed output: gather bins k in [0, px/2] from the column-major buffer, inverse real
-// FFT (unnormalised), write phi_ringed[j][i] for i = 0 (x = -1), 1..w (x = 0..w-1), w+1 (x = w).
-__global__ void __launch_bounds__(256) k_rows_c2r(const float2 *__restrict__ in, int ldi, int nrows, int w, int px,
-                                                  int logL, int rb, const float2 *__restrict__ tw, int tw_stride_half,
-                                                  int tw_stride_full, float *__restrict__ phi) {
+// Rows j in [0, h+2) of the ringed output: gather bins k in [0, L] from the column-major buffer, inverse real
+// FFT (unnormalised), write phi_ringed[j][i] for i = 0 (x = -1), 1..w (x = 0..w-1), w+1 (x = w). A block takes rb rows of
+// T threads each.
+template <int LOGL>
+__global__ void k_rows_c2r(const float2 *__restrict__ in, int ldi, int nrows, int w, int rb,
+                           const float2 *__restrict__ tw, int tw_stride_half, int tw_stride_full,
+                           float *__restrict__ phi) {
+    using F = Fft<LOGL>;
     extern __shared__ float2 lds[];
-    const int L = 1 << logL;
-    float2 *a = lds, *b = lds + rb * L;
+    constexpr int L = F::N;
     const int j0 = xcd_tile() * rb;  // as in k_rows_r2c: a bin's cache line read through one XCD's L2
     // Z_k = (X_k + conj X_{L-k}) + i W^{-k} (X_k - conj X_{L-k}), k in [0, L). Consecutive lanes take consecutive
     // rows of one bin, so the gather reads each bin's rb rows (and its mirror's) as contiguous segments of the
-    // column-major buffer.
-    for (int t = threadIdx.x; t < rb * L; t += blockDim.x) {
-        const int k = t / rb, r = t - k * rb, j = j0 + r;
-        float2 v = make_float2(0.f, 0.f);
+    // column-major buffer; X_k and X_{L-k} make Z_k and Z_{L-k} both, so each is read once.
+    for (int q = threadIdx.x; q < rb * (L / 2 + 1); q += blockDim.x) {
+        const int k = q / rb, r = q - k * rb, j = j0 + r;
+        float2 v = make_float2(0.f, 0.f), u = v;
         if (j < nrows) {
-            const float2 xk = in[(size_t)k * ldi + j];
-            const float2 xc = cconj(in[(size_t)(L - k) * ldi + j]);
+            const float2 xk = in[(size_t)k * ldi + j], xm = in[(size_t)(L - k) * ldi + j];
+            const float2 xc = cconj(xm);
             const float2 s = cadd(xk, xc), d = csub(xk, xc);
-            const float2 wk = cconj(tw[k * tw_stride_full]);
-            const float2 wd = cmul(wk, d);
+            const float2 wd = cmul(cconj(tw[k * tw_stride_full]), d);
             v = make_float2(s.x - wd.y, s.y + wd.x); // s + i * wd
+            // the mirror bin: s and d conjugated (d negated), W^{-(L-k)} = -W^k
+            u = make_float2(s.x + wd.y, -(s.y - wd.x));
         }
-        a[r * L + k] = v;
+        float2 *row = lds + r * F::LDS;
+        row[fft_at(k)] = v;
+        if (k > 0) row[fft_at(L - k)] = u;
     }
     __syncthreads();
-    float2 *z = lds_fft(a, b, L, logL, rb, tw, tw_stride_half, true);
-    const int rw = w + 2;
-    for (int t = threadIdx.x; t < rb * rw; t += blockDim.x) {
-        const int r = t / rw, i = t - r * rw, j = j0 + r;
-        if (j >= nrows) continue;
-        const int n = i == 0 ? px - 1 : i - 1;
-        const float2 v = z[r * L + (n >> 1)];
-        phi[(size_t)j * rw + i] = (n & 1) ? v.y : v.x;
+    const int r = threadIdx.x / F::T, t = threadIdx.x % F::T, j = j0 + r;
+    float2 *row = lds + r * F::LDS;
+    float2 v[F::E];
+#pragma unroll
+    for (int i = 0; i < F::E; i++) v[i] = row[fft_at(t + i * F::T)];
+    fft_passes<LOGL, 0, true>(v, row, t, tw, tw_stride_half);
+    if (j >= nrows) return;
+    float *o = phi + (size_t)j * (w + 2);
+#pragma unroll
+    for (int i = 0; i < F::E; i++) {
+        const int n = 2 * (t + i * F::T);
+        if (n <= w) o[n + 1] = v[i].x;
+        if (n + 1 <= w) o[n + 2] = v[i].y;
+        if (n + 2 == 2 * L) o[0] = v[i].y;
     }
 }
 
@@ -320,27 +451,74 @@ int Gravity::init(int w_, int h_, double G_, double dx_, double sigma_vac_, int 
     return SR_OK;
 }
 
-static int rows_per_block(int L) { return std::max(1, std::min(8, 4096 / L)); }
+// f with the transform's log2 length as a compile-time constant
+template <typename Fn> static int fft_length(int logn, Fn f) {
+    switch (logn) {
+    case 4: return f(std::integral_constant<int, 4>());
+    case 5: return f(std::integral_constant<int, 5>());
+    case 6: return f(std::integral_constant<int, 6>());
+    case 7: return f(std::integral_constant<int, 7>());
+    case 8: return f(std::integral_constant<int, 8>());
+    case 9: return f(std::integral_constant<int, 9>());
+    case 10: return f(std::integral_constant<int, 10>());
+    case 11: return f(std::integral_constant<int, 11>());
+    case 12: return f(std::integral_constant<int, 12>());
+    default: return fail(SR_ERR_BOX_AXIS, "a transform of 2^" + std::to_string(logn) + " points");
+    }
+}
+
+// the rows a block can take: up to 8, at most 1024 threads and the LDS a block may have
+static bool rows_fit(int logl, int rb) {
+    return fft_length(logl, [&](auto c) {
+               using F = Fft<decltype(c)::value>;
+               return rb <= 8 && rb * F::T <= 1024 && sizeof(float2) * rb * F::LDS <= (size_t)max_lds_bytes() ? 1 : 0;
+           }) == 1;
+}
+
+// Rows per block without the autotuner: the most (8: a bin's rows go out 64 bytes at a time) that still make
+// ROWS_FILL blocks, two (16 bytes) at least.
+#define ROWS_FILL 256
+static int rows_per_block(int logl, int h) {
+    int rb = 1;
+    while (rows_fit(logl, 2 * rb) && (rb < 2 || (h + 2 * rb - 1) / (2 * rb) >= ROWS_FILL)) rb *= 2;
+    return rb;
+}
 
 template <typename TIn> int Gravity::potential(const TIn *sigma, float *phi_ringed, hipStream_t s) {
-    const int L = px / 2, logL = ilog2(L), logpy = ilog2(py);
-    const int rb = this->rb > 0 ? this->rb : rows_per_block(L);
+    const int L = px / 2, logL = ilog2(L), logpy = ilog2(py), ncols = px / 2 + 1;
+    const int rb = this->rb > 0 ? this->rb : rows_per_block(logL, h);
     const int stride_half = nmax / L, stride_full = nmax / px;
-    hipLaunchKernelGGL(k_rows_r2c<TIn>, dim3((h + rb - 1) / rb), dim3(256), sizeof(float2) * 2 * rb * L, s, sigma, w,
-                       h, (TIn)sigma_vac, px, logL, rb, tw, stride_half, stride_full, spec, ld_spec);
-    hipLaunchKernelGGL(k_columns, dim3(px / 2 + 1), dim3(256), sizeof(float2) * 2 * py, s, spec, ld_spec, h, py,
-                       logpy, khat, tw, nmax / py, cols, ld_cols);
-    hipLaunchKernelGGL(k_rows_c2r, dim3((h + 2 + rb - 1) / rb), dim3(256), sizeof(float2) * 2 * rb * L, s, cols,
-                       ld_cols, h + 2, w, px, logL, rb, tw, stride_half, stride_full, phi_ringed);
+    SR_TRY(fft_length(logL, [&](auto c) {
+        using F = Fft<decltype(c)::value>;
+        hipLaunchKernelGGL((k_rows_r2c<TIn, decltype(c)::value>), dim3((h + rb - 1) / rb), dim3(rb * F::T),
+                           sizeof(float2) * rb * F::LDS, s, sigma, w, h, (TIn)sigma_vac, rb, tw, stride_half,
+                           stride_full, spec, ld_spec);
+        return SR_OK;
+    }));
+    SR_TRY(fft_length(logpy, [&](auto c) {
+        using F = Fft<decltype(c)::value>;
+        constexpr int cpb = F::T < 64 ? 64 / F::T : 1;
+        hipLaunchKernelGGL((k_columns<decltype(c)::value>), dim3((ncols + cpb - 1) / cpb), dim3(cpb * F::T),
+                           sizeof(float2) * cpb * F::LDS, s, spec, ld_spec, h, ncols, khat, tw, nmax / py, cols,
+                           ld_cols);
+        return SR_OK;
+    }));
+    SR_TRY(fft_length(logL, [&](auto c) {
+        using F = Fft<decltype(c)::value>;
+        hipLaunchKernelGGL((k_rows_c2r<decltype(c)::value>), dim3((h + 2 + rb - 1) / rb), dim3(rb * F::T),
+                           sizeof(float2) * rb * F::LDS, s, cols, ld_cols, h + 2, w, rb, tw, stride_half, stride_full,
+                           phi_ringed);
+        return SR_OK;
+    }));
     SR_HIP(hipGetLastError());
     return SR_OK;
 }
 
-// Rows per block 1, 2, 4 or 8 (as the LDS allows two rb x px/2 complex arrays), each timed as the best of three means
+// Rows per block 1, 2, 4 or 8 (as the LDS and the block size allow), each timed as the best of three means
 // of four convolutions between two events after one to warm; the heuristic's count is kept unless another is 3 %
 // faster.
 int Gravity::tune(const float *sigma, float *phi_ringed, hipStream_t s) {
-    const int L = px / 2, heur = rows_per_block(L);
+    const int logL = ilog2(px / 2), heur = rows_per_block(logL, h);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     SR_HIP(hipEventCreate(&e0));
     SR_HIP(hipEventCreate(&e1));
@@ -349,7 +527,7 @@ int Gravity::tune(const float *sigma, float *phi_ringed, hipStream_t s) {
     int rc = SR_OK;
     std::vector<int> cand = {heur};
     for (int r : {1, 2, 4, 8})
-        if (r != heur && (size_t)2 * r * L * sizeof(float2) <= (size_t)max_lds_bytes()) cand.push_back(r);
+        if (r != heur && rows_fit(logL, r)) cand.push_back(r);
     for (int r : cand) {
         rb = r;
         float ms = 0.0f;

@@ -93,3 +93,20 @@ def test_refusals(gpu_lib):
     with pytest.raises(gpu_lib.SrError) as e:
         gpu_lib.Gravity(3000, 64, max_padded=4096)
     assert e.value.kind == "BoxAxis"
+
+
+# one box per transform length of rows and columns (16 to 4096 points), odd sides among them, with rows left over in the
+# last block, and a box whose padded rows are twice the default cap
+@pytest.mark.parametrize("w,h,cap", [(3, 5, 4096), (16, 33, 4096), (33, 16, 4096), (65, 70, 4096), (130, 140, 4096),
+                                     (257, 300, 4096), (601, 520, 4096), (1030, 1100, 4096), (2048, 37, 4096),
+                                     (2100, 40, 8192)])
+def test_gravity_field_at_every_transform_length(gpu_lib, w, h, cap):
+    import torch
+    print(f"gravity {w}x{h}", flush=True)
+    sigma = np.random.default_rng(w + 7 * h).uniform(0.0, 1.0, (h, w)).astype(np.float32)
+    ph = oracle.reference_physics(G=1.0, dx=1.0, sigma_vac=1e-6, max_padded=cap)
+    phi, gx, gy, pr = oracle.gravity_field(ph, sigma.astype(np.float64), ringed=True)
+    gphi, ggx, ggy = gpu_lib.Gravity(w, h, max_padded=cap).field(torch.tensor(sigma, device="cuda"))
+    # f32 transforms: 1e-6 of phi (a few roundings per pass), g by its difference as above
+    assert rel_l2(gphi.cpu().numpy(), pr) < 1e-6
+    assert rel_l2(ggx.cpu().numpy(), gx) < 1e-4 and rel_l2(ggy.cpu().numpy(), gy) < 1e-4
