@@ -34,6 +34,12 @@ namespace sr {
 #define COARSE_NT 1024
 #define COARSE_LDS (150 * 1024)
 #define DENSE_MAX 16
+// Level 0's smoothers take 16x16 tiles on grids of fewer 32x32 tiles than this: those leave CUs idle, and a tile's
+// serial sweeps (its cells over the block's lanes) are the launch's time. One PCG iteration of a solve, 32x32 against
+// 16x16 tiles: 42.7 / 34.6 us at 128^2, 50.4 / 43.6 at 256^2, 57.9 / 52.7 at 500 x 300, 59.2 / 57.4 at 512^2, 75.3 /
+// 72.3 at 608^2 (361 tiles); beyond it the 16x16 tiles' wider halos cost more than they fill: 75.1 / 78.1 at 700^2 (484),
+// 91.2 / 115 at 1024^2. The results are the same bits but for the order of the dot products' partials.
+#define TILE0_FILL 384
 #define NET_RATE_AT 4 // learned iterations before its residual rate is compared with plain multigrid's
 // Restarts of the inner FP32 loop from the FP64 true residual before a solve gives up: where the FP32 inner solves
 // cannot carry the true residual below the goal (a goal at the edge of what they resolve), a Newton pass takes the
@@ -1599,7 +1605,9 @@ int FldSolver::init(int w, int h, int levels, int nu1_, int nu2_, double omega_)
     post_tile.assign(coarse_from, TILE_32);
     for (int l = 1; l < coarse_from; l++)
         if (((lv[l].w + 31) / 32) * ((lv[l].h + 31) / 32) < 512) pre_tile[l] = post_tile[l] = TILE_16;
-    ntiles0 = ((w + 31) / 32) * ((h + 31) / 32);
+    tile0 = ((w + 31) / 32) * ((h + 31) / 32) < TILE0_FILL ? TILE_16 : TILE_32;
+    const int t0 = tile0 == TILE_16 ? 16 : 32;
+    ntiles0 = ((w + t0 - 1) / t0) * ((h + t0 - 1) / t0);
     nbd_max = std::max(nbe, ntiles0);
     SR_HIP(hipMalloc(&gas, n));
     SR_HIP(hipMemset(gas, 1, n));
@@ -2017,7 +2025,7 @@ int FldSolver::launch_post_pair(int a, hipStream_t s, const int *gate) {
 int FldSolver::launch_pre_level(int l, const float *b, hipStream_t s, const int *gate) {
     const FldLevel &f = lv[l], &c = lv[l + 1];
     const Lv L = {f.w, f.h, f.own, f.ax, f.ay, f.cf};
-    switch (pre_tile[l]) {
+    switch (l == 0 ? tile0 : pre_tile[l]) {
     case TILE_16: launch_pre<16, 16>(nu1, s, L, b, f.z, c.b, c.w, gate); break;
     case TILE_64: launch_pre<PTX, PTY>(nu1, s, L, b, f.z, c.b, c.w, gate); break;
     default: launch_pre<32, 32>(nu1, s, L, b, f.z, c.b, c.w, gate); break;
@@ -2032,7 +2040,7 @@ int FldSolver::launch_post_level(int l, const float *b, float *zout, const float
     const FldLevel &f = lv[l], &c = lv[l + 1];
     const Lv L = {f.w, f.h, f.own, f.ax, f.ay, f.cf};
     int nb = 0;
-    switch (post_tile[l]) {
+    switch (l == 0 ? tile0 : post_tile[l]) {
     case TILE_16: nb = launch_post<16, 16>(nu2, s, L, b, f.z, c.zp, c.w, omega, zout, zold, part, gate); break;
     case TILE_64: nb = launch_post<PTX, PTY>(nu2, s, L, b, f.z, c.zp, c.w, omega, zout, zold, part, gate); break;
     default: nb = launch_post<32, 32>(nu2, s, L, b, f.z, c.zp, c.w, omega, zout, zold, part, gate); break;
@@ -2069,7 +2077,11 @@ int FldSolver::vcycle(const float *r, float *z, const float *zold, double *dots,
             if (l == 0 && upd) {
                 const int slot = tick(CLK_UPDATE_PRE0, s);
                 const FldLevel &f = lv[0];
-                launch_pre_upd<32, 32>(nu1, s, Lv{f.w, f.h, f.own, f.ax, f.ay, f.cf}, *upd, f.z, c.b, c.w);
+                const Lv L = {f.w, f.h, f.own, f.ax, f.ay, f.cf};
+                if (tile0 == TILE_16)
+                    launch_pre_upd<16, 16>(nu1, s, L, *upd, f.z, c.b, c.w);
+                else
+                    launch_pre_upd<32, 32>(nu1, s, L, *upd, f.z, c.b, c.w);
                 SR_TRY(tock(slot, s));
             } else {
                 const int slot = l == 0 ? tick(CLK_PRE0, s) : -1;

@@ -276,6 +276,32 @@ def test_ragged_grids_match_the_model(gpu_lib, w, h):
     assert np.linalg.norm(z.cpu().numpy() - zm) / np.linalg.norm(zm) <= 1e-5
 
 
+@pytest.mark.parametrize("w,h", [(1, 70), (17, 16), (608, 609), (640, 609)])
+def test_level_0_tiles_either_side_of_their_rule(gpu_lib, w, h):
+    """The smallest grids and one each side of the line (19 x 20 = 380 tiles of 32x32 take 16x16 tiles, 20 x 20 = 400
+    take 32x32): one V-cycle is the model's, and the solve with the update folded into level 0's first smoother is the
+    separate kernels' bit for bit (both count their dots' partials per tile)."""
+    import torch
+    print(f"level-0 tiles {w}x{h}", flush=True)
+    own, kx, ky, b = ragged_system(w, h, n=1024 if w > 256 else 256)
+    t = lambda a: torch.tensor(a.astype(np.float32), device="cuda").contiguous()
+    r = np.random.default_rng(3).standard_normal((h, w)).astype(np.float32)
+    zm = oracle.mg_apply(own, kx, ky, None, r.astype(np.float64), coarse_scale=1.2)
+    res = []
+    for on in (True, False):
+        f = gpu_lib.Fld(w, h, coarse_scale=1.2)
+        f.set_update_fusion(on)
+        f.set_system(t(own), t(kx), t(ky))
+        z = torch.empty((h, w), dtype=torch.float32, device="cuda")
+        f.apply_precond(t(r), z)
+        assert np.linalg.norm(z.cpu().numpy() - zm) / np.linalg.norm(zm) <= 1e-5  # the f32 cycle's bar above
+        x = torch.zeros((h, w), dtype=torch.float64, device="cuda")
+        it, rel = f.solve(torch.tensor(b, device="cuda"), x, tol=1e-8)
+        assert rel <= 1e-8
+        res.append((it, x.cpu().numpy()))
+    assert res[0][0] == res[1][0] and np.array_equal(res[0][1].view(np.uint64), res[1][1].view(np.uint64))
+
+
 def test_the_largest_axis_solves_to_1e8(gpu_lib):
     """4096^2 (the largest world axis): the stiff lognormal system solved to 1e-8, the residual recomputed in FP64 by
     the device's own matvec and again from the answer; a size-independent check, the oracle being too slow here."""
