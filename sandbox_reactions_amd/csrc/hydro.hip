@@ -6,15 +6,17 @@
 //   * one 320-thread block (five wave64s) per 16x16 tile: 256 threads own the tile's cells and 64 its one-cell
 //     ring (the face neighbours), so every predicted face state the tile's fluxes read is made once in the block;
 //   * primitives of the tile and a two-cell halo (ghosts by the edge rules) are staged in LDS as structure of
-//     arrays; the predicted faces go to LDS, each cell computes the HLL fluxes of its own four faces (a shared face
-//     is computed bit-identically by both cells, so the flux differences telescope);
+//     arrays; the slots' predicted low faces go to LDS and every HLL flux and gravity face work is made once, by the
+//     slot whose high face it is, and read back by the cell on the other side (so the flux differences telescope);
 //   * the ten species are not carried through the main pass: their mass-weighted mean 1/mu is linear in the
 //     fractions and rides along as a pseudo-species, and each species' face value and flux is made in a short loop
-//     after the main fluxes, the species' shared limiter factor kept in registers;
+//     after the main fluxes, the species' shared limiter factor kept in registers; a species that the staged cells
+//     hold none of is left out of both;
 //   * Sigma is stored and updated in FP64 (flux differences of FP32 fluxes summed in FP64), so the total mass is
 //     conserved to FP64 round-off; the other channels are FP32.
 // Two modes share the code: MID writes Sigma_mid = (Sigma^n + Sigma^{n+1}) / 2 from the mass fluxes
 // (hydro.rs:817-836) for the half-step gravity solve; UPDATE writes the next state.
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 
@@ -30,13 +32,18 @@ namespace sr {
 #define NSLOT (T * T + 4 * T) // 320
 #define NS 10
 #define HOT_FACE 2.0f
-#ifndef SR_HYDRO_SB
-#define SR_HYDRO_SB 1 // species per pass of the species phase (1, 2 or 5)
-#endif
 
 // (Z + 1) / A per species, assets/elements.json order: H He C O Ne Mg Si S Fe n (registry.rs:146-154)
 __constant__ float c_imu[NS] = {2.0f, 0.75f, 7.0f / 12.0f, 9.0f / 16.0f, 11.0f / 20.0f,
                                 13.0f / 24.0f, 15.0f / 28.0f, 17.0f / 32.0f, 27.0f / 56.0f, 1.0f};
+
+__device__ __forceinline__ unsigned long long wave_most(unsigned long long v) {
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long other = __shfl_xor(v, o, 64);
+        v = other > v ? other : v;
+    }
+    return v;
+}
 
 struct Prim {
     float s, u, v, p, im;
@@ -169,26 +176,35 @@ __device__ __forceinline__ void slot_pos(int t, int &x, int &y) {
     }
 }
 
-template <bool COLD> struct Lds {
-    float s[NPRIM], u[NPRIM], v[NPRIM], p[NPRIM], im[NPRIM];
+// The block's LDS. MULTI: the composition is staged (without it 1/mu is one number and no species is updated, so the
+// half step reads none). `f` holds, one after the other: the slots' predicted low faces (five fields, two axes) with
+// the half-step states; the high faces' fluxes, kicks and works; the species' low faces and fluxes; the partial sums.
+template <int MODE, bool COLD, bool MULTI> struct Lds {
+    static constexpr int NF = MODE == HYDRO_MID ? 10 : 13;
+    float s[NPRIM], u[NPRIM], v[NPRIM], p[NPRIM], im[MULTI ? NPRIM : 1];
     float ye[COLD ? NPRIM : 1];  // Y_e, with the cold pressure on
-    float x[NS][NPRIM];
-    // predicted face states of every slot: [field][face][slot], fields s u v p e; reused for species faces
-    float face[5][4][NSLOT];
-    float mid[3][NSLOT];
-    double red[8][5];
-    unsigned long long redk[8];
+    float x[MULTI ? NS : 1][MULTI ? NPRIM : 1];
+    alignas(8) float f[NF][NSLOT];
+    unsigned present[NSLOT / 64];
 };
 
-template <int MODE, bool COLD, bool SINKS = false>
-__global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, HydroState out,
+// What bounds it: vector instructions (2048^2, one species: the half step 98 us and its ALUs always busy, the update
+// 383 us and half busy, where the planes' traffic alone takes about 45 and 105 us). So every face's flux, work and
+// species fluxes are made once, by the slot on its low side, which holds its own side's state in registers and reads
+// only the other side's from LDS; and a species of which neither the tile nor its halo holds any is left out of the
+// limiter and of the species' loop (its fluxes are zeros). Before, with each face made on both sides and all species in
+// the loop, the two took 313 and 732 us; with all ten species and the cold pressure at 512^2 29 + 74 us now, 49 + 104
+// before. 41 KB of LDS and 96 registers: four blocks to a CU (loading the update's inputs ahead of the fluxes spilled
+// and cost 20 %).
+template <int MODE, bool COLD, bool SINKS = false, bool MULTI = true>
+__global__ void __launch_bounds__(NSLOT, 5) k_hydro(HydroParams P, HydroState in, HydroState out,
                                                  const double *__restrict__ scal, const float *__restrict__ gx,
                                                  const float *__restrict__ gy, const float *__restrict__ sigma_mid,
                                                  const float *__restrict__ phi_mid, const float *__restrict__ rfx,
                                                  const float *__restrict__ rfy, float *__restrict__ sigma_mid_out,
                                                  float *__restrict__ pushmag, double *__restrict__ escaped,
                                                  HydroPartials part, SinkPlanes SP) {
-    __shared__ Lds<COLD> L;
+    __shared__ Lds<MODE, COLD, MULTI> L;
     const int w = P.w, h = P.h;
     const int tile = xcd_tile();
     const int bx = (tile % gridDim.x) * T, by = (tile / gridDim.x) * T;
@@ -200,6 +216,7 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
     const size_t n = (size_t)w * h;
 
     // ---- phase 0: primitives of the tile and a two-cell halo, ghosts by the edge rules (hydro.rs:673-710)
+    unsigned present = 0u;  // the species that the lanes' cells hold
     for (int t = tid; t < NPRIM; t += NSLOT) {
         const int lx = t % PW, ly = t / PW;
         int gxi = bx + lx - HALO, gyi = by + ly - HALO;
@@ -217,11 +234,13 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
         const size_t i = (size_t)gyi * w + gxi;
         float xs[NS];
         float im = 0.0f, ye = 0.0f;
-        for (int s = 0; s < NS; s++) {
-            xs[s] = in.x[s * n + i];
-            im += xs[s] * c_imu[s];
-            if (COLD) ye += xs[s] * c_ye[s];
-        }
+        if constexpr (MULTI)
+            for (int s = 0; s < NS; s++) {
+                xs[s] = in.x[s * n + i];
+                im += xs[s] * c_imu[s];
+                if (COLD) ye += xs[s] * c_ye[s];
+                if (xs[s] != 0.0f) present |= 1u << s;
+            }
         if (P.fixed_imu > 0.0f) im = P.fixed_imu;
         const double sig = in.sigma[i];
         Prim q;
@@ -253,11 +272,24 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
         L.u[t] = q.u;
         L.v[t] = q.v;
         L.p[t] = q.p;
-        L.im[t] = im;
         if (COLD) L.ye[t] = ye;
-        for (int s = 0; s < NS; s++) L.x[s][t] = xs[s];
+        if constexpr (MULTI) {
+            L.im[t] = im;
+            for (int s = 0; s < NS; s++) L.x[s][t] = xs[s];
+        }
+    }
+    if constexpr (MULTI) {
+        for (int o = 32; o > 0; o >>= 1) present |= __shfl_xor(present, o, 64);
+        if ((tid & 63) == 0) L.present[tid >> 6] = present;
     }
     __syncthreads();
+    if constexpr (MULTI) {
+        present = 0u;
+        for (int k = 0; k < NSLOT / 64; k++) present |= L.present[k];
+        present = __builtin_amdgcn_readfirstlane(present);
+    }
+    auto imu_at = [&](int i) { return MULTI ? L.im[i] : P.fixed_imu; };
+    auto xn_at = [&](int i) { return COLD ? L.x[NS - 1][i] : 0.0f; };
 
     // ---- phase 1: every slot's slopes and Hancock predictor (hydro.rs:587-614)
     int sx_, sy_;
@@ -271,23 +303,27 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
     }
     float theta[2];            // the species' shared limiter factor per axis
     float fs_w[4], f0_w[4];    // reconstructed faces' Sigma and mass flux
-    float s_e[4];              // evolved faces' Sigma (0 when the unevolved face is kept)
-    float is_e[4];             // its reciprocal (0 when the unevolved face is kept)
+    float is_e[4];             // the evolved faces' 1 / Sigma (0 when the unevolved face is kept)
+    Prim hf[2];                // the high faces' predicted states
+    float hf_e[2];
+    float m0, m1, m2;          // the half-step state
     {
-        const Prim c = {L.s[lc], L.u[lc], L.v[lc], L.p[lc], L.im[lc], COLD ? L.ye[lc] : 0.0f, L.x[NS - 1][lc]};
+        const Prim c = {L.s[lc], L.u[lc], L.v[lc], L.p[lc], imu_at(lc), COLD ? L.ye[lc] : 0.0f, xn_at(lc)};
         Prim wf[4];
         for (int ax = 0; ax < 2; ax++) {
             const int off = ax ? PW : 1;
             const int il = lc - off, ir = lc + off;
-            const Prim l = {L.s[il], L.u[il], L.v[il], L.p[il], L.im[il], COLD ? L.ye[il] : 0.0f, L.x[NS - 1][il]};
-            const Prim r = {L.s[ir], L.u[ir], L.v[ir], L.p[ir], L.im[ir], COLD ? L.ye[ir] : 0.0f, L.x[NS - 1][ir]};
+            const Prim l = {L.s[il], L.u[il], L.v[il], L.p[il], imu_at(il), COLD ? L.ye[il] : 0.0f, xn_at(il)};
+            const Prim r = {L.s[ir], L.u[ir], L.v[ir], L.p[ir], imu_at(ir), COLD ? L.ye[ir] : 0.0f, xn_at(ir)};
             float ss = mc(l.s, c.s, r.s), su = mc(l.u, c.u, r.u), sv = mc(l.v, c.v, r.v), sp = mc(l.p, c.p, r.p);
             float th = 1.0f;
-            for (int s = 0; s < NS; s++) {
-                const float xl = L.x[s][il], xc = L.x[s][lc], xr = L.x[s][ir];
-                const float central = 0.5f * (xr - xl);
-                if (central != 0.0f) th = fminf(th, __fdividef(mc(xl, xc, xr), central));
-            }
+            if constexpr (MULTI)
+                for (unsigned todo = present; todo; todo &= todo - 1u) {
+                    const int s = __builtin_ctz(todo);
+                    const float xl = L.x[s][il], xc = L.x[s][lc], xr = L.x[s][ir];
+                    const float central = 0.5f * (xr - xl);
+                    if (central != 0.0f) th = fminf(th, __fdividef(mc(xl, xc, xr), central));
+                }
             theta[ax] = th;
             // 1/mu, Y_e and X_n are linear in the fractions: their faces take the species' shared slope
             const float sim = th * 0.5f * (r.im - l.im);
@@ -331,14 +367,16 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
         delta[6] = COLD ? hdx * ((fl[0][0] * wf[0].xn - fl[1][0] * wf[1].xn) +
                                  (fl[2][0] * wf[2].xn - fl[3][0] * wf[3].xn))
                         : 0.0f;
-        float m0 = c.s + delta[0], m1 = c.s * c.u + delta[1], m2 = c.s * c.v + delta[2];
+        m0 = c.s + delta[0], m1 = c.s * c.u + delta[1], m2 = c.s * c.v + delta[2];
         if (grav) {
             m1 += half * c.s * gcx;
             m2 += half * c.s * gcy;
         }
-        L.mid[0][tid] = m0;
-        L.mid[1][tid] = m1;
-        L.mid[2][tid] = m2;
+        if constexpr (MODE == HYDRO_UPDATE) {
+            L.f[10][tid] = m0;
+            L.f[11][tid] = m1;
+            L.f[12][tid] = m2;
+        }
         for (int k = 0; k < 4; k++) {
             const Prim &q = wf[k];
             float d1 = delta[1], d2 = delta[2], d3 = delta[3];
@@ -353,59 +391,107 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
             float oe;
             if (prim_of<COLD>(P, s0, mx, my, e, sim, sye, sxn, o)) {
                 oe = e;
-                s_e[k] = s0;
                 is_e[k] = 1.0f / s0;
             } else {
                 o = q;
                 oe = ue[k];
-                s_e[k] = 0.0f;
                 is_e[k] = 0.0f;
             }
-            L.face[0][k][tid] = o.s;
-            L.face[1][k][tid] = o.u;
-            L.face[2][k][tid] = o.v;
-            L.face[3][k][tid] = o.p;
-            L.face[4][k][tid] = oe;
+            const int ax = k >> 1;
+            if (k & 1) {
+                hf[ax] = o;
+                hf_e[ax] = oe;
+            } else {
+                L.f[5 * ax][tid] = o.s;
+                L.f[5 * ax + 1][tid] = o.u;
+                L.f[5 * ax + 2][tid] = o.v;
+                L.f[5 * ax + 3][tid] = o.p;
+                if constexpr (MODE == HYDRO_UPDATE) L.f[5 * ax + 4][tid] = oe;
+            }
         }
     }
     __syncthreads();
 
-    // ---- phase 2: the tile cells' four face fluxes (hydro.rs:744-778, boundary :569-582)
+    // ---- phase 2: the fluxes through the slots' high faces (hydro.rs:744-778, boundary :569-582): a cell's two, the
+    // left ring's x faces and the upper ring's y faces; the others' are not read
     const bool own = tid < T * T;
     const int gxc = bx + sx_, gyc = by + sy_;
     const bool live = own && gxc < w && gyc < h;
+    const int up_x = own ? (sx_ + 1 < T ? tid + 1 : T * T + T + sy_) : min(max(sy_, 0), T - 1) * T;  // (x + 1, y)
+    const int up_y = own ? (sy_ + 1 < T ? tid + T : T * T + 3 * T + sx_) : min(max(sx_, 0), T - 1);  // (x, y + 1)
     float F[4][4];  // fluxes of faces x-, x+, y-, y+ along +x / +y
-    bool upl[4];    // whether the low side is upwind
-    bool wallf[4];  // a wall face (bounce, or leave with inflow): no species flux
-    if (live) {
-        for (int k = 0; k < 4; k++) {
-            const int dir = k >> 1;
-            const bool high = k & 1;
-            const int nx = sx_ + (dir == 0 ? (high ? 1 : -1) : 0), ny = sy_ + (dir == 1 ? (high ? 1 : -1) : 0);
-            const int ns = slot_of(nx, ny);
-            // the low side's face toward +, the high side's face toward -
-            const int ls = high ? tid : ns, lk = high ? k : k + 1;
-            const int hs = high ? ns : tid, hk = high ? k - 1 : k;
-            const Prim lp = {L.face[0][lk][ls], L.face[1][lk][ls], L.face[2][lk][ls], L.face[3][lk][ls], 0.0f};
-            const Prim hp = {L.face[0][hk][hs], L.face[1][hk][hs], L.face[2][hk][hs], L.face[3][hk][hs], 0.0f};
-            const float le = L.face[4][lk][ls], he = L.face[4][hk][hs];
-            const bool edge = dir == 0 ? (high ? gxc == w - 1 : gxc == 0) : (high ? gyc == h - 1 : gyc == 0);
-            wallf[k] = false;
-            if (edge && P.edge == 0) {
-                for (int c4 = 0; c4 < 4; c4++) F[k][c4] = 0.0f;
-                F[k][1 + dir] = high ? lp.p : hp.p; // the own face's pressure
-                wallf[k] = true;
-                upl[k] = true;
-            } else {
-                upl[k] = hll(P, lp, le, hp, he, dir, F[k]);
-                if (edge) {
-                    const bool inflow = high ? F[k][0] < 0.0f : F[k][0] > 0.0f;
-                    if (inflow) {
-                        for (int c4 = 0; c4 < 4; c4++) F[k][c4] = 0.0f;
-                        F[k][1 + dir] = high ? lp.p : hp.p;
-                        wallf[k] = true;
-                    }
-                }
+    bool upl[2];    // whether the high faces' low side is upwind
+    bool wallf[2];  // a wall face (bounce, or leave with inflow): no species flux
+    float kick_f[4], work_l[2], work_h[4];  // gravity's source at the faces: kick, and the low and high sides' work
+    const int rw = w + 2;
+    const float *pr = nullptr, *ps = nullptr;
+    float phi_c = 0.0f;
+    if constexpr (MODE == HYDRO_UPDATE)
+        if (grav) {
+            const size_t at = (size_t)(min(gyc, h - 1) + 1) * rw + min(gxc, w - 1) + 1;
+            pr = phi_mid + at;
+            phi_c = pr[0];
+            // phi_mid as the faces' work reads it: the gas's with the sinks' potential
+            if constexpr (SINKS) {
+                ps = SP.ps + at;
+                phi_c += ps[0];
+            }
+        }
+    for (int ax = 0; ax < 2; ax++) {
+        const int k = 2 * ax + 1, hs = ax ? up_y : up_x;
+        const Prim lp = hf[ax];
+        const Prim hp = {L.f[5 * ax][hs], L.f[5 * ax + 1][hs], L.f[5 * ax + 2][hs], L.f[5 * ax + 3][hs], 0.0f};
+        const float he = MODE == HYDRO_UPDATE ? L.f[5 * ax + 4][hs] : 0.0f;
+        const int at = ax ? gyc : gxc, last = (ax ? h : w) - 1;
+        const bool low = at < 0, edge = low || at == last;
+        wallf[ax] = edge && P.edge == 0;
+        upl[ax] = true;
+        if (!wallf[ax]) {
+            upl[ax] = hll(P, lp, hf_e[ax], hp, he, ax, F[k]);
+            wallf[ax] = edge && (low ? F[k][0] > 0.0f : F[k][0] < 0.0f);
+        }
+        if (wallf[ax]) {
+            for (int c4 = 0; c4 < 4; c4++) F[k][c4] = 0.0f;
+            F[k][1 + ax] = low ? hp.p : lp.p; // the own face's pressure
+        }
+        if constexpr (MODE == HYDRO_UPDATE)
+            if (grav) {
+                // the world's edge does no work (the cell's own values on both sides)
+                const float mh = L.f[10][hs], ph = L.f[11 + ax][hs], ml = m0, pl = ax ? m2 : m1;
+                float pn = pr[ax ? rw : 1];
+                if constexpr (SINKS) pn += ps[ax ? rw : 1];
+                const float d = edge ? 0.0f : (phi_c - pn) * P.inv_dx;
+                float o[3];
+                face_work(F[k][0], low ? mh : ml, edge && !low ? ml : mh, low ? ph : pl, edge && !low ? pl : ph, d, dtf,
+                          o);
+                kick_f[k] = o[0];
+                work_l[ax] = o[1];
+                work_h[k] = o[2];
+            }
+    }
+    __syncthreads();
+    for (int ax = 0; ax < 2; ax++) {
+        const int k = 2 * ax + 1;
+        L.f[6 * ax][tid] = F[k][0];
+        if constexpr (MODE == HYDRO_UPDATE) {
+            for (int c4 = 1; c4 < 4; c4++) L.f[6 * ax + c4][tid] = F[k][c4];
+            if (grav) {
+                L.f[6 * ax + 4][tid] = kick_f[k];
+                L.f[6 * ax + 5][tid] = work_h[k];
+            }
+        }
+    }
+    __syncthreads();
+    const int dn_x = own ? (sx_ > 0 ? tid - 1 : T * T + sy_) : 0;          // (x - 1, y)
+    const int dn_y = own ? (sy_ > 0 ? tid - T : T * T + 2 * T + sx_) : 0;  // (x, y - 1)
+    for (int ax = 0; ax < 2; ax++) {
+        const int k = 2 * ax, ls = ax ? dn_y : dn_x;
+        F[k][0] = L.f[6 * ax][ls];
+        if constexpr (MODE == HYDRO_UPDATE) {
+            for (int c4 = 1; c4 < 4; c4++) F[k][c4] = L.f[6 * ax + c4][ls];
+            if (grav) {
+                kick_f[k] = L.f[6 * ax + 4][ls];
+                work_h[k] = L.f[6 * ax + 5][ls];
             }
         }
     }
@@ -427,7 +513,7 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
             sigma_mid_out[ci] = s >= (double)P.sigma_vac ? (float)s : 0.0f;
         }
         return;
-    }
+    } else {
 
     // ---- phase 3: the update (hydro.rs:864-984)
     double kick_net[2] = {0.0, 0.0}, push_net[3] = {0.0, 0.0, 0.0};
@@ -436,7 +522,7 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
     float u1 = 0.f, u2 = 0.f, u3 = 0.f;
     if (live && !empty) {
         if (vacuum) {
-            const Prim fq = {L.s[lc], L.u[lc], L.v[lc], L.p[lc], L.im[lc], COLD ? L.ye[lc] : 0.0f, L.x[NS - 1][lc]};
+            const Prim fq = {L.s[lc], L.u[lc], L.v[lc], L.p[lc], L.im[lc], COLD ? L.ye[lc] : 0.0f, xn_at(lc)};
             u1 = 0.0f;
             u2 = 0.0f;
             u3 = cons_e<COLD>(P, fq);
@@ -450,66 +536,23 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
         u1 -= dtdxf * ((F[1][1] - F[0][1]) + (F[3][1] - F[2][1]));
         u2 -= dtdxf * ((F[1][2] - F[0][2]) + (F[3][2] - F[2][2]));
         u3 -= dtdxf * ((F[1][3] - F[0][3]) + (F[3][3] - F[2][3]));
-        float phi_c = 0.0f;
         if (grav) {
-            const int rw = w + 2;
-            const float *pr = phi_mid + (size_t)(gyc + 1) * rw + gxc + 1;
             const float src = sigma_mid[ci];
             const float gmx = -(pr[1] - pr[-1]) * 0.5f * P.inv_dx, gmy = -(pr[rw] - pr[-rw]) * 0.5f * P.inv_dx;
             float kick[2] = {dtf * src * gmx, dtf * src * gmy};
             // the net kick taken back is the gas's own field's; the sinks' pull is the sinks' to book
             kick_net[0] = (double)kick[0];
             kick_net[1] = (double)kick[1];
-            // phi_mid as the faces' work reads it: the gas's with the sinks' potential
-            float pw[5] = {pr[0], pr[1], pr[-1], pr[rw], pr[-rw]};
             if constexpr (SINKS) {
-                const float *ps = SP.ps + (size_t)(gyc + 1) * rw + gxc + 1;
-                pw[0] += ps[0];
-                pw[1] += ps[1];
-                pw[2] += ps[-1];
-                pw[3] += ps[rw];
-                pw[4] += ps[-rw];
                 kick[0] += dtf * src * SP.gsx[ci];
                 kick[1] += dtf * src * SP.gsy[ci];
             }
-            phi_c = pw[0];
             if (src > 0.0f) dkey = ((unsigned long long)__float_as_uint(src) << 32) | (0xffffffffu - (unsigned)ci);
-            const float m0 = L.mid[0][tid], m1 = L.mid[1][tid], m2 = L.mid[2][tid];
-            float r[3], l[3], dn[3], up[3];
-            // neighbours' phi_mid and half-step state; the world's edge does no work (the cell's own values)
-            {
-                const bool has = gxc + 1 < w;
-                const int ns = slot_of(sx_ + 1, sy_);
-                const float pn = has ? pw[1] : phi_c;
-                face_work(F[1][0], m0, has ? L.mid[0][ns] : m0, m1, has ? L.mid[1][ns] : m1, (phi_c - pn) * P.inv_dx,
-                          dtf, r);
-            }
-            {
-                const bool has = gxc > 0;
-                const int ns = slot_of(sx_ - 1, sy_);
-                const float pn = has ? pw[2] : phi_c;
-                face_work(F[0][0], has ? L.mid[0][ns] : m0, m0, has ? L.mid[1][ns] : m1, m1, (pn - phi_c) * P.inv_dx,
-                          dtf, l);
-            }
-            {
-                const bool has = gyc + 1 < h;
-                const int ns = slot_of(sx_, sy_ + 1);
-                const float pn = has ? pw[3] : phi_c;
-                face_work(F[3][0], m0, has ? L.mid[0][ns] : m0, m2, has ? L.mid[2][ns] : m2, (phi_c - pn) * P.inv_dx,
-                          dtf, dn);
-            }
-            {
-                const bool has = gyc > 0;
-                const int ns = slot_of(sx_, sy_ - 1);
-                const float pn = has ? pw[4] : phi_c;
-                face_work(F[2][0], has ? L.mid[0][ns] : m0, m0, has ? L.mid[2][ns] : m2, m2, (pn - phi_c) * P.inv_dx,
-                          dtf, up);
-            }
-            kick[0] += r[0] - l[0];
-            kick[1] += dn[0] - up[0];
+            kick[0] += kick_f[1] - kick_f[0];
+            kick[1] += kick_f[3] - kick_f[2];
             u1 += kick[0];
             u2 += kick[1];
-            u3 += r[1] + l[2] + dn[1] + up[2];
+            u3 += work_l[0] + work_h[0] + work_l[1] + work_h[2];
         }
         if (rfx) {
             // the radiation force from the previous step's flux, capped by the heat above the floor
@@ -586,62 +629,57 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
     }
 
     const double inv_u0 = u0 != 0.0 ? 1.0 / u0 : 0.0;
-    // ---- phase 4: the species, SB at a time in the freed face buffer (flux = mass flux x the upwind face's
-    // fraction)
-    constexpr int SB = SR_HYDRO_SB;
-    static_assert(NS % SB == 0 && SB <= 5, "species batches fill the face buffer's five fields");
-    for (int s0 = 0; s0 < NS; s0 += SB) {
-        __syncthreads(); // the face buffer is reused
-#pragma unroll
-        for (int j = 0; j < SB; j++) {
-            const int s = s0 + j;
-            const int offs[2] = {1, PW};
-            float xf[4];
-            const float xc = L.x[s][lc];
-            for (int ax = 0; ax < 2; ax++) {
-                const float central = 0.5f * (L.x[s][lc + offs[ax]] - L.x[s][lc - offs[ax]]);
-                xf[2 * ax] = xc - 0.5f * theta[ax] * central;
-                xf[2 * ax + 1] = xc + 0.5f * theta[ax] * central;
-            }
-            const float ds = hdx * ((f0_w[0] * xf[0] - f0_w[1] * xf[1]) + (f0_w[2] * xf[2] - f0_w[3] * xf[3]));
-            for (int k = 0; k < 4; k++) L.face[j][k][tid] = s_e[k] > 0.0f ? (fs_w[k] * xf[k] + ds) * is_e[k] : xf[k];
+    // ---- phase 4: the species that are here, one at a time (flux = mass flux x the upwind face's fraction): fields 0
+    // and 1 of L.f hold its low faces, 2 and 3 its high faces' fluxes
+    const int nf = 2 * (w + h);
+    const int slots[4] = {gyc, h + gyc, 2 * h + gxc, 2 * h + w + gxc};
+    const bool edges[4] = {gxc == 0, gxc + 1 == w, gyc == 0, gyc + 1 == h};
+    __syncthreads(); // the fluxes' fields are reused
+    for (unsigned todo = present; todo; todo &= todo - 1u) {
+        const int s = __builtin_ctz(todo);
+        const float *xp = L.x[s];
+        const float xc = xp[lc];  // the cell's own fraction, staged in phase 0
+        const int offs[2] = {1, PW};
+        float xf[4], f[2];
+        for (int ax = 0; ax < 2; ax++) {
+            const float central = 0.5f * (xp[lc + offs[ax]] - xp[lc - offs[ax]]);
+            xf[2 * ax] = xc - 0.5f * theta[ax] * central;
+            xf[2 * ax + 1] = xc + 0.5f * theta[ax] * central;
+        }
+        const float ds = hdx * ((f0_w[0] * xf[0] - f0_w[1] * xf[1]) + (f0_w[2] * xf[2] - f0_w[3] * xf[3]));
+        for (int k = 0; k < 4; k++) {
+            const float v = is_e[k] != 0.0f ? (fs_w[k] * xf[k] + ds) * is_e[k] : xf[k];
+            if (k & 1)
+                f[k >> 1] = v;
+            else
+                L.f[k >> 1][tid] = v;
+        }
+        __syncthreads();
+        for (int ax = 0; ax < 2; ax++) {
+            const float hx = L.f[ax][ax ? up_y : up_x];
+            f[ax] = wallf[ax] ? 0.0f : F[2 * ax + 1][0] * (upl[ax] ? f[ax] : hx);
+            L.f[2 + ax][tid] = f[ax];
         }
         __syncthreads();
         if (live) {
-#pragma unroll
-            for (int j = 0; j < SB; j++) {
-                const int s = s0 + j;
-                const size_t pi = (size_t)s * n + ci;
-                const float xs0 = L.x[s][lc];  // the cell's own fraction, staged in phase 0
-                if (empty) {
-                    out.x[pi] = xs0;
-                    continue;
-                }
-                float fsx[4];
-                for (int k = 0; k < 4; k++) {
-                    if (wallf[k]) {
-                        fsx[k] = 0.0f;
-                        continue;
-                    }
-                    const int dir = k >> 1;
-                    const bool high = k & 1;
-                    const int nx = sx_ + (dir == 0 ? (high ? 1 : -1) : 0),
-                              ny = sy_ + (dir == 1 ? (high ? 1 : -1) : 0);
-                    const int ns = slot_of(nx, ny);
-                    const int ls = high ? tid : ns, lk = high ? k : k + 1;
-                    const int hs = high ? ns : tid, hk = high ? k - 1 : k;
-                    fsx[k] = F[k][0] * (upl[k] ? L.face[j][lk][ls] : L.face[j][hk][hs]);
-                }
-                const double um =
-                    start * (double)xs0 - dtdx * (((double)fsx[1] - fsx[0]) + ((double)fsx[3] - fsx[2]));
-                out.x[pi] = (float)(um * inv_u0);
-                const int nf = 2 * (w + h);
-                const int slots[4] = {gyc, h + gyc, 2 * h + gxc, 2 * h + w + gxc};
-                const bool edges[4] = {gxc == 0, gxc + 1 == w, gyc == 0, gyc + 1 == h};
+            const float fsx[4] = {L.f[2][dn_x], f[0], L.f[3][dn_y], f[1]};
+            const double um = start * (double)xc - dtdx * (((double)fsx[1] - fsx[0]) + ((double)fsx[3] - fsx[2]));
+            out.x[(size_t)s * n + ci] = empty ? xc : (float)(um * inv_u0);
+            if (!empty)
                 for (int k = 0; k < 4; k++)
                     if (edges[k])
                         escaped[(size_t)(4 + s) * nf + slots[k]] += ((k & 1) ? 1.0 : -1.0) * dtdx * fsx[k];
-            }
+        }
+    }
+    // the species that are not: no fluxes, unless the gas's are not numbers (those spread to every species)
+    if (live) {
+        const float none = empty ? 0.0f : (float)(0.0 * (start - dtdx * divm) * inv_u0);
+        for (unsigned todo = ~present & ((1u << NS) - 1u); todo; todo &= todo - 1u) {
+            const int s = __builtin_ctz(todo);
+            out.x[(size_t)s * n + ci] = none;
+            if (!empty)
+                for (int k = 0; k < 4; k++)
+                    if (edges[k] && !isfinite(F[k][0])) escaped[(size_t)(4 + s) * nf + slots[k]] += 0.0 * F[k][0];
         }
     }
 
@@ -649,48 +687,47 @@ __global__ void __launch_bounds__(NSLOT) k_hydro(HydroParams P, HydroState in, H
     if (grav || rfx) {
         const int lane = tid & 63, wid = tid >> 6;
         double v[5] = {kick_net[0], kick_net[1], push_net[0], push_net[1], push_net[2]};
-        for (int k = 0; k < 5; k++) v[k] = wave_sum(v[k]);
-        unsigned long long kk = dkey;
-        for (int o = 32; o > 0; o >>= 1) {
-            const unsigned long long other = __shfl_xor(kk, o, 64);
-            kk = other > kk ? other : kk;
-        }
+        for (int k = 0; k < 5; k++)
+            if (k < 2 ? grav : rfx != nullptr) v[k] = wave_sum(v[k]);
+        const unsigned long long kk = wave_most(dkey);
+        double(*red)[5] = (double(*)[5])L.f[0];
+        unsigned long long *redk = (unsigned long long *)L.f[1];
         __syncthreads();
         if (lane == 0) {
-            for (int k = 0; k < 5; k++) L.red[wid][k] = v[k];
-            L.redk[wid] = kk;
+            for (int k = 0; k < 5; k++) red[wid][k] = v[k];
+            redk[wid] = kk;
         }
         __syncthreads();
         if (tid == 0) {
             double acc[5] = {0, 0, 0, 0, 0};
             unsigned long long best = 0ull;
             for (int wv = 0; wv < NSLOT / 64; wv++) {
-                for (int k = 0; k < 5; k++) acc[k] += L.red[wv][k];
-                best = L.redk[wv] > best ? L.redk[wv] : best;
+                for (int k = 0; k < 5; k++) acc[k] += red[wv][k];
+                best = redk[wv] > best ? redk[wv] : best;
             }
             const int b = tile;  // partials in tile order
             for (int k = 0; k < 5; k++) part.sums[(size_t)b * 5 + k] = acc[k];
             part.keys[b] = best;
         }
     }
+    }
 }
 
 // The take-backs (hydro.rs:986-1001): the radiation force's net push from every pushed cell in proportion to its
-// push, gravity's net kick from the densest free cell. One block reduces the partials in a fixed order first.
-__global__ void __launch_bounds__(256) k_hydro_reduce(HydroPartials part, int nblocks, double *__restrict__ takeback) {
+// push, gravity's net kick from the densest free cell. Up to TAKE_ROWS blocks reduce the tiles' partials, each to one
+// row (five sums and the key), in a fixed order (2048^2's 16384 tiles: 4.6 us, by one block alone 31); every
+// block of the take-back adds the rows up itself. Without radiation one cell is changed and one block is launched.
+__global__ void __launch_bounds__(256) k_hydro_reduce(HydroPartials part, int nblocks, double *__restrict__ rows) {
     __shared__ double sh[4][5];
     __shared__ unsigned long long shk[4];
     double acc[5] = {0, 0, 0, 0, 0};
     unsigned long long best = 0ull;
-    for (int b = threadIdx.x; b < nblocks; b += blockDim.x) {
+    for (int b = blockIdx.x * 256 + threadIdx.x; b < nblocks; b += gridDim.x * 256) {
         for (int k = 0; k < 5; k++) acc[k] += part.sums[(size_t)b * 5 + k];
         best = part.keys[b] > best ? part.keys[b] : best;
     }
     for (int k = 0; k < 5; k++) acc[k] = wave_sum(acc[k]);
-    for (int o = 32; o > 0; o >>= 1) {
-        const unsigned long long other = __shfl_xor(best, o, 64);
-        best = other > best ? other : best;
-    }
+    best = wave_most(best);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (lane == 0) {
         for (int k = 0; k < 5; k++) sh[wid][k] = acc[k];
@@ -698,40 +735,49 @@ __global__ void __launch_bounds__(256) k_hydro_reduce(HydroPartials part, int nb
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double t[5] = {0, 0, 0, 0, 0};
-        unsigned long long bk = 0ull;
-        for (int wv = 0; wv < 4; wv++) {
-            for (int k = 0; k < 5; k++) t[k] += sh[wv][k];
-            bk = shk[wv] > bk ? shk[wv] : bk;
-        }
-        for (int k = 0; k < 5; k++) takeback[k] = t[k];
-        takeback[5] = bk ? (double)(0xffffffffu - (unsigned)(bk & 0xffffffffu)) : -1.0;
+        double *row = rows + (size_t)blockIdx.x * 6;
+        for (int k = 0; k < 5; k++) row[k] = sh[0][k] + sh[1][k] + sh[2][k] + sh[3][k];
+        for (int wv = 1; wv < 4; wv++) best = shk[wv] > best ? shk[wv] : best;
+        row[5] = __longlong_as_double((long long)best);
     }
 }
 
-__global__ void k_hydro_takeback(HydroState st, const float *__restrict__ pushmag, const double *__restrict__ tb,
-                                 int n, int radiation) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float mx = st.mx[i], my = st.my[i];
-    bool changed = false;
-    if (radiation && tb[4] > 0.0) {
-        const float m = pushmag[i];
-        if (m != 0.0f) {
-            mx -= (float)((double)m * tb[2] / tb[4]);
-            my -= (float)((double)m * tb[3] / tb[4]);
-            changed = true;
+__global__ void __launch_bounds__(256) k_hydro_takeback(HydroState st, const float *__restrict__ pushmag,
+                                                        const double *__restrict__ rows, int nrows, int n,
+                                                        int radiation) {
+    __shared__ double tb[5];
+    __shared__ unsigned long long key;
+    if (threadIdx.x < 64) {
+        const double *row = rows + (size_t)threadIdx.x * 6;
+        const bool has = (int)threadIdx.x < nrows;
+        for (int k = 0; k < 5; k++) {
+            const double v = wave_sum(has ? row[k] : 0.0);
+            if (threadIdx.x == 0) tb[k] = v;
         }
+        const unsigned long long best = wave_most(has ? (unsigned long long)__double_as_longlong(row[5]) : 0ull);
+        if (threadIdx.x == 0) key = best;
     }
-    if (tb[5] >= 0.0 && (int)tb[5] == i) {
+    __syncthreads();
+    const int densest = key ? (int)(0xffffffffu - (unsigned)(key & 0xffffffffu)) : -1;
+    int i = blockIdx.x * 256 + threadIdx.x;
+    if (!radiation) {
+        i = threadIdx.x == 0 ? densest : -1;
+        if (i < 0) return;
+    }
+    if (i >= n) return;
+    const float m = radiation && tb[4] > 0.0 ? pushmag[i] : 0.0f;
+    if (m == 0.0f && i != densest) return;
+    float mx = st.mx[i], my = st.my[i];
+    if (m != 0.0f) {
+        mx -= (float)((double)m * tb[2] / tb[4]);
+        my -= (float)((double)m * tb[3] / tb[4]);
+    }
+    if (i == densest) {
         mx -= (float)tb[0];
         my -= (float)tb[1];
-        changed = true;
     }
-    if (changed) {
-        st.mx[i] = mx;
-        st.my[i] = my;
-    }
+    st.mx[i] = mx;
+    st.my[i] = my;
 }
 
 // ------------------------------------------------------------------------------------------------------------ host
@@ -750,7 +796,10 @@ int hydro_launch(int mode, const HydroParams &P, const HydroState &in, const Hyd
                            sigma_mid_out, pushmag, escaped, part, sp);
     };
     if (mode == HYDRO_MID)
-        P.cold.on ? go(k_hydro<HYDRO_MID, true>) : go(k_hydro<HYDRO_MID, false>);
+        // one 1/mu and no cold pressure: the half step needs no composition
+        P.cold.on            ? go(k_hydro<HYDRO_MID, true>)
+        : P.fixed_imu > 0.0f ? go(k_hydro<HYDRO_MID, false, false, false>)
+                             : go(k_hydro<HYDRO_MID, false>);
     else if (with_sinks)
         P.cold.on ? go(k_hydro<HYDRO_UPDATE, true, true>) : go(k_hydro<HYDRO_UPDATE, false, true>);
     else
@@ -760,12 +809,12 @@ int hydro_launch(int mode, const HydroParams &P, const HydroState &in, const Hyd
 }
 
 int hydro_takeback(const HydroParams &P, const HydroState &st, const float *pushmag, const HydroPartials &part,
-                   double *takeback, bool radiation, hipStream_t s) {
-    const int nb = ((P.w + T - 1) / T) * ((P.h + T - 1) / T);
-    hipLaunchKernelGGL(k_hydro_reduce, dim3(1), dim3(256), 0, s, part, nb, takeback);
+                   double *rows, bool radiation, hipStream_t s) {
+    const int nb = hydro_blocks(P.w, P.h), nrows = std::min(TAKE_ROWS, (nb + 255) / 256);
+    hipLaunchKernelGGL(k_hydro_reduce, dim3(nrows), dim3(256), 0, s, part, nb, rows);
     const int n = P.w * P.h;
-    hipLaunchKernelGGL(k_hydro_takeback, dim3((n + 255) / 256), dim3(256), 0, s, st, pushmag, takeback, n,
-                       radiation ? 1 : 0);
+    hipLaunchKernelGGL(k_hydro_takeback, dim3(radiation ? (n + 255) / 256 : 1), dim3(256), 0, s, st, pushmag, rows,
+                       nrows, n, radiation ? 1 : 0);
     SR_HIP(hipGetLastError());
     return SR_OK;
 }

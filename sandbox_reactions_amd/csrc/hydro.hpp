@@ -28,6 +28,7 @@ struct HydroState {
     float *mx, *my, *e, *x;
 };
 
+#define TAKE_ROWS 64  // rows of six that the partials are reduced to before the take-backs
 struct HydroPartials {
     double *sums;              // 5 per block: net kick x, y; net push x, y; sum |push|
     unsigned long long *keys;  // per block: the densest free cell's key (Sigma_mid bits, ~index)
@@ -46,7 +47,7 @@ int hydro_launch(int mode, const HydroParams &P, const HydroState &in, const Hyd
                  const float *rfy, float *sigma_mid_out, float *pushmag, double *escaped, const HydroPartials &part,
                  hipStream_t s, const SinkPlanes *sinks = nullptr);
 int hydro_takeback(const HydroParams &P, const HydroState &st, const float *pushmag, const HydroPartials &part,
-                   double *takeback, bool radiation, hipStream_t s);
+                   double *rows, bool radiation, hipStream_t s);
 int hydro_blocks(int w, int h);
 
 } // namespace sr

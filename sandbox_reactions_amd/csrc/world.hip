@@ -487,7 +487,7 @@ extern "C" int sr_world_create(int w, int h, const sr_physics *ph, const sr_swit
         return bail(fail(SR_ERR_DEVICE, "hipHostMalloc"));
     const int nb = hydro_blocks(w, h);
     wd->box_nb = (int)std::min<size_t>(1024, (n + NT - 1) / NT);
-    if ((c = world_alloc(wd, (void **)&wd->takeback, sizeof(double) * 8)) ||
+    if ((c = world_alloc(wd, (void **)&wd->takeback, sizeof(double) * 6 * TAKE_ROWS)) ||
         (c = world_alloc(wd, (void **)&wd->part.sums, sizeof(double) * 5 * nb)) ||
         (c = world_alloc(wd, (void **)&wd->part.keys, sizeof(unsigned long long) * nb)) ||
         (c = world_alloc(wd, (void **)&wd->rpart, sizeof(double) * 16 * 4096)) ||

@@ -105,6 +105,34 @@ def test_mixed_species_and_vacuum_match_the_twin(gpu_lib):
     assert np.max(np.abs(g[4:] - t[4:])) <= 2e-5
 
 
+@pytest.mark.parametrize("edge", [0, 1])
+@pytest.mark.parametrize("mu", [0.0, 0.6])
+@pytest.mark.parametrize("w,h", [(8, 8), (40, 24)])
+def test_species_that_only_some_tiles_hold(gpu_lib, w, h, mu, edge):
+    """Species in one cell, up to a tile's border (x = 16), in one corner, and nowhere: a species is left out of the
+    tiles that hold none of it within two cells, so what crosses their borders must be the twin's (FP64; one f32 step
+    moves a plane by ~1e-7 of its largest value per operation, a few tens of operations), and an absent one stays 0."""
+    print(f"partial species {w}x{h} mu {mu} edge {edge}", flush=True)
+    rng = np.random.default_rng(w + edge)
+    p = np.zeros((14, h, w))
+    p[0] = rng.uniform(0.5, 2.0, (h, w))
+    p[1:3] = p[0] * rng.uniform(-1.0, 1.0, (2, h, w))
+    p[3] = p[0] * 3.0 + 0.5 * (p[1] ** 2 + p[2] ** 2) / p[0]
+    p[5, :, :16] = 0.3                              # helium up to the border
+    p[6, h // 2, min(15, w - 1)] = 0.5              # carbon in one cell beside it
+    p[7, min(16, h - 1), min(17, w - 1)] = 0.5      # oxygen in one cell, a column beyond it
+    p[13, -1, -1] = 0.25                            # neutrons in the last corner
+    p[4] = 1.0 - p[5:].sum(axis=0)
+    twin, world = run_pair(p, 2, gravity=True, edge=edge, mu=mu)
+    g, t = world.readback(), twin.state()
+    for c in range(4):
+        assert rel_l1(g[c], t[c]) <= 1e-5, (c, rel_l1(g[c], t[c]))
+    for c in (4, 5, 6, 7, 13):
+        assert np.max(np.abs(g[c] - t[c])) <= 1e-5, (c, np.max(np.abs(g[c] - t[c])))
+        assert np.array_equal(g[c] != 0.0, t[c].astype(np.float32) != 0.0), c
+    assert not g[8:13].any()
+
+
 def test_mass_is_conserved_to_fp64_roundoff_and_reruns_are_bitwise(gpu_lib):
     import sandbox_reactions_amd as sr
     print("conservation", flush=True)
