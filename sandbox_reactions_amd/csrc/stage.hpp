@@ -1,0 +1,33 @@
+// Host transfers through pinned chunks: large planes between a caller's pageable memory and the device.
+#pragma once
+#include "common.hpp"
+
+namespace sr {
+
+#define STAGE_THREADS 4
+#define STAGE_SLOTS 2               // per thread: one is copied by the host while the other is on the bus
+#define STAGE_CHUNK (2u << 20)      // bytes of one slot
+#define STAGE_LEAST (8u << 20)      // transfers below this stay with the runtime's own copy
+
+// Not for concurrent use (a world's transfers are its caller's, one at a time). The pinned memory and the events are
+// kept from the first large transfer until release().
+class HostStage {
+  public:
+    // Queued on s: when it returns src may be changed, the device's copy is ordered on s
+    int to_device(void *dst, const void *src, size_t bytes, hipStream_t s);
+    // Done when it returns (s's work before it too)
+    int to_host(void *dst, const void *src, size_t bytes, hipStream_t s);
+    // After s's work is done
+    void release();
+
+  private:
+    bool ready();
+    hipError_t chunks_up(int k, int threads, char *dev, const char *host, size_t bytes, hipStream_t s);
+    hipError_t chunks_down(int k, int threads, const char *dev, char *host, size_t bytes, hipStream_t s);
+    template <class F> int spread(size_t bytes, F part);
+    char *buf = nullptr;
+    hipEvent_t ev[STAGE_THREADS * STAGE_SLOTS] = {};
+    bool refused = false;  // no pinned memory to be had: the runtime's own copies
+};
+
+} // namespace sr

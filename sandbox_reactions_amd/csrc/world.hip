@@ -19,6 +19,7 @@
 #include "hydro.hpp"
 #include "react.hpp"
 #include "sinks.hpp"
+#include "stage.hpp"
 
 namespace sr {
 
@@ -408,6 +409,7 @@ struct sr_world {
     int *box = nullptr, *box_part = nullptr;
     int box_nb = 1;
     std::vector<void *> allocs;
+    HostStage stage;  // the planes' way in and out
 };
 
 static int world_alloc(sr_world *wd, void **p, size_t bytes) {
@@ -433,6 +435,7 @@ extern "C" void sr_destroy(sr_world *wd) {
     if (wd->s) (void)hipStreamSynchronize(wd->s);
     for (void *p : wd->allocs) (void)hipFree(p);
     if (wd->host_scal) (void)hipHostFree(wd->host_scal);
+    wd->stage.release();
     for (auto &e : wd->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto &row : wd->g_front)
@@ -633,7 +636,7 @@ extern "C" int sr_upload(sr_world *wd, const float *planes, size_t n) {
     if (!planes) return fail(SR_ERR_ARGUMENT, "sr_upload: null planes");
     float *tmp = nullptr;
     SR_HIP(hipMallocAsync((void **)&tmp, sizeof(float) * n, wd->s));
-    SR_HIP(hipMemcpyAsync(tmp, planes, sizeof(float) * n, hipMemcpyHostToDevice, wd->s));
+    SR_TRY(wd->stage.to_device(tmp, planes, sizeof(float) * n, wd->s));
     wd->cur = 0;
     hipLaunchKernelGGL(k_upload, dim3((wd->n + 255) / 256), dim3(256), 0, wd->s, tmp, wd->st[0], (int)wd->n);
     SR_HIP(hipFreeAsync(tmp, wd->s));
@@ -664,9 +667,8 @@ extern "C" int sr_readback(sr_world *wd, float *planes, size_t n) {
     float *tmp = nullptr;
     SR_HIP(hipMallocAsync((void **)&tmp, sizeof(float) * n, wd->s));
     hipLaunchKernelGGL(k_readback, dim3((wd->n + 255) / 256), dim3(256), 0, wd->s, wd->st[wd->cur], tmp, (int)wd->n);
-    SR_HIP(hipMemcpyAsync(planes, tmp, sizeof(float) * n, hipMemcpyDeviceToHost, wd->s));
+    SR_TRY(wd->stage.to_host(planes, tmp, sizeof(float) * n, wd->s));
     SR_HIP(hipFreeAsync(tmp, wd->s));
-    SR_HIP(hipStreamSynchronize(wd->s));
     return SR_OK;
 }
 
