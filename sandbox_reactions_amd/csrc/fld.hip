@@ -874,11 +874,58 @@ struct CoarseSet {
     int lw[16];        // log2 of the level's width when a power of two, else -1
     int head, ltx;     // register-resident levels (0 or 2); log2 TX of the block's TX x (COARSE_NT / TX) layout
     int offza, offzb, offrb;  // LDS: the head levels' published z, the second level's residuals
+    int offrec;        // the head's records in the pack (16-byte aligned)
+    int tail, offtail; // the first level a wave tail could run (or -1), its lanes' records in the pack and in LDS
     int wave;          // the first level the wave tail runs, or -1
+};
+
+// What a thread holding a 2x2 block of one level and its aggregate's cell of the next reads of the system, BLOCK_REC
+// floats: own and inverse diagonals of the block, its x faces (three to a row), its y faces (two to a row), then own,
+// inverse diagonal, left, right, up and down of the next level's cell; zeros off the grid. Formed at the rebuild and kept
+// as float4s of all threads one after the other (float4 q of thread t at q threads + t), for the head's threads and for
+// the wave tail's lanes: read cell by cell at the levels' own strides, they were 9300 of the launch's 29600 cycles at
+// 64^2 (4800 now) and 3000 of the wave tail's 8300. With the head's neighbours at addresses formed once and the inverse's
+// rows loaded ahead the launch takes 9.9 us instead of 14.6 at 64^2, 9.5 instead of 12.9 at 500 x 300.
+#define BLOCK_REC 28
+struct Block {
+    float o[4], rd[4], l[4], r[4], u[4], d[4];
+    float o1, rd1, l1, r1, u1, d1;
+    __device__ __forceinline__ Block(const float4 *rec, int threads) {
+        float f[BLOCK_REC];
+#pragma unroll
+        for (int q = 0; q < BLOCK_REC / 4; q++) {
+            const float4 v = rec[q * threads];
+            f[4 * q] = v.x;
+            f[4 * q + 1] = v.y;
+            f[4 * q + 2] = v.z;
+            f[4 * q + 3] = v.w;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i = k & 1, j = k >> 1;
+            o[k] = f[k];
+            rd[k] = f[4 + k];
+            l[k] = f[8 + 3 * j + i];
+            r[k] = f[9 + 3 * j + i];
+            u[k] = f[14 + 2 * j + i];
+            d[k] = f[16 + 2 * j + i];
+        }
+        o1 = f[20];
+        rd1 = f[21];
+        l1 = f[22];
+        r1 = f[23];
+        u1 = f[24];
+        d1 = f[25];
+    }
 };
 
 // (y, x) of entry t in rows of width w: a shift when w is a power of two (lw >= 0), a division otherwise
 __device__ __forceinline__ int row_of(int t, int w, int lw) { return lw >= 0 ? t >> lw : t / w; }
+
+// v of another lane of the row of 16, by the data-parallel primitives' control word; 0 past the row's end
+template <int CTRL> __device__ __forceinline__ float lane_move(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
 
 template <bool HEAD>
 __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *__restrict__ pack,
@@ -895,9 +942,11 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
     // cell (tx, ty)
     const int tx = HEAD ? (int)(threadIdx.x & ((1u << C.ltx) - 1)) : 0, ty = HEAD ? (int)(threadIdx.x >> C.ltx) : 0;
     const int wA = C.w[0], hA = C.h[0], wB = C.w[1], hB = C.h[1], x0 = 2 * tx, y0 = 2 * ty;
-    float ab[4], az[4], ao[4], ard[4], al[4], ar[4], au[4], ad[4];
-    float bb = 0.0f, zb = 0.0f, bo = 0.0f, brd = 0.0f, bl = 0.0f, br = 0.0f, bu = 0.0f, bd = 0.0f;
+    const bool in[4] = {x0 < wA && y0 < hA, x0 + 1 < wA && y0 < hA, x0 < wA && y0 + 1 < hA, x0 + 1 < wA && y0 + 1 < hA};
+    float ab[4], az[4];
+    float bb = 0.0f, zb = 0.0f;
     const bool vb = HEAD && tx < wB && ty < hB;
+    const Block A((const float4 *)(pack + (HEAD ? C.offrec : 0)) + (HEAD ? threadIdx.x : 0), HEAD ? COARSE_NT : 1);
     // one phase: every load issued before any is used (the pack's LDS part as float4, level 0's b or the head's
     // registers), then zeros elsewhere (every entry a sweep may read at a grid's rim is finite)
     {
@@ -912,29 +961,19 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
             v[k] = t < np4 ? p4[t] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
         if constexpr (HEAD) {
+            if (!(wA & 1) && !((uintptr_t)b0 & 7)) {  // a row's pair in one load (b0 may be a caller's)
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int x = x0 + (k & 1), y = y0 + (k >> 1);
-                const bool in = x < wA && y < hA;
-                const int i = y * wA + x;
-                ab[k] = in ? b0[i] : 0.0f;
-                ao[k] = in ? pack[offo[0] + i] : 0.0f;
-                ard[k] = in ? pack[offd[0] + i] : 0.0f;
-                al[k] = in ? pack[offx[0] + y * (wA + 1) + x] : 0.0f;
-                ar[k] = in ? pack[offx[0] + y * (wA + 1) + x + 1] : 0.0f;
-                au[k] = in ? pack[offy[0] + i] : 0.0f;
-                ad[k] = in ? pack[offy[0] + i + wA] : 0.0f;
-                az[k] = 0.0f;
+                for (int j = 0; j < 2; j++) {
+                    const float2 v2 = in[2 * j] ? *(const float2 *)(b0 + (y0 + j) * wA + x0) : make_float2(0.0f, 0.0f);
+                    ab[2 * j] = v2.x;
+                    ab[2 * j + 1] = v2.y;
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++) ab[k] = in[k] ? b0[(y0 + (k >> 1)) * wA + x0 + (k & 1)] : 0.0f;
             }
-            if (vb) {
-                const int i = ty * wB + tx;
-                bo = pack[offo[1] + i];
-                brd = pack[offd[1] + i];
-                bl = pack[offx[1] + ty * (wB + 1) + tx];
-                br = pack[offx[1] + ty * (wB + 1) + tx + 1];
-                bu = pack[offy[1] + i];
-                bd = pack[offy[1] + i + wB];
-            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) az[k] = 0.0f;
         } else {
 #pragma unroll
             for (int k = 0; k < VB; k++) {
@@ -1032,7 +1071,7 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
             const float *b = sm + offb[lc], *ainv = sm + offinv;
             if (threadIdx.x < m) {
                 float t = 0.0f;
-                for (int j = 0; j < m; j++) t += ainv[threadIdx.x * m + j] * b[j];
+                for (int j = 0; j < m; j++) t += ainv[threadIdx.x * DENSE_MAX + j] * b[j];
                 z[threadIdx.x] = t;
             }
             __syncthreads();
@@ -1047,45 +1086,34 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
             }
         }
     };
-    // the head's LDS: the first and second level's published z, the second level's residuals
-    float *za = sm + C.offza, *zbl = sm + C.offzb, *rb = sm + C.offrb;
-    // a first-level z outside the thread's block (clamped into the grid: a rim coupling is zero)
-    auto ZA = [&](int x, int y) {
-        return za[min(max(y, 0), hA - 1) * wA + min(max(x, 0), wA - 1)];
-    };
-    auto ZB = [&](int x, int y) {
-        return zbl[min(max(y, 0), hB - 1) * wB + min(max(x, 0), wB - 1)];
-    };
-    auto publish_a = [&](int k) {
-        const int x = x0 + (k & 1), y = y0 + (k >> 1);
-        if (x < wA && y < hA) za[y * wA + x] = az[k];
+    // the head's LDS: the first level's published z as four planes, one to a cell of the 2x2 block, the second level's
+    // as one, each a thread's entry beside its neighbours' within a rim of zeros: every exchange reads consecutive words
+    // from addresses formed once; and the second level's residuals
+    const int S = (1 << C.ltx) + 2, PS = S * ((COARSE_NT >> C.ltx) + 2), at = (ty + 1) * S + tx + 1;
+    float *p0 = sm + C.offza + at, *p1 = p0 + PS, *p2 = p1 + PS, *p3 = p2 + PS, *pb = sm + C.offzb + at;
+    float *rb = sm + C.offrb;
+    auto publish_a = [&](float *p, int k) {
+        if (in[k]) *p = az[k];
     };
     // a half sweep of the first level: colour 0 holds cells 0 and 3 of the block, colour 1 cells 1 and 2
     auto sweep_a = [&](int color) {
         if (color == 0) {
-            az[0] = (ab[0] + al[0] * ZA(x0 - 1, y0) + ar[0] * az[1] + au[0] * ZA(x0, y0 - 1) + ad[0] * az[2]) *
-                    ard[0];
-            az[3] = (ab[3] + al[3] * az[2] + ar[3] * ZA(x0 + 2, y0 + 1) + au[3] * az[1] +
-                     ad[3] * ZA(x0 + 1, y0 + 2)) *
-                    ard[3];
-            publish_a(0);
-            publish_a(3);
+            az[0] = (ab[0] + A.l[0] * p1[-1] + A.r[0] * az[1] + A.u[0] * p2[-S] + A.d[0] * az[2]) * A.rd[0];
+            az[3] = (ab[3] + A.l[3] * az[2] + A.r[3] * p2[1] + A.u[3] * az[1] + A.d[3] * p1[S]) * A.rd[3];
+            publish_a(p0, 0);
+            publish_a(p3, 3);
         } else {
-            az[1] = (ab[1] + al[1] * az[0] + ar[1] * ZA(x0 + 2, y0) + au[1] * ZA(x0 + 1, y0 - 1) + ad[1] * az[3]) *
-                    ard[1];
-            az[2] = (ab[2] + al[2] * ZA(x0 - 1, y0 + 1) + ar[2] * az[3] + au[2] * az[0] +
-                     ad[2] * ZA(x0, y0 + 2)) *
-                    ard[2];
-            publish_a(1);
-            publish_a(2);
+            az[1] = (ab[1] + A.l[1] * az[0] + A.r[1] * p0[1] + A.u[1] * p3[-S] + A.d[1] * az[3]) * A.rd[1];
+            az[2] = (ab[2] + A.l[2] * p3[-1] + A.r[2] * az[3] + A.u[2] * az[0] + A.d[2] * p0[S]) * A.rd[2];
+            publish_a(p1, 1);
+            publish_a(p2, 2);
         }
         __syncthreads();
     };
     auto sweep_b = [&](int color) {
         if (vb && ((tx + ty) & 1) == color) {
-            zb = (bb + bl * ZB(tx - 1, ty) + br * ZB(tx + 1, ty) + bu * ZB(tx, ty - 1) + bd * ZB(tx, ty + 1)) *
-                 brd;
-            zbl[ty * wB + tx] = zb;
+            zb = (bb + A.l1 * pb[-1] + A.r1 * pb[1] + A.u1 * pb[-S] + A.d1 * pb[S]) * A.rd1;
+            *pb = zb;
         }
         __syncthreads();
     };
@@ -1098,17 +1126,16 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
         }
         {
             float s = 0.0f;
-            const float zn[4][4] = {{ZA(x0 - 1, y0), az[1], ZA(x0, y0 - 1), az[2]},
-                                    {az[0], ZA(x0 + 2, y0), ZA(x0 + 1, y0 - 1), az[3]},
-                                    {ZA(x0 - 1, y0 + 1), az[3], az[0], ZA(x0, y0 + 2)},
-                                    {az[2], ZA(x0 + 2, y0 + 1), az[1], ZA(x0 + 1, y0 + 2)}};
+            const float zn[4][4] = {{p1[-1], az[1], p2[-S], az[2]},
+                                    {az[0], p0[1], p3[-S], az[3]},
+                                    {p3[-1], az[3], az[0], p0[S]},
+                                    {az[2], p2[1], az[1], p1[S]}};
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                const int x = x0 + (k & 1), y = y0 + (k >> 1);
-                if (x >= wA || y >= hA) continue;
+                if (!in[k]) continue;
                 const float zi = az[k];
-                const float azi = ao[k] * zi + al[k] * (zi - zn[k][0]) + ar[k] * (zi - zn[k][1]) +
-                                  au[k] * (zi - zn[k][2]) + ad[k] * (zi - zn[k][3]);
+                const float azi = A.o[k] * zi + A.l[k] * (zi - zn[k][0]) + A.r[k] * (zi - zn[k][1]) +
+                                  A.u[k] * (zi - zn[k][2]) + A.d[k] * (zi - zn[k][3]);
                 s += ab[k] - azi;
             }
             bb = s;
@@ -1120,8 +1147,8 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
         }
         if (vb) {
             const float zi = zb;
-            const float azi = bo * zi + bl * (zi - ZB(tx - 1, ty)) + br * (zi - ZB(tx + 1, ty)) +
-                              bu * (zi - ZB(tx, ty - 1)) + bd * (zi - ZB(tx, ty + 1));
+            const float azi =
+                A.o1 * zi + A.l1 * (zi - pb[-1]) + A.r1 * (zi - pb[1]) + A.u1 * (zi - pb[-S]) + A.d1 * (zi - pb[S]);
             rb[ty * wB + tx] = bb - azi;
         }
         __syncthreads();
@@ -1153,33 +1180,43 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
         const int lane = (int)threadIdx.x, qx = lane & 7, qy = lane >> 3;
         const int w = C.w[s0], h = C.h[s0], s1 = s0 + 1, w1 = C.w[s1], h1 = C.h[s1];
         auto nb = [&](float v, int src) { return __shfl(v, src, 64); };
-        float b[4], z[4], o[4], rd[4], cl[4], cr[4], cu[4], cd[4];
+        // the lane before and the lane after, within rows of 16 lanes (two of the grid's: past their ends a zero, by
+        // data-parallel moves, not through LDS)
+        auto before = [](float v) { return lane_move<0x111>(v); };
+        auto after = [](float v) { return lane_move<0x101>(v); };
+        const Block Q((const float4 *)(sm + C.offtail) + lane, 64);
+        float b[4], z[4];
         bool in[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const int x = 2 * qx + (k & 1), y = 2 * qy + (k >> 1), i = y * w + x;
+            const int x = 2 * qx + (k & 1), y = 2 * qy + (k >> 1);
             in[k] = x < w && y < h;
-            b[k] = in[k] ? sm[offb[s0] + i] : 0.0f;
-            o[k] = in[k] ? sm[offo[s0] + i] : 0.0f;
-            rd[k] = in[k] ? sm[offd[s0] + i] : 0.0f;
-            cl[k] = in[k] ? sm[offx[s0] + y * (w + 1) + x] : 0.0f;
-            cr[k] = in[k] ? sm[offx[s0] + y * (w + 1) + x + 1] : 0.0f;
-            cu[k] = in[k] ? sm[offy[s0] + i] : 0.0f;
-            cd[k] = in[k] ? sm[offy[s0] + i + w] : 0.0f;
+            const float v = sm[offb[s0] + (in[k] ? y * w + x : 0)];
+            b[k] = in[k] ? v : 0.0f;
             z[k] = 0.0f;
+        }
+        // the lane's row of the inverse (zeros past its m entries), all its loads in flight together
+        float inv[DENSE_MAX];
+#pragma unroll
+        for (int j = 0; j < DENSE_MAX; j += 4) {
+            const float4 v = *(const float4 *)(sm + offinv + (lane < m ? lane : 0) * DENSE_MAX + j);
+            inv[j] = v.x;
+            inv[j + 1] = v.y;
+            inv[j + 2] = v.z;
+            inv[j + 3] = v.w;
         }
         // colour 0 holds cells 0 and 3 of the block, colour 1 cells 1 and 2
         auto sweep0 = [&](int color) {
             if (color == 0) {
-                const float L1 = nb(z[1], lane - 1), U2 = nb(z[2], lane - 8), R2 = nb(z[2], lane + 1),
+                const float L1 = before(z[1]), U2 = nb(z[2], lane - 8), R2 = after(z[2]),
                             D1 = nb(z[1], lane + 8);
-                if (in[0]) z[0] = (b[0] + cl[0] * L1 + cr[0] * z[1] + cu[0] * U2 + cd[0] * z[2]) * rd[0];
-                if (in[3]) z[3] = (b[3] + cl[3] * z[2] + cr[3] * R2 + cu[3] * z[1] + cd[3] * D1) * rd[3];
+                if (in[0]) z[0] = (b[0] + Q.l[0] * L1 + Q.r[0] * z[1] + Q.u[0] * U2 + Q.d[0] * z[2]) * Q.rd[0];
+                if (in[3]) z[3] = (b[3] + Q.l[3] * z[2] + Q.r[3] * R2 + Q.u[3] * z[1] + Q.d[3] * D1) * Q.rd[3];
             } else {
-                const float R0 = nb(z[0], lane + 1), U3 = nb(z[3], lane - 8), L3 = nb(z[3], lane - 1),
+                const float R0 = after(z[0]), U3 = nb(z[3], lane - 8), L3 = before(z[3]),
                             D0 = nb(z[0], lane + 8);
-                if (in[1]) z[1] = (b[1] + cl[1] * z[0] + cr[1] * R0 + cu[1] * U3 + cd[1] * z[3]) * rd[1];
-                if (in[2]) z[2] = (b[2] + cl[2] * L3 + cr[2] * z[3] + cu[2] * z[0] + cd[2] * D0) * rd[2];
+                if (in[1]) z[1] = (b[1] + Q.l[1] * z[0] + Q.r[1] * R0 + Q.u[1] * U3 + Q.d[1] * z[3]) * Q.rd[1];
+                if (in[2]) z[2] = (b[2] + Q.l[2] * L3 + Q.r[2] * z[3] + Q.u[2] * z[0] + Q.d[2] * D0) * Q.rd[2];
             }
         };
         for (int k = 0; k < nu1; k++) {
@@ -1189,17 +1226,17 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
         // the residual of the block restricted into the lane's cell of the next level (cells in row order)
         float b1 = 0.0f;
         {
-            const float L1 = nb(z[1], lane - 1), U2 = nb(z[2], lane - 8), R0 = nb(z[0], lane + 1),
-                        U3 = nb(z[3], lane - 8), L3 = nb(z[3], lane - 1), D0 = nb(z[0], lane + 8),
-                        R2 = nb(z[2], lane + 1), D1 = nb(z[1], lane + 8);
+            const float L1 = before(z[1]), U2 = nb(z[2], lane - 8), R0 = after(z[0]),
+                        U3 = nb(z[3], lane - 8), L3 = before(z[3]), D0 = nb(z[0], lane + 8),
+                        R2 = after(z[2]), D1 = nb(z[1], lane + 8);
             const float zn[4][4] = {{L1, z[1], U2, z[2]}, {z[0], R0, U3, z[3]}, {L3, z[3], z[0], D0},
                                     {z[2], R2, z[1], D1}};
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 if (!in[k]) continue;
                 const float zi = z[k];
-                const float azi = o[k] * zi + cl[k] * (zi - zn[k][0]) + cr[k] * (zi - zn[k][1]) +
-                                  cu[k] * (zi - zn[k][2]) + cd[k] * (zi - zn[k][3]);
+                const float azi = Q.o[k] * zi + Q.l[k] * (zi - zn[k][0]) + Q.r[k] * (zi - zn[k][1]) +
+                                  Q.u[k] * (zi - zn[k][2]) + Q.d[k] * (zi - zn[k][3]);
                 b1 += b[k] - azi;
             }
         }
@@ -1212,12 +1249,12 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
 #pragma unroll
             for (int j = 0; j < DENSE_MAX; j++) bj[j] = nb(bv, src(j));
             float zt = 0.0f;
-            if (lane < m) {
 #pragma unroll
-                for (int j = 0; j < DENSE_MAX; j++)
-                    if (j < m) zt += sm[offinv + lane * m + j] * bj[j];
+            for (int j = 0; j < DENSE_MAX; j++) {
+                const float next = zt + inv[j] * bj[j];
+                zt = j < m ? next : zt;
             }
-            return zt;
+            return lane < m ? zt : 0.0f;
         };
         if (s1 == lc) {
             // the next level is the coarsest
@@ -1227,14 +1264,10 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
             for (int k = 0; k < 4; k++)
                 if (in[k]) z[k] += omega * z1;
         } else {
-            const float o1 = v1 ? sm[offo[s1] + i1] : 0.0f, rd1 = v1 ? sm[offd[s1] + i1] : 0.0f;
-            const float l1 = v1 ? sm[offx[s1] + qy * (w1 + 1) + qx] : 0.0f;
-            const float r1 = v1 ? sm[offx[s1] + qy * (w1 + 1) + qx + 1] : 0.0f;
-            const float u1 = v1 ? sm[offy[s1] + i1] : 0.0f, d1 = v1 ? sm[offy[s1] + i1 + w1] : 0.0f;
             float z1 = 0.0f;
             auto sweep1 = [&](int color) {
-                const float L = nb(z1, lane - 1), R = nb(z1, lane + 1), U = nb(z1, lane - 8), D = nb(z1, lane + 8);
-                if (v1 && ((qx + qy) & 1) == color) z1 = (b1 + l1 * L + r1 * R + u1 * U + d1 * D) * rd1;
+                const float L = before(z1), R = after(z1), U = nb(z1, lane - 8), D = nb(z1, lane + 8);
+                if (v1 && ((qx + qy) & 1) == color) z1 = (b1 + Q.l1 * L + Q.r1 * R + Q.u1 * U + Q.d1 * D) * Q.rd1;
             };
             for (int k = 0; k < nu1; k++) {
                 sweep1(0);
@@ -1243,8 +1276,8 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
             // the residual, restricted into the coarsest (lane t forming its cell t), the dense solve
             float r = 0.0f;
             {
-                const float L = nb(z1, lane - 1), R = nb(z1, lane + 1), U = nb(z1, lane - 8), D = nb(z1, lane + 8);
-                const float azi = o1 * z1 + l1 * (z1 - L) + r1 * (z1 - R) + u1 * (z1 - U) + d1 * (z1 - D);
+                const float L = before(z1), R = after(z1), U = nb(z1, lane - 8), D = nb(z1, lane + 8);
+                const float azi = Q.o1 * z1 + Q.l1 * (z1 - L) + Q.r1 * (z1 - R) + Q.u1 * (z1 - U) + Q.d1 * (z1 - D);
                 r = b1 - azi;
             }
             const int w2 = C.w[lc], X = lane % w2, Y = lane / w2;
@@ -1279,20 +1312,20 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
             if (in[k]) sm[offz[s0] + y * w + x] = z[k];
         }
     };
-    const int S = C.wave >= 0 ? C.wave : lc;
-    for (int l = T; l < S; l++) down(l);
+    const int last = C.wave >= 0 ? C.wave : lc;
+    for (int l = T; l < last; l++) down(l);
     if (C.wave >= 0) {
-        if (threadIdx.x < 64) wave_tail(S);
+        if (threadIdx.x < 64) wave_tail(last);
         __syncthreads();
     } else {
         coarsest();
     }
-    for (int l = S - 1; l >= T; l--) up(l);
+    for (int l = last - 1; l >= T; l--) up(l);
     if constexpr (HEAD) {
         // the second level: the tail's correction prolonged, published, post-smoothed
         if (vb) {
             zb += omega * sm[offz[T] + (ty >> 1) * C.w[T] + (tx >> 1)];
-            zbl[ty * wB + tx] = zb;
+            *pb = zb;
         }
         __syncthreads();
         for (int k = 0; k < nu2; k++) {
@@ -1302,19 +1335,24 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse(CoarseSet C, const float *
         // the first level: the second level's correction (the thread's own cell) prolonged, published,
         // post-smoothed, written out
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            az[k] += omega * zb;
-            publish_a(k);
-        }
+        for (int k = 0; k < 4; k++) az[k] += omega * zb;
+        publish_a(p0, 0);
+        publish_a(p1, 1);
+        publish_a(p2, 2);
+        publish_a(p3, 3);
         __syncthreads();
         for (int k = 0; k < nu2; k++) {
             sweep_a(1);
             sweep_a(0);
         }
+        if (!(wA & 1) && !((uintptr_t)z0 & 7)) {
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int x = x0 + (k & 1), y = y0 + (k >> 1);
-            if (x < wA && y < hA) z0[y * wA + x] = az[k];
+            for (int j = 0; j < 2; j++)
+                if (in[2 * j]) *(float2 *)(z0 + (y0 + j) * wA + x0) = make_float2(az[2 * j], az[2 * j + 1]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (in[k]) z0[(y0 + (k >> 1)) * wA + x0 + (k & 1)] = az[k];
         }
     } else {
         for (int t = threadIdx.x; t < n0; t += COARSE_NT) z0[t] = sm[offz[0] + t];
@@ -1385,6 +1423,49 @@ __global__ void k_coarsen_faces(Lv f, float *__restrict__ axc, float *__restrict
 // Gauss-Jordan elimination (the matrix is SPD, so no pivoting); both into the pack. The elimination runs on the first
 // wave alone, row i of [A | I] in lane i's registers and the pivot row read across lanes, so it needs no block
 // barrier; the other waves form the inverse diagonals meanwhile.
+// The records (struct Block) of `threads` threads, 2^ltx to a row, over set level l and the next; entries t0, t0 + nt, ..
+__device__ inline void block_records(const CoarseSet &C, float *pack, int l, int ltx, int threads, int offrec, int t0,
+                                     int nt) {
+    const int w = C.w[l], h = C.h[l], w1 = C.w[l + 1], h1 = C.h[l + 1];
+    const float *own = pack + C.offo[l], *fx = pack + C.offx[l], *fy = pack + C.offy[l];
+    const float *own1 = pack + C.offo[l + 1], *fx1 = pack + C.offx[l + 1], *fy1 = pack + C.offy[l + 1];
+    for (int t = t0; t < threads; t += nt) {
+        const int tx = t & ((1 << ltx) - 1), ty = t >> ltx, x0 = 2 * tx, y0 = 2 * ty;
+        float r[BLOCK_REC];
+#pragma unroll
+        for (int j = 0; j < BLOCK_REC; j++) r[j] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int i = 0; i < 3; i++)
+                if (x0 + i <= w && y0 + j < h) r[8 + 3 * j + i] = fx[(y0 + j) * (w + 1) + x0 + i];
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                if (x0 + i < w && y0 + j <= h) r[14 + 2 * j + i] = fy[(y0 + j) * w + x0 + i];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i = k & 1, j = k >> 1;
+            if (x0 + i >= w || y0 + j >= h) continue;
+            r[k] = own[(y0 + j) * w + x0 + i];
+            r[4 + k] = 1.0f / (r[k] + r[8 + 3 * j + i] + r[9 + 3 * j + i] + r[14 + 2 * j + i] + r[16 + 2 * j + i]);
+        }
+        if (tx < w1 && ty < h1) {
+            r[20] = own1[ty * w1 + tx];
+            r[22] = fx1[ty * (w1 + 1) + tx];
+            r[23] = fx1[ty * (w1 + 1) + tx + 1];
+            r[24] = fy1[ty * w1 + tx];
+            r[25] = fy1[(ty + 1) * w1 + tx];
+            r[21] = 1.0f / (r[20] + r[22] + r[23] + r[24] + r[25]);
+        }
+        float4 *rec = (float4 *)(pack + offrec) + t;
+#pragma unroll
+        for (int q = 0; q < BLOCK_REC / 4; q++)
+            rec[q * threads] = make_float4(r[4 * q], r[4 * q + 1], r[4 * q + 2], r[4 * q + 3]);
+    }
+}
+
 __global__ void __launch_bounds__(COARSE_NT) k_coarse_prep(CoarseSet C, float *__restrict__ pack) {
     const int lc = C.n - 1, wl = C.w[lc], m = wl * C.h[lc];
     const bool dense = m <= DENSE_MAX;
@@ -1433,12 +1514,14 @@ __global__ void __launch_bounds__(COARSE_NT) k_coarse_prep(CoarseSet C, float *_
             float *ainv = pack + C.offinv;
 #pragma unroll
             for (int j = 0; j < 2 * DENSE_MAX; j++)
-                if (j >= m && j < 2 * m) ainv[i * m + j - m] = A[j] / d;
+                if (j >= m && j < 2 * m) ainv[i * DENSE_MAX + j - m] = A[j] / d;
         }
     }
     const int t0 = dense ? (int)threadIdx.x - 64 : (int)threadIdx.x, nt = dense ? COARSE_NT - 64 : COARSE_NT;
     if (t0 < 0) return;
-    for (int l = 0; l < C.n; l++) {
+    if (C.head) block_records(C, pack, 0, C.ltx, COARSE_NT, C.offrec, t0, nt);
+    if (C.tail >= 0) block_records(C, pack, C.tail, 3, 64, C.offtail, t0, nt);
+    for (int l = C.head; l < C.n; l++) {
         const int w = C.w[l], h = C.h[l];
         const float *own = pack + C.offo[l], *al = pack + C.offx[l], *au = pack + C.offy[l];
         float *rd = pack + C.offd[l];
@@ -1574,6 +1657,7 @@ int FldSolver::init(int w, int h, int levels, int nu1_, int nu2_, double omega_)
     pack_floats = DENSE_MAX * DENSE_MAX;
     for (int l = coarse_from; l < (int)lv.size(); l++)
         pack_floats += (int)level_floats(lv[l].w, lv[l].h) + lv[l].w * lv[l].h;  // + the inverse diagonals
+    pack_floats += BLOCK_REC * (64 + (head ? COARSE_NT : 0)) + 4;
     SR_HIP(hipMalloc(&pack, sizeof(float) * pack_floats));
     SR_HIP(hipMemset(pack, 0, sizeof(float) * pack_floats));
     {
@@ -1634,9 +1718,9 @@ int FldSolver::init(int w, int h, int levels, int nu1_, int nu2_, double omega_)
     SR_HIP(hipMemset(ticket, 0, sizeof(unsigned)));
     SR_HIP(hipHostMalloc(&host_ctl, sizeof(SolveCtl)));
     SR_HIP(hipFuncSetAttribute((const void *)k_coarse<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               COARSE_LDS));
+                               COARSE_LDS + (int)sizeof(float) * BLOCK_REC * 64));
     SR_HIP(hipFuncSetAttribute((const void *)k_coarse<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               COARSE_LDS));
+                               COARSE_LDS + (int)sizeof(float) * BLOCK_REC * 64));
     return SR_OK;
 }
 
@@ -1655,10 +1739,10 @@ int FldSolver::set_system(const float *own, const float *ax, const float *ay, co
     return rebuild(true, s);
 }
 
-// The single-block levels' layout. The pack holds first the tail levels' own, ax, ay, the coarsest's inverse and the
-// tail levels' inverse diagonals (the part the block copies into LDS, at the same offsets there), then the head
-// levels' own, ax, ay and inverse diagonals (read into registers). In LDS after the tail part: z and b per tail level,
-// then the head's published z of its two levels and the second level's residuals.
+// The single-block levels' layout. The pack holds first the coarsest's inverse (rows of DENSE_MAX), the wave tail's
+// records, the tail levels' own, ax, ay and inverse diagonals (the part the block copies into LDS, at the same offsets
+// there), then the head levels' own, ax and ay and the head's records (read into registers). In LDS after the tail part:
+// z and b per tail level, then the head's published z of its two levels and the second level's residuals.
 CoarseSet FldSolver::coarse_set() const {
     const int nl = (int)lv.size();
     CoarseSet C;
@@ -1680,20 +1764,25 @@ CoarseSet FldSolver::coarse_set() const {
         C.h[k] = lv[coarse_from + k].h;
         C.lw[k] = is_pow2(C.w[k]) ? ilog2(C.w[k]) : -1;
     }
+    // a wave tail could run from the first level past the head of at most 16 x 16 cells, when one or two levels follow
+    // it and the last is solved by the dense inverse
+    const int lc = C.n - 1;
+    int first = head;
+    while (first < C.n && (C.w[first] > 16 || C.h[first] > 16)) first++;
+    const bool tail = (lc - first == 1 || lc - first == 2) && C.w[lc] * C.h[lc] <= DENSE_MAX;
+    C.tail = tail ? first : -1;
+    C.wave = coarse_wave ? C.tail : -1;
+    C.offinv = 0;
+    C.offtail = DENSE_MAX * DENSE_MAX;
+    o = C.offtail + (tail ? BLOCK_REC * 64 : 0);
     for (int k = head; k < C.n; k++) level(k);
-    C.offinv = o;
-    o += DENSE_MAX * DENSE_MAX;
     for (int k = head; k < C.n; k++) {
         C.offd[k] = o;
         o += C.w[k] * C.h[k];
     }
     C.pack_floats = o;
     for (int k = 0; k < head; k++) level(k);
-    for (int k = 0; k < head; k++) {
-        C.offd[k] = o;
-        o += C.w[k] * C.h[k];
-    }
-    // o is the whole pack's size here
+    C.offrec = (o + 3) & ~3;  // the pack's end
     o = C.pack_floats;
     for (int k = head; k < C.n; k++) {
         C.offz[k] = o;
@@ -1703,23 +1792,15 @@ CoarseSet FldSolver::coarse_set() const {
     }
     C.offza = C.offzb = C.offrb = o;
     if (head) {
+        const int plane = ((1 << ltx) + 2) * ((COARSE_NT >> ltx) + 2);
         C.offza = o;
-        o += C.w[0] * C.h[0];
+        o += 4 * plane;
         C.offzb = o;
-        o += C.w[1] * C.h[1];
+        o += plane;
         C.offrb = o;
         o += C.w[1] * C.h[1];
     }
     C.total = o;
-    // the wave tail: from the first level past the head of at most 16 x 16 cells, when one or two levels follow it
-    // and the last is solved by the dense inverse
-    C.wave = -1;
-    if (coarse_wave) {
-        int s = head;
-        while (s < C.n && (C.w[s] > 16 || C.h[s] > 16)) s++;
-        const int lc = C.n - 1;
-        if (s < C.n && (lc - s == 1 || lc - s == 2) && C.w[lc] * C.h[lc] <= DENSE_MAX) C.wave = s;
-    }
     return C;
 }
 

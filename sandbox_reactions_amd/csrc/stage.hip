@@ -1,8 +1,8 @@
 // Host transfers through pinned chunks. The runtime copies pageable memory through one staging buffer on the calling
-// thread: 26 GB/s up and 10 GB/s down (into fresh pages) at 235 MB. Here a few threads
-// copy chunks between the caller's memory and pinned slots while the copies of the slots before are on the bus: 36 GB/s both ways. Four threads of two 2 MiB slots: 1 MiB slots
-// take 18 % longer; below 8 MiB the threads and the pinned memory (0.4 ms once) cost what they give (3.7 MB: 0.24 ms
-// either way).
+// thread: 26 GB/s up and 10 GB/s down (into fresh pages) at 235 MB. Here a few threads copy chunks between the caller's
+// memory and pinned slots while the copies of the slots before are on the bus: 36 GB/s both ways. Four threads of two
+// 2 MiB slots: 1 MiB slots take 18 % longer; below 8 MiB the threads and the pinned memory (0.4 ms once) cost what they
+// give (3.7 MB: 0.24 ms either way).
 #include <algorithm>
 #include <cstring>
 #include <system_error>
