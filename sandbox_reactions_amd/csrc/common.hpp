@@ -163,24 +163,56 @@ __device__ inline void block_partials(double (&v)[K], double *part, int nb, int 
     }
 }
 
-// The sum of nb partials in a fixed order; every thread of the block gets the result.
-__device__ inline double sum_partials(const double *part, int nb) {
-    __shared__ double shp[16];
-    __shared__ double res;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-    double s = 0.0;
-    for (int i = threadIdx.x; i < nb; i += blockDim.x) s += part[i];
-    s = wave_sum(s);
+// The sums of K arrays of partials (n[k] of array k), each in a fixed order that K does not change; every thread of the
+// block gets the results. The loads of SUM_AHEAD turns of every array are in flight together: with an array and a turn at
+// a time, each waiting for its own load, the PCG update took 29.2 us instead of 25.2 at 2048^2, the matrix-vector product
+// 13.4 instead of 11.8 at 1024^2 and the pre-smoother with the update 20.8 instead of 19.3.
+#define SUM_AHEAD 4
+template <int K>
+__device__ inline void sum_partials(const double *const (&part)[K], const int (&n)[K], double (&out)[K]) {
+    __shared__ double shp[K][16];
+    __shared__ double res[K];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6, step = blockDim.x;
+    int most = 0;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        out[k] = 0.0;
+        most = n[k] > most ? n[k] : most;
+    }
+    for (int i = threadIdx.x; i < most; i += SUM_AHEAD * step) {
+        double v[K][SUM_AHEAD];
+#pragma unroll
+        for (int k = 0; k < K; k++)
+#pragma unroll
+            for (int j = 0; j < SUM_AHEAD; j++) v[k][j] = i + j * step < n[k] ? part[k][i + j * step] : 0.0;
+#pragma unroll
+        for (int j = 0; j < SUM_AHEAD; j++)
+#pragma unroll
+            for (int k = 0; k < K; k++) out[k] += v[k][j];
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) out[k] = wave_sum(out[k]);
     __syncthreads();
-    if (lane == 0) shp[wid] = s;
+    if (lane == 0)
+#pragma unroll
+        for (int k = 0; k < K; k++) shp[k][wid] = out[k];
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < K) {
         double t = 0.0;
-        for (int i = 0; i < nw; i++) t += shp[i];
-        res = t;
+        for (int i = 0; i < nw; i++) t += shp[threadIdx.x][i];
+        res[threadIdx.x] = t;
     }
     __syncthreads();
-    return res;
+#pragma unroll
+    for (int k = 0; k < K; k++) out[k] = res[k];
+}
+
+__device__ inline double sum_partials(const double *part, int nb) {
+    const double *const p[1] = {part};
+    const int n[1] = {nb};
+    double s[1];
+    sum_partials<1>(p, n, s);
+    return s[0];
 }
 
 inline int ilog2(long n) {

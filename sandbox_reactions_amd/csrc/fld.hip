@@ -287,12 +287,23 @@ __global__ void __launch_bounds__(NT) k_slot_head(L0 a, const double *__restrict
     *cout = c;
 }
 
+// alpha = r.z / p.q from the partials
+__device__ inline double alpha_of(const double *dots_cur, int nbd, const double *pq_part, int nbq) {
+    const double *const p[2] = {dots_cur, pq_part};
+    const int n[2] = {nbd, nbq};
+    double s[2];
+    sum_partials<2>(p, n, s);
+    return s[1] != 0.0 ? s[0] / s[1] : 0.0;
+}
+
 // beta from the preconditioner's partials: (r.z_new - r.z_old) / (r.z of the previous iteration), 0 on a restart
 __device__ inline float beta_of(const double *dots_cur, const double *dots_prev, int nbd, int nbp, int restart) {
     if (restart) return 0.0f;
-    const double rzn = sum_partials(dots_cur, nbd), rzo = sum_partials(dots_cur + nbd, nbd);
-    const double rzp = sum_partials(dots_prev, nbp);
-    return rzp != 0.0 ? (float)((rzn - rzo) / rzp) : 0.0f;
+    const double *const p[3] = {dots_cur, dots_cur + nbd, dots_prev};
+    const int n[3] = {nbd, nbd, nbp};
+    double rz[3];
+    sum_partials<3>(p, n, rz);
+    return rz[2] != 0.0 ? (float)((rz[0] - rz[1]) / rz[2]) : 0.0f;
 }
 
 // p = z + beta p_old (into p_new), q = A p_new in FP32; partials of p.q. Blocks of 256 columns x `rows` rows; each
@@ -359,8 +370,7 @@ __global__ void __launch_bounds__(NT) k_update(int n, const float *__restrict__ 
                                                int nbd, const double *pq_part, int nbq, double *part,
                                                const int *gate) {
     if (gated_off(gate)) return;
-    const double rz = sum_partials(dots_cur, nbd), pq = sum_partials(pq_part, nbq);
-    const double alpha = pq != 0.0 ? rz / pq : 0.0;
+    const double alpha = alpha_of(dots_cur, nbd, pq_part, nbq);
     const float af = (float)alpha;
     double v[1] = {0.0};
     for (int base = blockIdx.x * NT * UNROLL + threadIdx.x; base < n; base += gridDim.x * NT * UNROLL) {
@@ -624,8 +634,7 @@ __global__ void __launch_bounds__(NT) k_pre_upd(Lv L, PendingUpdate U, float *__
     using RG = Region<TX, TY, HW>;
     __shared__ RG R;
     __shared__ float own_in[TX * TY];
-    const double rz = sum_partials(U.dots_cur, U.nbd), pq = sum_partials(U.pq, U.nbq);
-    const double alpha = pq != 0.0 ? rz / pq : 0.0;
+    const double alpha = alpha_of(U.dots_cur, U.nbd, U.pq, U.nbq);
     const float af = (float)alpha;
     const int tile = xcd_tile();
     const int x0 = (tile % gridDim.x) * TX, y0 = (tile / gridDim.x) * TY;
