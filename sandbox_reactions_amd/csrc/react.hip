@@ -13,6 +13,7 @@
 
 #include "common.hpp"
 #include "react.hpp"
+#include "react_solve.hpp"
 
 namespace sr {
 
@@ -73,8 +74,6 @@ void react_build(const sr_react_params *p, const sr_physics &ph, ReactDev *out) 
     out->P = *p;
     for (int r = 0; r < p->n_records; r++) {
         const sr_react_record &c = p->rec[r];
-        for (int k = 0; k < c.n_out; k++) out->nu[r][c.out_species[k]] += c.out_share[k];
-        for (int k = 0; k < c.n_in; k++) out->nu[r][c.in_species[k]] -= c.in_share[k];
         // rates.rs:62-71: log-spaced nodes from T_thr over the span; a record of the same law as an earlier one reads its
         out->f_of[r] = -1;
         if (c.n_terms == 0) continue;
@@ -92,35 +91,7 @@ void react_build(const sr_react_params *p, const sr_physics &ph, ReactDev *out) 
             out->ln_f[out->f_of[r]][i] =
                 std::log(f_sum(c, c.t_thr * std::exp(std::log(2.5) * (double)i / (double)(REACT_TABLE - 1))));
     }
-    // the linear system's entries, items and elimination pattern
-    for (int r = 0; r < p->n_records; r++) {
-        out->ent0[r] = out->entries;
-        out->slot[r] = out->slots;
-        if (r == p->nfe) continue;
-        out->entries += p->rec[r].n_in;
-        out->slots++;
-    }
-    out->ent0[p->n_records] = out->entries;
-    unsigned reach[NS];  // the columns a row can hold a value in
-    for (int i = 0; i < NS; i++) {
-        reach[i] = 1u << i;
-        for (int j = 0; j < NS; j++) {
-            const int first = out->items;
-            for (int r = 0; r < p->n_records; r++) {
-                if (r == p->nfe || out->nu[r][i] == 0.0) continue;
-                for (int k = 0; k < p->rec[r].n_in; k++)
-                    if (p->rec[r].in_species[k] == j)
-                        out->item[out->items++] = {out->nu[r][i], out->ent0[r] + k, 0};
-            }
-            if (out->items == first) continue;
-            out->item[out->items - 1].last = 1;
-            out->row[i] |= 1u << j;
-            reach[i] |= 1u << j;
-        }
-        for (int j = 0; j < i; j++)
-            if (reach[i] >> j & 1) reach[i] |= reach[j] >> j << j;
-        out->row[i] |= (reach[i] & ((1u << i) - 1)) << 16;
-    }
+    react_shape(out);
     out->sigma_vac = ph.sigma_vac;
     out->t_floor = ph.t_floor;
     const double k[2][2] = {{ph.k1e, ph.k2e}, {ph.k1n, ph.k2n}};
@@ -145,17 +116,6 @@ __device__ inline void comp(const double *x, double *mu, double *y_e) {
     *mu = 1.0 / im;
     *y_e = ye;
 }
-
-// The tables and the threads' private arrays in LDS: the cold pairs' ln u, f's tables, then per thread a value by species
-// (x while the rates are formed, dX after a solve), omega by record and the derivatives by entry. A species or record
-// index is the wave's own but not the compiler's, so such an array in registers would go to scratch memory (as the whole
-// pass's did: 587 us a pass at 512^2, 105 now). A thread's element k lies NT values from its element
-// k - 1: no bank conflicts. NT = 256 threads share the tables, so that two blocks (two waves a SIMD) fit a CU; with so many
-// inputs that they would not (the shipped records: 78 KB), 64.
-struct Lds {
-    const double *cold, *ln_f;
-    double *v, *omega, *grad;  // the thread's own: element k at [k * NT]
-};
 
 // u(x) of one pair from its FP64 table: linear in (ln x, ln u), the K1 x^2 power law below the first node
 __device__ inline double cold_u_d(const ReactDev &D, const double *lnu, double x) {
@@ -248,98 +208,6 @@ __device__ double nfe_exact(const ReactDev &D, double sigma, double *x, double d
     x[fe] -= dm;
     x[n] += dm;
     return dm;
-}
-
-// (I - h J) dX = h S, Gaussian elimination with partial pivoting, the last of equal pivots (react.rs:515-560): the form
-// for a system that needs a row exchange, its matrix in scratch memory
-template <int NT>
-__device__ __noinline__ void solve_pivoted(const ReactDev &D, const Lds &M, const double *s, double h, double *dx) {
-    double a[NS][NS + 1];
-    int q = 0;
-    for (int i = 0; i < NS; i++) {
-        for (int j = 0; j < NS; j++) {
-            a[i][j] = i == j ? 1.0 : 0.0;
-            if (D.row[i] >> j & 1) do {
-                    a[i][j] -= h * D.item[q].nu * M.grad[D.item[q].e * NT];
-                } while (!D.item[q++].last);
-        }
-        a[i][NS] = h * s[i];
-    }
-    for (int col = 0; col < NS; col++) {
-        int piv = col;
-        for (int p = col + 1; p < NS; p++)
-            if (fabs(a[p][col]) >= fabs(a[piv][col])) piv = p;
-        if (piv != col)
-            for (int j = 0; j <= NS; j++) {
-                const double t = a[col][j];
-                a[col][j] = a[piv][j];
-                a[piv][j] = t;
-            }
-        const double d = a[col][col];
-        if (d == 0.0) continue;
-        for (int row = col + 1; row < NS; row++) {
-            const double f = a[row][col] / d;
-            if (f != 0.0)
-                for (int j = col; j <= NS; j++) a[row][j] -= f * a[col][j];
-        }
-    }
-    for (int i = NS - 1; i >= 0; i--) {
-        double v = a[i][NS];
-        for (int j = i + 1; j < NS; j++) v -= a[i][j] * dx[j];
-        dx[i] = a[i][i] == 0.0 ? 0.0 : v / a[i][i];
-    }
-}
-
-// The same system by rows in registers: each row is built and reduced by the rows above it (the columns it can hold a
-// value in, `lower`), the same operations in the same order on every element as by columns. Where the pivoted form would
-// exchange rows (an element at least as large as its pivot) the pivoted form solves the system instead; the consumed
-// species' diagonal 1 + h sum of its losses exceeds what any product's row holds, so no physical system is. NA: the
-// species to solve for (9 where the last, the neutrons, has no items, as with N_Fe in closed form: dX = 0).
-template <int NA, int NT>
-__device__ inline void solve(const ReactDev &D, const Lds &M, const double (&s)[NS], double h, double (&dx)[NS]) {
-    double u[NA][NA];
-    bool exchange = false;
-    int q = 0;
-#pragma unroll
-    for (int i = 0; i < NA; i++) {
-        double b = h * s[i];
-        const unsigned shape = D.row[i];
-#pragma unroll
-        for (int j = 0; j < NA; j++) {
-            u[i][j] = i == j ? 1.0 : 0.0;
-            if (shape >> j & 1) do {
-                    u[i][j] -= h * D.item[q].nu * M.grad[D.item[q].e * NT];
-                } while (!D.item[q++].last);
-        }
-#pragma unroll
-        for (int col = 0; col < i; col++) {
-            if (!(shape >> (16 + col) & 1)) continue;
-            const double d = u[col][col];
-            exchange |= fabs(u[i][col]) >= fabs(d);
-            const double f = u[i][col] / d;
-#pragma unroll
-            for (int j = col + 1; j < NS; j++) u[i][j] -= f * u[col][j];
-            b -= f * dx[col];
-        }
-        dx[i] = b;
-    }
-#pragma unroll
-    for (int i = NA - 1; i >= 0; i--) {
-        double v = dx[i];
-#pragma unroll
-        for (int j = i + 1; j < NA; j++) v -= u[i][j] * dx[j];
-        exchange |= u[i][i] == 0.0;
-        dx[i] = v / u[i][i];
-    }
-#pragma unroll
-    for (int i = NA; i < NS; i++) dx[i] = 0.0;
-    if (exchange) {
-        double sv[NS], dv[NS];
-        for (int i = 0; i < NS; i++) sv[i] = s[i];
-        solve_pivoted<NT>(D, M, sv, h, dv);
-#pragma unroll
-        for (int i = 0; i < NS; i++) dx[i] = dv[i];
-    }
 }
 
 struct CellOut {

@@ -5,40 +5,11 @@
 #include "../../include/sr_hip.h"
 #include "cold.hpp"
 #include "hydro.hpp"
+#include "react_dev.hpp"
 
 namespace sr {
 
-#define REACT_NS 10
-#define REACT_TABLE 256
-#define REACT_ITEMS (SR_REACT_RECORDS * 4 * 8)  // a record's inputs times the species it changes, at most
-
-// Everything the pass reads besides the state, in device memory: the records and constants as given, each record's
-// nu (outputs' shares minus inputs'), its ln f table, Sigma_vac, T_floor and the cold energy's tables in FP64 (the
-// electrons' and the neutrons' ln u at the nodes, a pair's flag 0 when it is off; ln x_min and the node spacing in
-// ln x), so that T = mu (e - eps_cold) carries no f32 rounding into the rates
-struct ReactDev {
-    sr_react_params P;
-    double nu[SR_REACT_RECORDS][REACT_NS];
-    double ln_f[SR_REACT_RECORDS][REACT_TABLE];
-    double sigma_vac, t_floor;
-    double cold_lnu[2][COLD_POINTS];
-    int cold_pair[2];
-    double cold_ln_min, cold_step;
-    // The linear system's shape, built on the host from the records. Entry e is a record's derivative by one of its inputs
-    // (the records in order, N_Fe left out, ent0[r] the first of record r). The matrix's items in row order, a position's
-    // together, its last flagged: entry e times nu. Row i: bits 0..9 the columns that have items, bits
-    // 16..25 the columns j < i that can be nonzero when the row is eliminated without exchanges.
-    struct Item {
-        double nu;
-        int e, last;
-    };
-    int entries, items, ent0[SR_REACT_RECORDS + 1], slots, slot[SR_REACT_RECORDS];  // slot: a record's but N_Fe's
-    unsigned row[REACT_NS];
-    Item item[REACT_ITEMS];
-    // f's tables: record r reads table f_of[r] (records of the same law share one), tables in all; ln T_thr per record
-    int f_of[SR_REACT_RECORDS], tables;
-    double ln_thr[SR_REACT_RECORDS];
-};
+static_assert(REACT_COLD == COLD_POINTS, "the cold energy's nodes");
 
 // the host's checks of the records and the device copy's build (tables in FP64 on the host) for the world's physics
 int react_check(const sr_react_params *p);
