@@ -159,7 +159,8 @@ int sr_fft2(float *data_dev, int nx, int ny, int inverse, void *stream);
 int sr_fft2_noalloc(float *data_dev, int nx, int ny, int inverse, void *stream);
 
 /* Convolution::new + Gravity::new (step/fft.rs:136-182, step/grav.rs:133-200; twin reference/grav.rs:99-121):
- * a gravity solver for a w x h box, its kernel's spectrum built once (f64 on the host, stored f32). */
+ * a gravity solver for a w x h box, its kernel's spectrum built once (f64 on the host, stored f32). Padded axes go up to
+ * max_padded (0: 4096) and at most 16384 along x and 8192 along y (SR_ERR_BOX_AXIS past either). */
 int sr_gravity_create(int w, int h, double G, double dx, double sigma_vac, int max_padded, sr_gravity **out);
 /* Gravity::field (reference/grav.rs:115-121): phi on the box grown by one ring ((w+2) x (h+2)), and g = -grad phi
  * over the box (gx, gy may be NULL). sigma_dev is the w x h surface density; cells below sigma_vac are no source. */

@@ -186,8 +186,9 @@ __global__ void k_rows_r2c(const TIn *__restrict__ sigma, int w, int h, TIn sigm
 // memory through the registers. At 2048^2 (py 4096) 54 us, 154 with
 // radix-4 passes in LDS; the row transforms 31 us each way, 61 and 50.
 template <int LOGN>
-__global__ void __launch_bounds__(256) k_columns(const float2 *__restrict__ spec, int ld, int h, int ncols, const float *__restrict__ khat,
-                          const float2 *__restrict__ tw, int tw_stride, float2 *__restrict__ out, int ldo) {
+__global__ void __launch_bounds__(Fft<LOGN>::T > 256 ? Fft<LOGN>::T : 256)
+    k_columns(const float2 *__restrict__ spec, int ld, int h, int ncols, const float *__restrict__ khat,
+              const float2 *__restrict__ tw, int tw_stride, float2 *__restrict__ out, int ldo) {
     using F = Fft<LOGN>;
     extern __shared__ float2 lds[];
     constexpr int N = F::N;
@@ -312,6 +313,8 @@ __global__ void __launch_bounds__(256) k_c2c_cols(float2 *data, int nx, int ny, 
 
 // -------------------------------------------------------------------------------------------------------- host
 
+// the longest transform that one block's registers and LDS carry (512 threads, 70 KB)
+#define FFT_MOST 8192
 static const double SELF_CELL = 3.525494348078172; // 4 ln(1 + sqrt 2): the potential of a unit square at its centre
 
 // In-place f64 radix-2 transform on the host (the kernel's spectrum is built once per padded size in f64).
@@ -431,8 +434,9 @@ int Gravity::init(int w_, int h_, double G_, double dx_, double sigma_vac_, int 
     sigma_vac = sigma_vac_;
     SR_TRY(padded_size(w, max_padded, &px));
     SR_TRY(padded_size(h, max_padded, &py));
-    if ((size_t)py * 2 * sizeof(float2) > (size_t)max_lds_bytes())
-        return fail(SR_ERR_BOX_AXIS, "a padded column of " + std::to_string(py) + " does not fit the LDS");
+    if (py > FFT_MOST) return fail(SR_ERR_BOX_AXIS, "a padded column of " + std::to_string(py) + " does not fit the LDS");
+    if (px > 2 * FFT_MOST)
+        return fail(SR_ERR_BOX_AXIS, "a padded row of " + std::to_string(px) + " does not fit the LDS");
     nmax = std::max(px, py);
     std::vector<float2> t(nmax);
     for (int i = 0; i < nmax; i++) {
@@ -451,7 +455,7 @@ int Gravity::init(int w_, int h_, double G_, double dx_, double sigma_vac_, int 
     return SR_OK;
 }
 
-// f with the transform's log2 length as a compile-time constant
+// f with the transform's log2 length as a compile-time constant: 16 (half a padded row of 32) to FFT_MOST points
 template <typename Fn> static int fft_length(int logn, Fn f) {
     switch (logn) {
     case 4: return f(std::integral_constant<int, 4>());
@@ -463,6 +467,7 @@ template <typename Fn> static int fft_length(int logn, Fn f) {
     case 10: return f(std::integral_constant<int, 10>());
     case 11: return f(std::integral_constant<int, 11>());
     case 12: return f(std::integral_constant<int, 12>());
+    case 13: return f(std::integral_constant<int, 13>());
     default: return fail(SR_ERR_BOX_AXIS, "a transform of 2^" + std::to_string(logn) + " points");
     }
 }

@@ -93,13 +93,17 @@ def test_refusals(gpu_lib):
     with pytest.raises(gpu_lib.SrError) as e:
         gpu_lib.Gravity(3000, 64, max_padded=4096)
     assert e.value.kind == "BoxAxis"
+    for w, h in ((40, 4100), (8200, 40)):  # a column past 8192 points, a row past 16384
+        with pytest.raises(gpu_lib.SrError) as e:
+            gpu_lib.Gravity(w, h, max_padded=32768)
+        assert e.value.kind == "BoxAxis"
 
 
-# one box per transform length of rows and columns (16 to 4096 points), odd sides among them, with rows left over in the
-# last block, and a box whose padded rows are twice the default cap
-@pytest.mark.parametrize("w,h,cap", [(3, 5, 4096), (16, 33, 4096), (33, 16, 4096), (65, 70, 4096), (130, 140, 4096),
-                                     (257, 300, 4096), (601, 520, 4096), (1030, 1100, 4096), (2048, 37, 4096),
-                                     (2100, 40, 8192)])
+# one box per transform length of rows (16 to 8192 points) and columns (32 to 8192), odd sides among them, with rows left
+# over in the last block, the longest ones past the default cap
+@pytest.mark.parametrize("w,h,cap", [(3, 5, 4096), (16, 33, 4096), (20, 25, 4096), (33, 16, 4096), (65, 70, 4096),
+                                     (130, 140, 4096), (257, 300, 4096), (601, 520, 4096), (1030, 1100, 4096),
+                                     (2048, 37, 4096), (2100, 40, 8192), (40, 2100, 8192), (4100, 40, 16384)])
 def test_gravity_field_at_every_transform_length(gpu_lib, w, h, cap):
     import torch
     print(f"gravity {w}x{h}", flush=True)
