@@ -483,20 +483,33 @@ static bool react_neutrons(const ReactDev &h) {
     return any != 0;
 }
 
+#define REACT_LDS (78 * 1024)  // a block of 256 threads: two blocks, each with 2 KB of partial sums, fill a CU's 160 KB
+static int react_lds(int nt, int tables, int slots, int entries) {
+    return (int)sizeof(double) * (2 * COLD_POINTS + tables * REACT_TABLE + nt * (NS + slots + entries));
+}
+
 ReactLaunch react_plan(const ReactDev &h) {
-    auto lds = [&](int nt) {
-        return (int)sizeof(double) * (2 * COLD_POINTS + h.tables * REACT_TABLE + nt * (NS + h.slots + h.entries));
-    };
-    const int nt = lds(256) <= 78 * 1024 ? 256 : REACT_NT_LEAST;  // and 2 KB of partial sums
-    return {nt, lds(nt), react_neutrons(h)};
+    const bool fits = react_lds(256, h.tables, h.slots, h.entries) <= REACT_LDS;
+    const int nt = fits ? 256 : REACT_NT_LEAST;
+    return {nt, react_lds(nt, h.tables, h.slots, h.entries), react_neutrons(h)};
+}
+
+static auto react_kernel(const ReactLaunch &plan) {
+    return plan.nt == 256 ? (plan.neutrons ? k_react<NS, 256> : k_react<NS - 1, 256>)
+                          : (plan.neutrons ? k_react<NS, REACT_NT_LEAST> : k_react<NS - 1, REACT_NT_LEAST>);
+}
+
+int react_prepare(const ReactLaunch &plan) {
+    // a kernel's limit is the process's, not the world's: always the most that any records take (87 KB with 64 threads)
+    const int most = plan.nt == 256 ? REACT_LDS : react_lds(plan.nt, NR, NR, 4 * NR);
+    SR_HIP(hipFuncSetAttribute((const void *)react_kernel(plan), hipFuncAttributeMaxDynamicSharedMemorySize, most));
+    return SR_OK;
 }
 
 int react_launch(const ReactDev *D, const ReactLaunch &plan, const HydroState &st, int n, double dt, const double *scal,
                  double *nuclear, double *lost, double *snu, double *psum, double *pmax, int *nblocks, hipStream_t s) {
     const int nb = plan.blocks(n);
-    auto kernel = plan.nt == 256 ? (plan.neutrons ? k_react<NS, 256> : k_react<NS - 1, 256>)
-                                 : (plan.neutrons ? k_react<NS, REACT_NT_LEAST> : k_react<NS - 1, REACT_NT_LEAST>);
-    SR_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, plan.lds));
+    auto kernel = react_kernel(plan);
     hipLaunchKernelGGL(kernel, dim3(nb), dim3(plan.nt), plan.lds, s, D, st, n, dt, scal, nuclear, lost, snu, psum, pmax);
     if (nblocks) *nblocks = nb;
     SR_HIP(hipGetLastError());

@@ -27,6 +27,8 @@ struct ReactLaunch {
 };
 constexpr int REACT_NT_LEAST = 64;
 ReactLaunch react_plan(const ReactDev &h);
+// once before a plan's first launch
+int react_prepare(const ReactLaunch &plan);
 int react_launch(const ReactDev *D, const ReactLaunch &plan, const HydroState &st, int n, double dt, const double *scal,
                  double *nuclear, double *lost, double *snu, double *psum, double *pmax, int *nblocks, hipStream_t s);
 

@@ -1083,9 +1083,11 @@ extern "C" int sr_set_reactions(sr_world *wd, const sr_react_params *p) {
     ReactDev *h = new ReactDev;
     react_build(p, wd->ph, h);
     const ReactLaunch plan = react_plan(*h);
+    const int prepared = react_prepare(plan);
     const hipError_t e = hipMemcpyAsync(wd->react_dev_mem, h, sizeof(ReactDev), hipMemcpyHostToDevice, wd->s);
     const hipError_t e2 = e == hipSuccess ? hipStreamSynchronize(wd->s) : e;
     delete h;
+    SR_TRY(prepared);
     if (e2 != hipSuccess) return fail(SR_ERR_DEVICE, std::string("sr_set_reactions: ") + hipGetErrorString(e2));
     wd->react = wd->react_dev_mem;
     wd->react_plan = plan;

@@ -5,7 +5,7 @@
 #include <cstring>
 #include <random>
 
-#include "../sandbox_reactions_amd/csrc/react_solve.hpp"
+#include "../../sandbox_reactions_amd/csrc/react_solve.hpp"
 
 using namespace sr;
 

@@ -361,3 +361,34 @@ def test_general_records_are_the_oracles(gpu_lib, kind):
     assert (np.abs(got[3] - o[3]) <= 1e-6 * np.maximum(np.abs(o[3]), 1e-30)).all()
     nuc, _, _ = r.world.read_react_planes()
     assert np.abs(nuc - onuc.reshape(nuc.shape)).max() <= 1e-9 * np.abs(onuc).max()
+
+
+def test_worlds_of_different_records_step_side_by_side(gpu_lib):
+    """Four worlds with one to sixteen records, stepped by four host threads: each the bits that it reaches alone."""
+    sr = gpu_lib
+    print("ensemble of different records", flush=True)
+
+    def make(k):
+        p = react.params(only=[])
+        p.n_records = (1, 5, 16, 3)[k]
+        for r in range(p.n_records):
+            plain_record(p.rec[r], [(sp, 1.0 / (1 + k), 1.0) for sp in ("H", "He", "C", "O")[:1 + k]], [("Ne", 1.0)],
+                         0.2 * (r + 1))
+        w = sr.World(32, 32, gravity=False, hydro=True, heat=False)
+        w.set_reactions(p)
+        planes = np.zeros((14, 32, 32), np.float32)
+        planes[0] = 1.0 + 0.1 * k
+        planes[3] = 100.0
+        planes[4:8] = 0.25
+        w.upload(planes)
+        return w
+
+    alone = []
+    for k in range(4):
+        w = make(k)
+        w.run(5)
+        alone.append(w.readback())
+    together = [make(k) for k in range(4)]
+    sr.ensemble_run(together, 5, threads=4)
+    for a, w in zip(alone, together):
+        assert np.array_equal(a.view(np.uint32), w.readback().view(np.uint32))
