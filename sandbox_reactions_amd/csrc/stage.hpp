@@ -13,7 +13,8 @@ namespace sr {
 // kept from the first large transfer until release().
 class HostStage {
   public:
-    // Queued on s: when it returns src may be changed, the device's copy is ordered on s
+    // Queued on s: pageable memory may be changed when it returns (pinned memory once s's work is done), the device's copy
+    // is ordered on s
     int to_device(void *dst, const void *src, size_t bytes, hipStream_t s);
     // Done when it returns (s's work before it too)
     int to_host(void *dst, const void *src, size_t bytes, hipStream_t s);

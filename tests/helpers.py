@@ -1,7 +1,14 @@
 """Shared test helpers: one set of constants for the oracle and the HIP library, comparisons."""
+import os
+import subprocess
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 
 import oracle
+
+HOST = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host")
+CSRC = os.path.join(os.path.dirname(HOST), os.pardir, "sandbox_reactions_amd", "csrc")
 
 # the reference's physics.json values the path reads (assets/physics.json)
 REFERENCE = dict(gamma=2.0, G=1.0, dx=1.0, sigma_vac=1e-6, sigma_floor=1e-8, t_floor=0.05, cfl=0.4, eta_g=0.3,
@@ -51,3 +58,28 @@ def mass_radius(sigma, vac=1e-6, fraction=0.9):
     k = int(np.searchsorted(c, fraction * mass))
     below, rp = (c[k - 1], r[k - 1]) if k > 0 else (0.0, 0.0)
     return rp + (r[k] - rp) * (fraction * mass - below) / pm[k], mass
+
+
+def host_program(tmp_path, name, sources):
+    """tests/host/NAME.cpp with the library's host code of `sources` (no device code) over the stand-in for the HIP
+    runtime, tests/host/fake_hip.hpp."""
+    from sandbox_reactions_amd.build import HIPCC
+
+    def compile(src):
+        obj = str(tmp_path / (os.path.basename(src) + ".o"))
+        subprocess.run([HIPCC, "-x", "hip", "--offload-arch=gfx950", "--cuda-host-only", "-O1", "-std=c++17", "-w", "-c",
+                        src, "-o", obj], check=True)
+        return obj
+
+    with ThreadPoolExecutor(max_workers=8) as ex:
+        objs = list(ex.map(compile, [os.path.join(HOST, name + ".cpp")] + [os.path.join(CSRC, f) for f in sources]))
+    exe = str(tmp_path / name)
+    # the device code's sections are not there: nothing reads them
+    subprocess.run([HIPCC, "-o", exe] + objs + ["-lpthread", "-Wl,--unresolved-symbols=ignore-all"], check=True)
+    return exe
+
+
+def run_host(*command):
+    r = subprocess.run(command, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+    return r.stdout
