@@ -1,8 +1,7 @@
 // Host transfers through pinned chunks. The runtime copies pageable memory through one staging buffer on the calling
 // thread: 26 GB/s up and 10 GB/s down (into fresh pages) at 235 MB. Here a few threads copy chunks between the caller's
 // memory and pinned slots while the copies of the slots before are on the bus: 36 GB/s both ways. Four threads of two
-// 2 MiB slots: 1 MiB slots take 18 % longer; below 8 MiB the threads and the pinned memory (0.4 ms once) cost what they
-// give (3.7 MB: 0.24 ms either way).
+// 2 MiB slots: 1 MiB slots take 18 % longer; the pinned memory costs 0.4 ms once.
 #include <algorithm>
 #include <cstring>
 #include <system_error>
@@ -112,7 +111,7 @@ template <class F> int HostStage::spread(size_t bytes, F part) {
 }
 
 int HostStage::to_device(void *dst, const void *src, size_t bytes, hipStream_t s) {
-    if (bytes < STAGE_LEAST || !pageable(src) || !ready()) {
+    if (bytes < STAGE_LEAST_UP || !pageable(src) || !ready()) {
         SR_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
         return SR_OK;
     }
@@ -122,7 +121,7 @@ int HostStage::to_device(void *dst, const void *src, size_t bytes, hipStream_t s
 }
 
 int HostStage::to_host(void *dst, const void *src, size_t bytes, hipStream_t s) {
-    if (bytes < STAGE_LEAST || !pageable(dst) || !ready()) {
+    if (bytes < STAGE_LEAST_DOWN || !pageable(dst) || !ready()) {
         SR_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
         SR_HIP(hipStreamSynchronize(s));
         return SR_OK;

@@ -7,7 +7,11 @@ namespace sr {
 #define STAGE_THREADS 4
 #define STAGE_SLOTS 2               // per thread: one is copied by the host while the other is on the bus
 #define STAGE_CHUNK (2u << 20)      // bytes of one slot
-#define STAGE_LEAST (8u << 20)      // transfers below this stay with the runtime's own copy
+// Transfers below these stay with the runtime's own copy. Up, by the runtime against the slots: 0.49 / 0.52 ms at 14.7 MB,
+// 0.73 / 0.72 at 22.9, 1.10 / 0.97 at 33.0, 8.5 / 6.3 at 235. Down: 0.29 / 0.26 at 3.7 (within its spread), 0.57 / 0.36 at
+// 8.6, 1.39 / 0.68 at 22.9, 13.5 / 5.9 at 235.
+#define STAGE_LEAST_UP (24u << 20)
+#define STAGE_LEAST_DOWN (8u << 20)
 
 // Not for concurrent use (a world's transfers are its caller's, one at a time). The pinned memory and the events are
 // kept from the first large transfer until release().

@@ -25,7 +25,8 @@ static bool round_trips(char *a, size_t most, hipStream_t s) {
     HostStage stage;
     std::vector<char> dev(most);
     bool ok = true;
-    for (size_t n : {(size_t)1000, (size_t)STAGE_LEAST - 1, (size_t)STAGE_LEAST, (size_t)STAGE_LEAST + 4321, most}) {
+    for (size_t n : {(size_t)1000, (size_t)STAGE_LEAST_DOWN - 1, (size_t)STAGE_LEAST_DOWN, (size_t)STAGE_LEAST_UP - 1,
+                     (size_t)STAGE_LEAST_UP + 4321, most}) {
         for (size_t i = 0; i < n; i++) a[i] = (char)(i * 2654435761u >> 24);
         starting = no_threads;
         ok &= stage.to_device(dev.data(), a, n, s) == SR_OK;
@@ -48,11 +49,11 @@ int main(int, char **argv) {
     bool ok = false;
     if (name == "pageable") {
         std::vector<char> a(most);
-        ok = round_trips(a.data(), most, s) && fake::largest_copy == STAGE_LEAST - 1;
+        ok = round_trips(a.data(), most, s) && fake::largest_copy == STAGE_LEAST_UP - 1;  // 24 MiB up
     } else if (name == "pinned") {  // in one copy
         void *a = nullptr;
         (void)hipHostMalloc(&a, most);
-        ok = round_trips((char *)a, most, s) && fake::copies == 10 && fake::largest_copy == most;
+        ok = round_trips((char *)a, most, s) && fake::copies == 12 && fake::largest_copy == most;
     } else if (name == "threads") {  // none to be had: the caller's own
         std::vector<char> a(most);
         no_threads = true;

@@ -1,6 +1,6 @@
-"""The planes' way in and out of a world: the same bits back, below and above the size from which several host threads
-copy through pinned chunks (8 MiB: 384^2's 14 planes are 8.26 MB), at sizes that end inside a chunk, and from several
-threads at once, each with its own world."""
+"""The planes' way in and out of a world: the same bits back, below and above the sizes from which several host threads
+copy through pinned chunks (8 MiB down, 24 MiB up: 14 planes are 8.26 MB at 384^2, 24.7 at 664^2 and 25.3 at 672^2), at
+sizes that end inside a chunk, and from several threads at once, each with its own world."""
 import threading
 
 import numpy as np
@@ -8,7 +8,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [(8, 8), (384, 384), (392, 392), (1024, 200), (1304, 728)]
+SIZES = [(8, 8), (384, 384), (392, 392), (1024, 200), (664, 664), (672, 672), (1304, 728)]
 
 
 def planes(w, h, seed):
