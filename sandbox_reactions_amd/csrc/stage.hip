@@ -11,12 +11,17 @@
 
 namespace sr {
 
-bool HostStage::ready() {
+// on the stream's device, which need not be the calling thread's current one
+bool HostStage::ready(hipStream_t s) {
     if (buf) return true;
     if (refused) return false;
     const int n = STAGE_THREADS * STAGE_SLOTS;
-    bool ok = hipHostMalloc(&buf, (size_t)STAGE_CHUNK * n) == hipSuccess;
+    int current = 0;
+    bool ok = hipGetDevice(&current) == hipSuccess && hipStreamGetDevice(s, &device) == hipSuccess &&
+              hipSetDevice(device) == hipSuccess;
+    ok = ok && hipHostMalloc(&buf, (size_t)STAGE_CHUNK * n) == hipSuccess;
     for (int i = 0; ok && i < n; i++) ok = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) == hipSuccess;
+    (void)hipSetDevice(current);
     if (!ok) {
         (void)hipGetLastError();
         release();
@@ -87,8 +92,6 @@ hipError_t HostStage::chunks_down(int k, int threads, const char *dev, char *hos
 // or no memory for one) leaves its share to this one
 template <class F> int HostStage::spread(size_t bytes, F part) {
     const int threads = (int)std::min<size_t>(STAGE_THREADS, (bytes + STAGE_CHUNK - 1) / STAGE_CHUNK);
-    int device = 0;
-    SR_HIP(hipGetDevice(&device));
     hipError_t err[STAGE_THREADS] = {};
     std::thread th[STAGE_THREADS];
     for (int k = 1; k < threads; k++) {
@@ -111,7 +114,7 @@ template <class F> int HostStage::spread(size_t bytes, F part) {
 }
 
 int HostStage::to_device(void *dst, const void *src, size_t bytes, hipStream_t s) {
-    if (bytes < STAGE_LEAST_UP || !pageable(src) || !ready()) {
+    if (bytes < STAGE_LEAST_UP || !pageable(src) || !ready(s)) {
         SR_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
         return SR_OK;
     }
@@ -121,7 +124,7 @@ int HostStage::to_device(void *dst, const void *src, size_t bytes, hipStream_t s
 }
 
 int HostStage::to_host(void *dst, const void *src, size_t bytes, hipStream_t s) {
-    if (bytes < STAGE_LEAST_DOWN || !pageable(dst) || !ready()) {
+    if (bytes < STAGE_LEAST_DOWN || !pageable(dst) || !ready(s)) {
         SR_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
         SR_HIP(hipStreamSynchronize(s));
         return SR_OK;

@@ -13,8 +13,8 @@ namespace sr {
 #define STAGE_LEAST_UP (24u << 20)
 #define STAGE_LEAST_DOWN (8u << 20)
 
-// Not for concurrent use (a world's transfers are its caller's, one at a time). The pinned memory and the events are
-// kept from the first large transfer until release().
+// Not for concurrent use (a world's transfers are its caller's, one at a time, all on one device's streams). The pinned
+// memory and the events are kept from the first large transfer until release().
 class HostStage {
   public:
     // Queued on s: pageable memory may be changed when it returns (pinned memory once s's work is done), the device's copy
@@ -26,11 +26,12 @@ class HostStage {
     void release();
 
   private:
-    bool ready();
+    bool ready(hipStream_t s);
     hipError_t chunks_up(int k, int threads, char *dev, const char *host, size_t bytes, hipStream_t s);
     hipError_t chunks_down(int k, int threads, const char *dev, char *host, size_t bytes, hipStream_t s);
     template <class F> int spread(size_t bytes, F part);
     char *buf = nullptr;
+    int device = 0;  // the stream's, where the events are
     hipEvent_t ev[STAGE_THREADS * STAGE_SLOTS] = {};
     bool refused = false;  // no pinned memory to be had: the runtime's own copies
 };

@@ -10,6 +10,6 @@ def stage(tmp_path_factory):
     return host_program(tmp_path_factory.mktemp("stage"), "stage", ["stage.hip", "util.cpp"])
 
 
-@pytest.mark.parametrize("case", ["pageable", "pinned", "threads"])
+@pytest.mark.parametrize("case", ["pageable", "pinned", "threads", "device"])
 def test_transfers(stage, case):
     run_host(stage, case)
