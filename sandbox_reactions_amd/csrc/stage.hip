@@ -90,7 +90,7 @@ hipError_t HostStage::chunks_down(int k, int threads, const char *dev, char *hos
 
 // part(k, threads) on up to STAGE_THREADS threads, this one among them; a thread that cannot be started (none to be had,
 // or no memory for one) leaves its share to this one
-template <class F> int HostStage::spread(size_t bytes, F part) {
+template <class F> int HostStage::spread(size_t bytes, hipStream_t s, F part) {
     const int threads = (int)std::min<size_t>(STAGE_THREADS, (bytes + STAGE_CHUNK - 1) / STAGE_CHUNK);
     hipError_t err[STAGE_THREADS] = {};
     std::thread th[STAGE_THREADS];
@@ -109,6 +109,8 @@ template <class F> int HostStage::spread(size_t bytes, F part) {
             th[k].join();
         else
             err[k] = part(k, threads);
+    for (int k = 0; k < threads; k++)
+        if (err[k] != hipSuccess) (void)hipStreamSynchronize(s);  // no copy goes on in a slot that the next call takes
     for (int k = 0; k < threads; k++) SR_HIP(err[k]);
     return SR_OK;
 }
@@ -118,7 +120,7 @@ int HostStage::to_device(void *dst, const void *src, size_t bytes, hipStream_t s
         SR_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
         return SR_OK;
     }
-    return spread(bytes, [&](int k, int threads) {
+    return spread(bytes, s, [&](int k, int threads) {
         return chunks_up(k, threads, (char *)dst, (const char *)src, bytes, s);
     });
 }
@@ -129,7 +131,7 @@ int HostStage::to_host(void *dst, const void *src, size_t bytes, hipStream_t s) 
         SR_HIP(hipStreamSynchronize(s));
         return SR_OK;
     }
-    return spread(bytes, [&](int k, int threads) {
+    return spread(bytes, s, [&](int k, int threads) {
         return chunks_down(k, threads, (const char *)src, (char *)dst, bytes, s);
     });
 }

@@ -29,7 +29,7 @@ class HostStage {
     bool ready(hipStream_t s);
     hipError_t chunks_up(int k, int threads, char *dev, const char *host, size_t bytes, hipStream_t s);
     hipError_t chunks_down(int k, int threads, const char *dev, char *host, size_t bytes, hipStream_t s);
-    template <class F> int spread(size_t bytes, F part);
+    template <class F> int spread(size_t bytes, hipStream_t s, F part);
     char *buf = nullptr;
     int device = 0;  // the stream's, where the events are
     hipEvent_t ev[STAGE_THREADS * STAGE_SLOTS] = {};

@@ -595,6 +595,26 @@ extern "C" int sr_world_create(int w, int h, const sr_physics *ph, const sr_swit
     return SR_OK;
 }
 
+// Device memory for the length of a call, in the order of the world's stream: given back however the call ends
+template <typename T> struct CallMem {
+    T *p = nullptr;
+    hipStream_t s;
+    explicit CallMem(hipStream_t stream) : s(stream) {}
+    CallMem(const CallMem &) = delete;
+    CallMem &operator=(const CallMem &) = delete;
+    int get(size_t count) {
+        SR_HIP(hipMallocAsync((void **)&p, sizeof(T) * count, s));
+        return SR_OK;
+    }
+    int give_back() {
+        T *q = p;
+        p = nullptr;
+        if (q) SR_HIP(hipFreeAsync(q, s));
+        return SR_OK;
+    }
+    ~CallMem() { (void)give_back(); }
+};
+
 static int state_ok(sr_world *wd, size_t n) {
     if (!wd) return fail(SR_ERR_ARGUMENT, "null world");
     if (n != SR_COMPONENTS * wd->n)
@@ -634,12 +654,12 @@ static int p89(sr_world *wd, int apply) {
 extern "C" int sr_upload(sr_world *wd, const float *planes, size_t n) {
     SR_TRY(state_ok(wd, n));
     if (!planes) return fail(SR_ERR_ARGUMENT, "sr_upload: null planes");
-    float *tmp = nullptr;
-    SR_HIP(hipMallocAsync((void **)&tmp, sizeof(float) * n, wd->s));
-    SR_TRY(wd->stage.to_device(tmp, planes, sizeof(float) * n, wd->s));
+    CallMem<float> tmp(wd->s);
+    SR_TRY(tmp.get(n));
+    SR_TRY(wd->stage.to_device(tmp.p, planes, sizeof(float) * n, wd->s));
     wd->cur = 0;
-    hipLaunchKernelGGL(k_upload, dim3((wd->n + 255) / 256), dim3(256), 0, wd->s, tmp, wd->st[0], (int)wd->n);
-    SR_HIP(hipFreeAsync(tmp, wd->s));
+    hipLaunchKernelGGL(k_upload, dim3((wd->n + 255) / 256), dim3(256), 0, wd->s, tmp.p, wd->st[0], (int)wd->n);
+    SR_TRY(tmp.give_back());
     hipLaunchKernelGGL(k_scal_reset, dim3(1), dim3(64), 0, wd->s, wd->scal);
     SR_HIP(hipMemsetAsync(wd->escaped, 0, sizeof(double) * 14 * 2 * (wd->w + wd->h), wd->s));
     wd->have_flux = false;
@@ -664,12 +684,11 @@ extern "C" int sr_upload(sr_world *wd, const float *planes, size_t n) {
 extern "C" int sr_readback(sr_world *wd, float *planes, size_t n) {
     SR_TRY(state_ok(wd, n));
     if (!planes) return fail(SR_ERR_ARGUMENT, "sr_readback: null planes");
-    float *tmp = nullptr;
-    SR_HIP(hipMallocAsync((void **)&tmp, sizeof(float) * n, wd->s));
-    hipLaunchKernelGGL(k_readback, dim3((wd->n + 255) / 256), dim3(256), 0, wd->s, wd->st[wd->cur], tmp, (int)wd->n);
-    SR_TRY(wd->stage.to_host(planes, tmp, sizeof(float) * n, wd->s));
-    SR_HIP(hipFreeAsync(tmp, wd->s));
-    return SR_OK;
+    CallMem<float> tmp(wd->s);
+    SR_TRY(tmp.get(n));
+    hipLaunchKernelGGL(k_readback, dim3((wd->n + 255) / 256), dim3(256), 0, wd->s, wd->st[wd->cur], tmp.p, (int)wd->n);
+    SR_TRY(wd->stage.to_host(planes, tmp.p, sizeof(float) * n, wd->s));
+    return tmp.give_back();
 }
 
 __global__ void k_sigma_in(const double *__restrict__ src, double *__restrict__ sigma, int n) {
@@ -698,13 +717,13 @@ extern "C" int sr_resume(sr_world *wd, const sr_resume_records *rec, const float
         wd->have_flux = true;
     }
     if (sigma) {
-        double *tmp = nullptr;
-        SR_HIP(hipMallocAsync((void **)&tmp, sizeof(double) * wd->n, wd->s));
-        SR_HIP(hipMemcpyAsync(tmp, sigma, sizeof(double) * wd->n, hipMemcpyHostToDevice, wd->s));
-        hipLaunchKernelGGL(k_sigma_in, dim3((wd->n + 255) / 256), dim3(256), 0, wd->s, (const double *)tmp,
+        CallMem<double> tmp(wd->s);
+        SR_TRY(tmp.get(wd->n));
+        SR_HIP(hipMemcpyAsync(tmp.p, sigma, sizeof(double) * wd->n, hipMemcpyHostToDevice, wd->s));
+        hipLaunchKernelGGL(k_sigma_in, dim3((wd->n + 255) / 256), dim3(256), 0, wd->s, (const double *)tmp.p,
                            wd->st[wd->cur].sigma, (int)wd->n);
         SR_HIP(hipGetLastError());
-        SR_HIP(hipFreeAsync(tmp, wd->s));
+        SR_TRY(tmp.give_back());
     }
     SR_HIP(hipStreamSynchronize(wd->s));
     return SR_OK;
@@ -739,14 +758,15 @@ extern "C" int sr_apply_heat_precond(sr_world *wd, const float *r, float *z, siz
     if (!wd || !r || !z) return fail(SR_ERR_ARGUMENT, "sr_apply_heat_precond: null pointer");
     if (!wd->first_built) return fail(SR_ERR_ARGUMENT, "sr_apply_heat_precond: no sr_heat_first_system yet");
     if (n != wd->n) return fail(SR_ERR_LENGTH, "sr_apply_heat_precond: n must be w*h");
-    float *d = nullptr;
-    SR_HIP(hipMallocAsync((void **)&d, sizeof(float) * 2 * n, wd->s));
+    CallMem<float> mem(wd->s);
+    SR_TRY(mem.get(2 * n));
+    float *d = mem.p;
     SR_HIP(hipMemcpyAsync(d, r, sizeof(float) * n, hipMemcpyHostToDevice, wd->s));
     SR_TRY(wd->heat.solver.apply_precond(d, d + n, wd->precond, wd->s));
     std::vector<uint8_t> gas(n);
     SR_HIP(hipMemcpyAsync(z, d + n, sizeof(float) * n, hipMemcpyDeviceToHost, wd->s));
     SR_HIP(hipMemcpyAsync(gas.data(), wd->heat.solver.gas0(), n, hipMemcpyDeviceToHost, wd->s));
-    SR_HIP(hipFreeAsync(d, wd->s));
+    SR_TRY(mem.give_back());
     SR_HIP(hipStreamSynchronize(wd->s));
     for (size_t i = 0; i < n; i++)
         if (!gas[i]) z[i] = 0.0f;  // rows off the gas are no part of the system
@@ -987,14 +1007,14 @@ extern "C" int sr_read_field(sr_world *wd, int field, float *out, size_t n) {
     if (!wd || !out) return fail(SR_ERR_ARGUMENT, "null pointer");
     if (n != wd->n) return fail(SR_ERR_LENGTH, "a side field holds w*h values");
     const float *src = nullptr;
-    float *tmp = nullptr;
+    CallMem<float> tmp(wd->s);
     switch (field) {
     case SR_FIELD_PHI:
     case SR_FIELD_PHI_MID:
-        SR_HIP(hipMallocAsync((void **)&tmp, sizeof(float) * n, wd->s));
+        SR_TRY(tmp.get(n));
         hipLaunchKernelGGL(k_extract_box, dim3((n + 255) / 256), dim3(256), 0, wd->s,
-                           field == SR_FIELD_PHI ? wd->phi : wd->phi_mid, wd->w, wd->h, tmp);
-        src = tmp;
+                           field == SR_FIELD_PHI ? wd->phi : wd->phi_mid, wd->w, wd->h, tmp.p);
+        src = tmp.p;
         break;
     case SR_FIELD_GX: src = wd->gx; break;
     case SR_FIELD_GY: src = wd->gy; break;
@@ -1004,7 +1024,7 @@ extern "C" int sr_read_field(sr_world *wd, int field, float *out, size_t n) {
     default: return fail(SR_ERR_ARGUMENT, "unknown field");
     }
     SR_HIP(hipMemcpyAsync(out, src, sizeof(float) * n, hipMemcpyDeviceToHost, wd->s));
-    if (tmp) SR_HIP(hipFreeAsync(tmp, wd->s));
+    SR_TRY(tmp.give_back());
     SR_HIP(hipStreamSynchronize(wd->s));
     return SR_OK;
 }

@@ -13,3 +13,9 @@ def stage(tmp_path_factory):
 @pytest.mark.parametrize("case", ["pageable", "pinned", "threads", "device"])
 def test_transfers(stage, case):
     run_host(stage, case)
+
+
+def test_a_failed_transfer_leaves_no_device_memory(tmp_path):
+    run_host(host_program(tmp_path, "world_transfer",
+                          [f + ".hip" for f in ("fld", "grav", "heat", "hydro", "net", "react", "sinks", "stage", "world")]
+                          + ["util.cpp"]))
