@@ -193,20 +193,26 @@ template <int CIN, int R, int S> struct ConvSlab {
     // every chunk's products, the wave walking its R + 2 input rows, each row's pixels read once and used by up to three
     // output rows, the next chunk's weights loading meanwhile. Lane l of an MFMA holds A[m = l % 16][k = 8 (l / 16) + j],
     // B[k = 8 (l / 16) + j][n = l % 16] and D[m = 4 (l / 16) + j][n = l % 16]: m the output channel, n the pixel, so a
-    // lane ends with four consecutive channels of one pixel. A padded pair reads the slab's first pair (inside the
-    // stencil) against zero weights.
+    // lane ends with four consecutive channels of one pixel. A padded pair's zero weights meet the zeros at `zeros` (not a
+    // pixel, which may be infinite).
     template <int NT>
-    static __device__ inline void products(const bf16 *wt, const bf16 *tile, bf16x8 (&w)[3][NT], f32x4 (&acc)[R][NT]) {
+    static __device__ inline void products(const bf16 *wt, const bf16 *tile, const bf16 *zeros, bf16x8 (&w)[3][NT],
+                                           f32x4 (&acc)[R][NT]) {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c16 = lane & 15;
 #pragma unroll
         for (int c = 0; c < C; c++) {
-            const int pair = 4 * c + g < 3 * OCT ? 4 * c + g : 0, tx = pair / OCT, o = pair % OCT;
+            const int pair = 4 * c + g, tx = pair / OCT, o = pair % OCT;
             const bf16 *px = tile + (16 * wave + c16 + tx) * CP + 8 * o;
+            int row = RW * CP;
+            if (4 * c + 3 >= 3 * OCT && pair >= 3 * OCT) {
+                px = zeros;
+                row = 0;
+            }
             bf16x8 wn[3][NT];
             if (c + 1 < C) weights<NT>(wt, c + 1, wn);
 #pragma unroll
             for (int i = 0; i < RH; i++) {
-                const bf16x8 p = ld8(px + i * RW * CP);
+                const bf16x8 p = ld8(px + i * row);
 #pragma unroll
                 for (int ty = 0; ty < 3; ty++) {
                     const int r = i - ty;
@@ -226,8 +232,8 @@ template <int CIN, int R, int S> struct ConvSlab {
 };
 
 template <int CIN, int R, int NT, int S>
-__device__ inline void conv_slabs(const ConvArgs &a, bf16 *tile, int x0, int y0, const ConvSlab<CIN, R, S> &slab,
-                                  f32x4 (&acc)[R][NT]) {
+__device__ inline void conv_slabs(const ConvArgs &a, bf16 *tile, const bf16 *zeros, int x0, int y0,
+                                  const ConvSlab<CIN, R, S> &slab, f32x4 (&acc)[R][NT]) {
     using SL = ConvSlab<CIN, R, S>;
     bf16x8 w[3][NT];
     SL::template weights<NT>(a.wt, 0, w);
@@ -236,11 +242,11 @@ __device__ inline void conv_slabs(const ConvArgs &a, bf16 *tile, int x0, int y0,
     if constexpr (SL::CB + SL::SC < CIN) {
         ConvSlab<CIN, R, S + 1> next;
         next.load(a, x0, y0);
-        SL::template products<NT>(a.wt, tile, w, acc);
+        SL::template products<NT>(a.wt, tile, zeros, w, acc);
         __syncthreads();  // the slab is read
-        conv_slabs<CIN, R, NT, S + 1>(a, tile, x0, y0, next, acc);
+        conv_slabs<CIN, R, NT, S + 1>(a, tile, zeros, x0, y0, next, acc);
     } else {
-        SL::template products<NT>(a.wt, tile, w, acc);
+        SL::template products<NT>(a.wt, tile, zeros, w, acc);
     }
 }
 
@@ -275,7 +281,9 @@ __global__ void __launch_bounds__(NTH) k_conv(ConvArgs a) {
     constexpr int SUMMED = EPI == CONV_SPLIT ? COUT / 3 * 2 : 0;  // the concat's upsampled channels
     static_assert(CIN % 8 == 0 && COUT % 16 == 0 && R % 2 == 0, "channel counts, rows");
     static_assert(EPI != CONV_OUT || COUT == 16, "the output layer reads 16 channels");
-    __shared__ __attribute__((aligned(16))) bf16 tile[(R + 2) * (TW + 2) * CPM];
+    constexpr int PIXELS = (R + 2) * (TW + 2) * CPM;
+    __shared__ __attribute__((aligned(16))) bf16 tile[PIXELS + 8];  // and eight zeros
+    if (threadIdx.x == 0) st8(tile + PIXELS, bf16x8{});
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c16 = lane & 15;
     const int blk = xcd_tile(), x0 = (blk % gridDim.x) * TW, y0 = (blk / gridDim.x) * R;
     f32x4 acc[R][NT];
@@ -286,7 +294,7 @@ __global__ void __launch_bounds__(NTH) k_conv(ConvArgs a) {
     {
         ConvSlab<CIN, R, 0> first;
         first.load(a, x0, y0);
-        conv_slabs<CIN, R, NT, 0>(a, tile, x0, y0, first, acc);
+        conv_slabs<CIN, R, NT, 0>(a, tile, tile + PIXELS, x0, y0, first, acc);
     }
     const int x = x0 + 16 * wave + c16, H = a.H, W = a.W;
     if (x0 + 16 * wave >= W) return;  // the whole wave is past the image

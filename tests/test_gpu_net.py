@@ -354,3 +354,50 @@ def test_last_layers_weight_gradient_over_ragged_tiles(gpu_lib, w, h):
         assert bool((err <= 2.0 ** -8 * size + 1e-30).all()), (t, float((err / size).max()))
     err = (torch.tensor(g["d1.b"], device="cuda") - ga.sum((0, 1))).abs()
     assert bool((err <= 2.0 ** -8 * ga.abs().sum((0, 1)) + 1e-30).all())
+
+
+def one_infinite_pixel(w, h, x, y):
+    """A system whose share of the diagonal is 0 at one cell: its third feature, log(own / d), is -inf there alone."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(31)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    own, kx, ky = rnd(h, w).exp(), rnd(h, w + 1).exp(), rnd(h + 1, w).exp()
+    own[y, x] = 0.0
+    return own, kx, ky, rnd(h, w), rnd(h, w)
+
+
+def single_path(p):
+    """e1a passes minus the third feature of its own pixel into channel 0, so that an infinite one stays one pixel of one
+    channel; every other weight of the layer is 0 (0 times infinity is no number, which the ReLU makes 0)."""
+    p["e1a.w"][:] = 0.0
+    p["e1a.b"][:] = 0.0
+    p["e1a.w"][1, 1, 2, 0] = -1.0
+
+
+# R = 2 rows a wave, then 8 (68 x 36 and 2052 x 1028 as above), the pixel inside a tile and at its left border
+@pytest.mark.parametrize("w,h,x,y", [(68, 36, 20, 9), (68, 36, 64, 35), (2052, 1028, 128, 200)])
+def test_an_infinite_activation_meets_no_padding(gpu_lib, w, h, x, y):
+    """An infinite input pixel reaches the nine outputs around it and those are infinite (or, negative, 0): a layer of 8
+    or 16 input channels pads its products, and the padding reads no pixel."""
+    import torch
+    import sandbox_reactions_amd as sr
+    print(f"net infinite {w}x{h}", flush=True)
+    own, kx, ky, r, _ = one_infinite_pixel(w, h, x, y)
+    z = torch.empty(h, w, device="cuda")
+    for name, src in (("e1a", "x"), ("e1", "e1a")):
+        p = random_params(32)
+        if name == "e1":
+            single_path(p)
+        net = sr.Net(w, h, p)
+        net.apply(own, kx, ky, r, z)
+        inp = torch.tensor(net.activation(src, w, h))[:, :, :3 if name == "e1a" else 16].double()
+        assert int(torch.isinf(inp).sum()) == 1 and not bool(torch.isnan(inp).any())
+        got = torch.tensor(net.activation(name, w, h)).double()
+        wt = torch.tensor(bf16(p[name + ".w"])).double()
+        for dy in range(-1, 2):
+            for dx in range(-1, 2):
+                if 0 <= y + dy < h and 0 <= x + dx < w:
+                    sign = wt[1 - dy, 1 - dx, 2 if name == "e1a" else 0] * (-1.0 if name == "e1a" else 1.0)
+                    assert torch.equal(torch.isinf(got[y + dy, x + dx]), sign > 0), (name, dy, dx)
+        assert int(torch.isinf(got).sum()) == int(torch.isinf(got[max(y - 1, 0):y + 2, max(x - 1, 0):x + 2]).sum())
