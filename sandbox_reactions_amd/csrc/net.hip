@@ -515,8 +515,9 @@ __global__ void __launch_bounds__(NTH) k_dw(const bf16 *__restrict__ in, const b
             st8(gs + px * GP + 8 * o, v);
         }
         __syncthreads();
+        const int rows = min(DW_TH, H - y0);  // a row below the image takes no part (its zeros may meet infinite pixels)
 #pragma unroll 1
-        for (int r = 0; r < DW_TH; r++) {
+        for (int r = 0; r < rows; r++) {
             bf16x8 gv[NBK];
 #pragma unroll
             for (int t = 0; t < NBK; t++) gv[t] = tr8(gs + r * DW_TW * GP + 16 * t, GP);

@@ -401,3 +401,29 @@ def test_an_infinite_activation_meets_no_padding(gpu_lib, w, h, x, y):
                     sign = wt[1 - dy, 1 - dx, 2 if name == "e1a" else 0] * (-1.0 if name == "e1a" else 1.0)
                     assert torch.equal(torch.isinf(got[y + dy, x + dx]), sign > 0), (name, dy, dx)
         assert int(torch.isinf(got).sum()) == int(torch.isinf(got[max(y - 1, 0):y + 2, max(x - 1, 0):x + 2]).sum())
+
+
+def test_a_weight_gradient_reads_no_pixel_past_the_last_row(gpu_lib):
+    """An infinite activation in the last row of a half-resolution layer whose outputs around it the ReLU all stops: the
+    weight gradient's sums for the row taps whose output pixel would lie below the image hold no such pixel, in a tile of
+    four rows that ends two rows past the image (six rows)."""
+    import torch
+    import sandbox_reactions_amd as sr
+    print("net dW past the last row", flush=True)
+    w, h = 16, 12
+    own, kx, ky, r, e = one_infinite_pixel(w, h, 5, 11)
+    p = random_params(33)
+    single_path(p)
+    for name in ("e1", "e2a"):
+        p[name + ".w"][:, :, 0] = 0.0
+        p[name + ".w"][1, 1, 0, 0] = 1.0  # the pixel goes on in channel 0 alone
+    p["e2.w"][:, :, 0] = -1.0             # and is stopped here
+    p["e2.b"][:] = 1.0
+    net = sr.Net(w, h, p)
+    net.loss_grad(own, kx, ky, r, e)
+    x, y = torch.tensor(net.activation("e2a", w, h)), torch.tensor(net.activation("e2", w, h))
+    assert torch.isinf(x).nonzero().tolist() == [[5, 2, 0]] and not bool(torch.isnan(x).any())
+    assert bool((y[4:, 1:4] == 0).all()) and not bool(torch.isinf(y).any())
+    g = sr.net.unflatten(net.grads())["e2.w"]
+    assert np.isnan(g[1:, :, 0]).all()       # 0 times infinity, the pixel's own row and the one above
+    assert np.isfinite(g[0, :, 0]).all() and np.isfinite(g[:, :, 1:]).all()
