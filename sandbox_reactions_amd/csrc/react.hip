@@ -30,18 +30,6 @@ __constant__ double r_zp1_a[NS] = {2.0, 3.0 / 4.0, 7.0 / 12.0, 9.0 / 16.0, 11.0 
                                    17.0 / 32.0, 27.0 / 56.0, 1.0};
 __constant__ double r_z_a[NS] = {1.0, 0.5, 0.5, 0.5, 0.5, 0.5, 0.5, 0.5, 26.0 / 56.0, 0.0};
 
-// ln of one Gamow-shaped term and f's direct form (rates.rs:44-53), on either side
-__host__ __device__ inline double term_ln(double t_k, double nu, double w, double t) {
-    const double u = log(t / t_k);
-    return log(w) - 2.0 / 3.0 * u - (3.0 * nu + 2.0) * expm1(-u / 3.0);
-}
-
-__host__ __device__ inline double f_sum(const sr_react_record &r, double t) {
-    double s = 0.0;
-    for (int k = 0; k < r.n_terms; k++) s += exp(term_ln(r.t_k[k], r.nu[k], r.w[k], t));
-    return s;
-}
-
 int react_check(const sr_react_params *p) {
     if (!p) return SR_OK;
     if (p->n_records < 0 || p->n_records > NR) return SR_ERR_ARGUMENT;
@@ -77,7 +65,6 @@ void react_build(const sr_react_params *p, const sr_physics &ph, ReactDev *out) 
         // rates.rs:62-71: log-spaced nodes from T_thr over the span; a record of the same law as an earlier one reads its
         out->f_of[r] = -1;
         if (c.n_terms == 0) continue;
-        out->ln_thr[r] = std::log(c.t_thr);
         for (int q = 0; q < r && out->f_of[r] < 0; q++) {
             const sr_react_record &o = p->rec[q];
             bool same = o.n_terms == c.n_terms && o.t_thr == c.t_thr;
@@ -142,20 +129,6 @@ __device__ __forceinline__ double ipow(double x, double n) {
     if (n == 3.0) return x * x * x;
     if (n == 0.0) return 1.0;
     return pow(x, n);
-}
-
-// f(T) through the table (rates.rs:98-118) from T and ln T: 0 below T_thr, the direct sum past the table's span
-__device__ inline double temp_factor(const ReactDev &D, const Lds &M, int r, double t, double ln_t) {
-    const sr_react_record &c = D.P.rec[r];
-    if (c.n_terms == 0) return 1.0;
-    if (t < c.t_thr) return 0.0;
-    const double step = log(2.5) / (double)(REACT_TABLE - 1);
-    const double pos = fmax(ln_t - D.ln_thr[r], 0.0) / step;
-    if (pos >= (double)(REACT_TABLE - 1)) return f_sum(c, t);
-    const int i = (int)floor(pos);
-    const double frac = pos - (double)i;
-    const double *ln_f = M.ln_f + D.f_of[r] * REACT_TABLE;
-    return exp(ln_f[i] + frac * (ln_f[i + 1] - ln_f[i]));
 }
 
 // the gate g(Y_e Sigma) (rates.rs:119-125)
@@ -270,14 +243,13 @@ __device__ inline void burn(const ReactDev &D, const Lds &M, double sigma, doubl
         }
         double enu = P.neutrinos && t >= P.t_nu ? P.a_nu * pow(t / P.t_nu, P.m_nu) : 0.0;
         int any = 0, f_last = -1;
-        const double ln_t = log(t);
         double f_val = 1.0;
         for (int r = 0; r < nr; r++) {
             if (r == P.nfe) continue;
             const sr_react_record &c = P.rec[r];
             // omega at X and, for each input j, at X with X_j = 1 (whose factor 1^n is exactly 1): f, g and A Sigma^a
             // once (f kept for a next record of the same law), each input's power once, the products in their order
-            if (c.n_terms == 0 || D.f_of[r] != f_last) f_val = temp_factor(D, M, r, t, ln_t);
+            if (c.n_terms == 0 || D.f_of[r] != f_last) f_val = temp_factor(D, M, r, t);
             f_last = D.f_of[r];
             const double f = f_val, g = gate(c, sigma, y_e);
             const double ap = c.a_coef * ipow(sigma, c.a_sigma);

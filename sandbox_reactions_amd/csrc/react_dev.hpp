@@ -33,9 +33,8 @@ struct ReactDev {
     int entries, items, ent0[SR_REACT_RECORDS + 1], slots, slot[SR_REACT_RECORDS];  // slot: a record's but N_Fe's
     unsigned row[REACT_NS];
     Item item[REACT_ITEMS];
-    // f's tables: record r reads table f_of[r] (records of the same law share one), tables in all; ln T_thr per record
+    // f's tables: record r reads table f_of[r] (records of the same law share one), tables in all
     int f_of[SR_REACT_RECORDS], tables;
-    double ln_thr[SR_REACT_RECORDS];
 };
 
 // nu, and the linear system's entries, items and elimination pattern, from out->P (the rest of *out zeroed)

@@ -1,5 +1,6 @@
-// P6 burning: the sub-step's linear system, (I - h J) dX = h S (crates/sr-physics/src/reference/react.rs:515-560). Compiled
-// for the device by react.hip; plain C++, so a CPU compiler builds it too.
+// P6 burning: the rates' temperature factor (crates/sr-physics/src/rates.rs:44-118) and the sub-step's linear system,
+// (I - h J) dX = h S (reference/react.rs:515-560). Compiled for the device by react.hip; plain C++, so a CPU compiler builds
+// it too.
 #pragma once
 #include <cmath>
 
@@ -23,6 +24,33 @@ struct Lds {
     const double *cold, *ln_f;
     double *v, *omega, *grad;  // the thread's own: element k at [k * NT]
 };
+
+// ln of one Gamow-shaped term and f's direct form (rates.rs:44-53), on either side
+REACT_HD inline double term_ln(double t_k, double nu, double w, double t) {
+    const double u = log(t / t_k);
+    return log(w) - 2.0 / 3.0 * u - (3.0 * nu + 2.0) * expm1(-u / 3.0);
+}
+
+REACT_HD inline double f_sum(const sr_react_record &r, double t) {
+    double s = 0.0;
+    for (int k = 0; k < r.n_terms; k++) s += exp(term_ln(r.t_k[k], r.nu[k], r.w[k], t));
+    return s;
+}
+
+// f(T) through the table (rates.rs:98-118): 0 below T_thr, the direct sum past the table's span (and for a T that is no
+// number, which stays none)
+REACT_HD inline double temp_factor(const ReactDev &D, const Lds &M, int r, double t) {
+    const sr_react_record &c = D.P.rec[r];
+    if (c.n_terms == 0) return 1.0;
+    if (t < c.t_thr) return 0.0;
+    const double step = log(2.5) / (double)(REACT_TABLE - 1);
+    const double pos = log(t / c.t_thr) / step;
+    if (!(pos < (double)(REACT_TABLE - 1))) return f_sum(c, t);
+    const int i = (int)floor(pos);
+    const double frac = pos - (double)i;
+    const double *ln_f = M.ln_f + D.f_of[r] * REACT_TABLE;
+    return exp(ln_f[i] + frac * (ln_f[i + 1] - ln_f[i]));
+}
 
 // (I - h J) dX = h S, Gaussian elimination with partial pivoting, the last of equal pivots (react.rs:515-560): the form
 // for a system that needs a row exchange, its matrix in scratch memory

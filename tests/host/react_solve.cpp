@@ -1,4 +1,4 @@
-// The P6 sub-step's linear system on the CPU: random records, derivatives and steps through solve<9> (no neutrons) and
+// P6's temperature factor and linear system on the CPU. The system: random records, derivatives and steps through solve<9> (no neutrons) and
 // solve<10>, against Gaussian elimination with partial pivoting in long double. Prints the largest error of a system's dX
 // over its largest element, and how many systems needed a row exchange.
 #include <cstdio>
@@ -74,7 +74,35 @@ template <int NA> static void run(int systems) {
     std::printf("%d %.3e\n", NA, worst);
 }
 
+// f(T) from just above T_thr to past the table's span against the same interpolation in long double, and T that is no
+// number. Prints the largest relative error.
+static void factor() {
+    double worst = 0.0;
+    for (int n = 0; n < 20000; n++) {
+        static ReactDev D;
+        std::memset(&D, 0, sizeof D);
+        sr_react_record &c = D.P.rec[0];
+        c.n_terms = 1;
+        c.t_thr = std::exp(uniform(-20.0, 20.0));
+        c.t_k[0] = 100.0 * c.t_thr;
+        c.nu[0] = uniform(1.0, 8.0);
+        c.w[0] = 1.0;
+        double ln_f[REACT_TABLE];
+        for (int i = 0; i < REACT_TABLE; i++)
+            ln_f[i] = std::log(f_sum(c, c.t_thr * std::exp(std::log(2.5) * i / (REACT_TABLE - 1))));
+        const Lds M = {nullptr, ln_f, nullptr, nullptr, nullptr};
+        const double t = c.t_thr * (n % 2 ? uniform(1.0, 2.49) : 1.0 + std::exp(uniform(-30.0, 0.0)));
+        const long double pos = logl((long double)t / c.t_thr) / (logl(2.5L) / (REACT_TABLE - 1));
+        const int i = (int)floorl(pos);
+        const long double ref = expl(ln_f[i] + (pos - i) * ((long double)ln_f[i + 1] - ln_f[i]));
+        worst = std::max(worst, (double)fabsl(temp_factor(D, M, 0, t) / ref - 1.0L));
+        if (!std::isnan(temp_factor(D, M, 0, NAN)) || temp_factor(D, M, 0, 0.999 * c.t_thr) != 0.0) worst = NAN;
+    }
+    std::printf("factor %.3e\n", worst);
+}
+
 int main() {
+    factor();
     run<REACT_NS - 1>(4000);
     run<REACT_NS>(4000);
 }
