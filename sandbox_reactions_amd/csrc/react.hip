@@ -446,6 +446,26 @@ __global__ void __launch_bounds__(NT, 2) k_react(const ReactDev *__restrict__ Dp
     block_partials<REACT_MAXES, 1>(vm, pmax, gridDim.x);
 }
 
+// The report's sums and maxima over the blocks, a block each, in a fixed order. On the host, over one block's worth of
+// partials per 64 or 256 cells, reading the report took 236 us at 2048^2.
+__global__ void __launch_bounds__(256) k_react_report(const double *psum, const double *pmax, int nb, double *out) {
+    const int k = blockIdx.x;
+    if (k < REACT_SUMS) {
+        const double s = sum_partials(psum + (size_t)k * nb, nb);
+        if (threadIdx.x == 0) out[k] = s;
+    } else {
+        double m[1] = {0.0};
+        for (int i = threadIdx.x; i < nb; i += 256) m[0] = fmax(m[0], pmax[(size_t)(k - REACT_SUMS) * nb + i]);
+        block_partials<1, 1>(m, out, 1, k);
+    }
+}
+
+int react_report(const double *psum, const double *pmax, int nb, double *out, hipStream_t s) {
+    hipLaunchKernelGGL(k_react_report, dim3(REACT_SUMS + REACT_MAXES), dim3(256), 0, s, psum, pmax, nb, out);
+    SR_HIP(hipGetLastError());
+    return SR_OK;
+}
+
 // whether the records' system leaves the neutrons out
 static bool react_neutrons(const ReactDev &h) {
     unsigned any = h.row[ID_N];

@@ -31,5 +31,7 @@ ReactLaunch react_plan(const ReactDev &h);
 int react_prepare(const ReactLaunch &plan);
 int react_launch(const ReactDev *D, const ReactLaunch &plan, const HydroState &st, int n, double dt, const double *scal,
                  double *nuclear, double *lost, double *snu, double *psum, double *pmax, int *nblocks, hipStream_t s);
+// the partials of nb blocks into out: the REACT_SUMS sums, then the REACT_MAXES maxima
+int react_report(const double *psum, const double *pmax, int nb, double *out, hipStream_t s);
 
 } // namespace sr

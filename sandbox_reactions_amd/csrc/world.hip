@@ -398,7 +398,7 @@ struct sr_world {
     // P6: the records and constants on the device (null: off), the last pass's per-cell bookings and partials
     ReactDev *react = nullptr, *react_dev_mem = nullptr;
     double *react_nuc = nullptr, *react_lost = nullptr, *react_snu = nullptr, *react_psum = nullptr,
-           *react_pmax = nullptr;
+           *react_pmax = nullptr, *react_out = nullptr;
     int react_nb = 0;
     ReactLaunch react_plan{};
     bool sinks_on = false;  // P3 in the step
@@ -1096,6 +1096,7 @@ extern "C" int sr_set_reactions(sr_world *wd, const sr_react_params *p) {
         SR_TRY(world_alloc(wd, (void **)&wd->react_nuc, sizeof(double) * SR_REACT_GROUPS * n));
         SR_TRY(world_alloc(wd, (void **)&wd->react_lost, sizeof(double) * n));
         SR_TRY(world_alloc(wd, (void **)&wd->react_snu, sizeof(double) * n));
+        SR_TRY(world_alloc(wd, (void **)&wd->react_out, sizeof(double) * (REACT_SUMS + REACT_MAXES)));
         const size_t most = (n + REACT_NT_LEAST - 1) / REACT_NT_LEAST;  // blocks
         SR_TRY(world_alloc(wd, (void **)&wd->react_psum, sizeof(double) * REACT_SUMS * most));
         SR_TRY(world_alloc(wd, (void **)&wd->react_pmax, sizeof(double) * REACT_MAXES * most));
@@ -1129,15 +1130,11 @@ extern "C" int sr_read_react(sr_world *wd, sr_react_report *out) {
     *out = sr_react_report{};
     const int nb = wd->react_nb;
     if (!wd->react_nuc || nb == 0) return SR_OK;
-    std::vector<double> ps((size_t)REACT_SUMS * nb), pm((size_t)REACT_MAXES * nb);
-    SR_HIP(hipMemcpyAsync(ps.data(), wd->react_psum, sizeof(double) * ps.size(), hipMemcpyDeviceToHost, wd->s));
-    SR_HIP(hipMemcpyAsync(pm.data(), wd->react_pmax, sizeof(double) * pm.size(), hipMemcpyDeviceToHost, wd->s));
+    double sum[REACT_SUMS + REACT_MAXES];
+    const double *mx = sum + REACT_SUMS;
+    SR_TRY(react_report(wd->react_psum, wd->react_pmax, nb, wd->react_out, wd->s));
+    SR_HIP(hipMemcpyAsync(sum, wd->react_out, sizeof sum, hipMemcpyDeviceToHost, wd->s));
     SR_HIP(hipStreamSynchronize(wd->s));
-    double sum[REACT_SUMS] = {}, mx[REACT_MAXES] = {};
-    for (int k = 0; k < REACT_SUMS; k++)
-        for (int b = 0; b < nb; b++) sum[k] += ps[(size_t)k * nb + b];
-    for (int k = 0; k < REACT_MAXES; k++)
-        for (int b = 0; b < nb; b++) mx[k] = std::max(mx[k], pm[(size_t)k * nb + b]);
     out->substeps = (uint64_t)sum[0];
     out->retried = (uint64_t)sum[1];
     out->unfinished = (uint64_t)sum[2];

@@ -60,6 +60,10 @@ def mass_radius(sigma, vac=1e-6, fraction=0.9):
     return rp + (r[k] - rp) * (fraction * mass - below) / pm[k], mass
 
 
+WORLD_SOURCES = [f + ".hip" for f in ("fld", "grav", "heat", "hydro", "net", "react", "sinks", "stage", "world")] + [
+    "util.cpp"]
+
+
 def host_program(tmp_path, name, sources):
     """tests/host/NAME.cpp with the library's host code of `sources` (no device code) over the stand-in for the HIP
     runtime, tests/host/fake_hip.hpp."""

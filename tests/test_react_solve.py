@@ -4,7 +4,7 @@ launches of worlds with different records, over a stand-in for the HIP runtime (
 import os
 import subprocess
 
-from helpers import HOST, host_program, run_host
+from helpers import HOST, WORLD_SOURCES, host_program, run_host
 
 
 def test_factor_and_system_within_their_arrays(tmp_path):
@@ -21,3 +21,7 @@ def test_factor_and_system_within_their_arrays(tmp_path):
 
 def test_no_world_lowers_the_lds_limit_of_another(tmp_path):
     run_host(host_program(tmp_path, "react_launch", ["react.hip", "util.cpp"]))
+
+
+def test_the_report_is_summed_on_the_device(tmp_path):
+    run_host(host_program(tmp_path, "react_report", WORLD_SOURCES))

@@ -2,7 +2,7 @@
 same bytes both ways whatever the caller's memory is and whatever fails."""
 import pytest
 
-from helpers import host_program, run_host
+from helpers import WORLD_SOURCES, host_program, run_host
 
 
 @pytest.fixture(scope="module")
@@ -16,6 +16,4 @@ def test_transfers(stage, case):
 
 
 def test_a_failed_transfer_leaves_no_device_memory(tmp_path):
-    run_host(host_program(tmp_path, "world_transfer",
-                          [f + ".hip" for f in ("fld", "grav", "heat", "hydro", "net", "react", "sinks", "stage", "world")]
-                          + ["util.cpp"]))
+    run_host(host_program(tmp_path, "world_transfer", WORLD_SOURCES))
