@@ -190,10 +190,12 @@ int sr_fld_levels(sr_fld *f, int *levels);
 int sr_fld_set_solve_mode(sr_fld *f, int mode);
 /* Tile shapes of the smoothers of the levels above the single-block ones (SR_TILE_16 16x16, SR_TILE_32 32x32,
  * SR_TILE_64 64x32, the last for nu1, nu2 <= 2 only): the project's autotuner times every shape on the first system
- * built and keeps the fastest per level below level 0 and smoother; sr_fld_set_tiles fixes them instead. Level 0
- * keeps 32x32 (its dot partials are counted per tile). No result bit depends on the shapes (exact red-black
- * Gauss-Seidel in every tiling). No counterpart in the reference, whose tiles are fixed by WebGPU's limits
- * (heat.wgsl:1401-1445: 16x16 with 4 RB pairs). */
+ * built and keeps the fastest per level below level 0 and smoother; sr_fld_set_tiles fixes them instead. Level 0's go by
+ * the grid's size, 16x16 on grids of fewer than 384 tiles of 32x32 and 32x32 on others (its dot partials are counted per
+ * tile): sr_fld_tiles reports what runs, and sr_fld_set_tiles takes that or SR_TILE_32 for both of its smoothers, which
+ * changes nothing there. No result bit depends on the other levels' shapes (exact red-black Gauss-Seidel in every
+ * tiling). No counterpart in the reference, whose tiles are fixed by WebGPU's limits (heat.wgsl:1401-1445: 16x16 with 4
+ * RB pairs). */
 int sr_fld_tiles(sr_fld *f, int *pre, int *post, int max_levels, int *levels);
 int sr_fld_set_tiles(sr_fld *f, const int *pre, const int *post, int levels);
 /* The last two tile-smoothed levels' pre-smoothers in one launch and their post-smoothers in another, when at least
@@ -210,8 +212,8 @@ int sr_fld_set_fusion(sr_fld *f, int pre, int post);
  * reference (its one coarse workgroup, heat.wgsl:1485-1526). */
 int sr_fld_set_coarse_wave(sr_fld *f, int on);
 /* Host-decided solves: each PCG iteration's update (x += alpha p, r -= alpha q, ||r||^2 partials) folded into the next
- * preconditioner application's level-0 pre-smoother (on, the default, where level 0 has 32 x 32 tiles apart from the
- * fused pair and at most 2^20 + 2^18 cells: on larger grids the update streams faster on its own), or launched on
+ * preconditioner application's level-0 pre-smoother (on, the default, where level 0 is tile-smoothed apart from the
+ * fused pair and has at most 2^20 + 2^18 cells: on larger grids the update streams faster on its own), or launched on
  * its own (off). x, r and z take the same values either way; the ||r||^2 partials are
  * summed per tile when folded. No counterpart in the reference (its update is a round of its chained dispatches,
  * heat.wgsl:605-877). */

@@ -1693,13 +1693,14 @@ int FldSolver::init(int w, int h, int levels, int nu1_, int nu2_, double omega_)
     const size_t n = (size_t)w * h;
     nbe = (int)std::max<size_t>(1, std::min<size_t>(NB_MAX, (n + NT * UNROLL - 1) / (NT * UNROLL)));
     // until the autotuner runs: 32x32 tiles, 16x16 on levels below level 0 that would launch fewer than 512 blocks of
-    // 32x32 (four times the blocks and a quarter of the serial work per thread where the launch is latency-bound)
+    // 32x32 (four times the blocks and a quarter of the serial work per thread where the launch is latency-bound); level 0's
+    // for good, by its own line
     pre_tile.assign(coarse_from, TILE_32);
     post_tile.assign(coarse_from, TILE_32);
     for (int l = 1; l < coarse_from; l++)
         if (((lv[l].w + 31) / 32) * ((lv[l].h + 31) / 32) < 512) pre_tile[l] = post_tile[l] = TILE_16;
-    tile0 = ((w + 31) / 32) * ((h + 31) / 32) < TILE0_FILL ? TILE_16 : TILE_32;
-    const int t0 = tile0 == TILE_16 ? 16 : 32;
+    const int tile0 = ((w + 31) / 32) * ((h + 31) / 32) < TILE0_FILL ? TILE_16 : TILE_32, t0 = tile0 == TILE_16 ? 16 : 32;
+    if (coarse_from > 0) pre_tile[0] = post_tile[0] = tile0;
     ntiles0 = ((w + t0 - 1) / t0) * ((h + t0 - 1) / t0);
     nbd_max = std::max(nbe, ntiles0);
     SR_HIP(hipMalloc(&gas, n));
@@ -1885,8 +1886,7 @@ int FldSolver::rebuild(bool faces, hipStream_t s) {
 // The autotuner: on the system just built, each tile-smoothed level's pre- and post-smoother below level 0 is timed
 // in every tile shape (one launch to warm, then the best of three means of eight launches, each between two events)
 // and keeps the fastest; a shape must beat the one kept by 3 % to replace it, so near-ties keep the default order's
-// choice. Level 0 keeps 32x32 tiles: it is the HBM-bound level the shape was chosen for by measurement, its
-// post-smoother's dot partials are counted per tile, and its pre-smoother is the kernel the bench's roofline names.
+// choice. Level 0 keeps its rule's tiles (TILE0_FILL): its post-smoother's dot partials are counted per tile.
 // The smoothers compute exact red-black Gauss-Seidel sweeps whatever the tiling, so the choice changes no result bit.
 // The launches write only the hierarchy's own work arrays (z, the coarse b, zp), which every V-cycle rewrites before
 // it reads them.
@@ -1996,10 +1996,13 @@ int FldSolver::set_tiles(const int *pre, const int *post, int levels) {
             if (v != TILE_16 && v != TILE_32 && !(v == TILE_64 && nu1 <= 2 && nu2 <= 2))
                 return fail(SR_ERR_ARGUMENT, "set_tiles: an unknown tile shape (or 64x32 with more than 2 sweeps)");
     }
-    if (levels > 0 && (pre[0] != TILE_32 || post[0] != TILE_32))
-        return fail(SR_ERR_ARGUMENT, "set_tiles: level 0 keeps 32x32 tiles");
-    pre_tile.assign(pre, pre + levels);
-    post_tile.assign(post, post + levels);
+    // level 0 runs its rule's shape whatever is asked: 32x32 stands for it in a plan, and what tiles() reports is taken
+    if (levels > 0 && (pre[0] != post[0] || (pre[0] != TILE_32 && pre[0] != pre_tile[0])))
+        return fail(SR_ERR_ARGUMENT, "set_tiles: level 0's tiles go by the grid's size");
+    for (int l = 1; l < levels; l++) {
+        pre_tile[l] = pre[l];
+        post_tile[l] = post[l];
+    }
     tuned = true;
     autotune = false;
     tiles_version++;
@@ -2115,7 +2118,7 @@ int FldSolver::launch_post_pair(int a, hipStream_t s, const int *gate) {
 int FldSolver::launch_pre_level(int l, const float *b, hipStream_t s, const int *gate) {
     const FldLevel &f = lv[l], &c = lv[l + 1];
     const Lv L = {f.w, f.h, f.own, f.ax, f.ay, f.cf};
-    switch (l == 0 ? tile0 : pre_tile[l]) {
+    switch (pre_tile[l]) {
     case TILE_16: launch_pre<16, 16>(nu1, s, L, b, f.z, c.b, c.w, gate); break;
     case TILE_64: launch_pre<PTX, PTY>(nu1, s, L, b, f.z, c.b, c.w, gate); break;
     default: launch_pre<32, 32>(nu1, s, L, b, f.z, c.b, c.w, gate); break;
@@ -2130,7 +2133,7 @@ int FldSolver::launch_post_level(int l, const float *b, float *zout, const float
     const FldLevel &f = lv[l], &c = lv[l + 1];
     const Lv L = {f.w, f.h, f.own, f.ax, f.ay, f.cf};
     int nb = 0;
-    switch (l == 0 ? tile0 : post_tile[l]) {
+    switch (post_tile[l]) {
     case TILE_16: nb = launch_post<16, 16>(nu2, s, L, b, f.z, c.zp, c.w, omega, zout, zold, part, gate); break;
     case TILE_64: nb = launch_post<PTX, PTY>(nu2, s, L, b, f.z, c.zp, c.w, omega, zout, zold, part, gate); break;
     default: nb = launch_post<32, 32>(nu2, s, L, b, f.z, c.zp, c.w, omega, zout, zold, part, gate); break;
@@ -2147,8 +2150,7 @@ int FldSolver::launch_post_level(int l, const float *b, float *zout, const float
 // kernel. So it is taken up to FOLD_MAX_CELLS (about 1145^2).
 #define FOLD_MAX_CELLS ((1u << 20) + (1u << 18))
 bool FldSolver::update_fusable() const {
-    return fuse_update && coarse_from > 0 && pair_level() != 0 && !pre_tile.empty() && pre_tile[0] == TILE_32 &&
-           nu1 >= 1 && nu1 <= 3 && (size_t)w0 * h0 <= FOLD_MAX_CELLS;
+    return fuse_update && coarse_from > 0 && pair_level() != 0 && nu1 >= 1 && nu1 <= 3 && (size_t)w0 * h0 <= FOLD_MAX_CELLS;
 }
 
 int FldSolver::vcycle(const float *r, float *z, const float *zold, double *dots, int *nbd, hipStream_t s,
@@ -2168,7 +2170,7 @@ int FldSolver::vcycle(const float *r, float *z, const float *zold, double *dots,
                 const int slot = tick(CLK_UPDATE_PRE0, s);
                 const FldLevel &f = lv[0];
                 const Lv L = {f.w, f.h, f.own, f.ax, f.ay, f.cf};
-                if (tile0 == TILE_16)
+                if (pre_tile[0] == TILE_16)
                     launch_pre_upd<16, 16>(nu1, s, L, *upd, f.z, c.b, c.w);
                 else
                     launch_pre_upd<32, 32>(nu1, s, L, *upd, f.z, c.b, c.w);

@@ -123,7 +123,6 @@ class FldSolver {
     // the tile shape (TILE_16, TILE_32, TILE_64) of each tile-smoothed level's pre- and post-smoother: the autotuner's
     // choice at the first rebuild, or the caller's (set_tiles)
     std::vector<int> pre_tile, post_tile;
-    int tile0 = TILE_32;  // level 0's, by the grid's size (its dot partials are counted per tile)
     bool tuned = false, autotune = true;
     int fuse_pre = FUSE_SMALL, fuse_post = FUSE_SMALL;
     bool coarse_wave = true;  // the single-block V-cycle's levels of at most 16 x 16 cells on one wave
