@@ -1427,11 +1427,6 @@ __global__ void k_coarsen_faces(Lv f, float *__restrict__ axc, float *__restrict
     }
 }
 
-// Once per rebuild, for the single-block V-cycle: every cell's inverse diagonal 1 / (own + its four couplings) on
-// every level of the set, and, when the coarsest holds at most DENSE_MAX cells, the inverse of its dense matrix by
-// Gauss-Jordan elimination (the matrix is SPD, so no pivoting); both into the pack. The elimination runs on the first
-// wave alone, row i of [A | I] in lane i's registers and the pivot row read across lanes, so it needs no block
-// barrier; the other waves form the inverse diagonals meanwhile.
 // The records (struct Block) of `threads` threads, 2^ltx to a row, over set level l and the next; entries t0, t0 + nt, ..
 __device__ inline void block_records(const CoarseSet &C, float *pack, int l, int ltx, int threads, int offrec, int t0,
                                      int nt) {
@@ -1475,6 +1470,11 @@ __device__ inline void block_records(const CoarseSet &C, float *pack, int l, int
     }
 }
 
+// Once per rebuild, for the single-block V-cycle, into the pack: the head's records and the wave tail's (inverse diagonals
+// among them), the inverse diagonals 1 / (own + its four couplings) of the levels below the head, and, when the coarsest
+// holds at most DENSE_MAX cells, the inverse of its dense matrix by Gauss-Jordan elimination (the matrix is SPD, so no
+// pivoting). The elimination runs on the first wave alone, row i of [A | I] in lane i's registers and the pivot row read
+// across lanes, so it needs no block barrier; the other waves form the rest meanwhile.
 __global__ void __launch_bounds__(COARSE_NT) k_coarse_prep(CoarseSet C, float *__restrict__ pack) {
     const int lc = C.n - 1, wl = C.w[lc], m = wl * C.h[lc];
     const bool dense = m <= DENSE_MAX;

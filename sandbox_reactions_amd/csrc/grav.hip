@@ -481,7 +481,9 @@ static bool rows_fit(int logl, int rb) {
 }
 
 // Rows per block without the autotuner: the most (8: a bin's rows go out 64 bytes at a time) that still make
-// ROWS_FILL blocks, two (16 bytes) at least.
+// ROWS_FILL blocks, two (16 bytes) at least. A field with 64, 128, 256, 512 and 1024: 27.0 / 24.7 / 23.9 / 23.9 / 24.0 us at
+// 512^2, 51.6 / 51.7 / 47.4 / 47.4 / 47.6 at 1024^2, 77.8 / 63.5 / 64.4 / 64.0 / 64.5 at 1300 x 700, 131.2 / 130.7 / 131.0 /
+// 120.3 / 122.8 at 2048^2, the same within 1 % at 601 x 433 from 128 on and at 4096^2.
 #define ROWS_FILL 256
 static int rows_per_block(int logl, int h) {
     int rb = 1;

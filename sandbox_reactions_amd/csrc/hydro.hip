@@ -195,7 +195,8 @@ template <int MODE, bool COLD, bool MULTI> struct Lds {
 // limiter and of the species' loop (its fluxes are zeros). Before, with each face made on both sides and all species in
 // the loop, the two took 313 and 732 us; with all ten species and the cold pressure at 512^2 29 + 74 us now, 49 + 104
 // before. 41 KB of LDS and 96 registers: four blocks to a CU (loading the update's inputs ahead of the fluxes spilled
-// and cost 20 %).
+// and cost 20 %). With the sinks two registers spill (12 bytes a lane; 20 steps of 512^2 with four sinks 5.2 ms, 6.1 before);
+// with the cold pressure it is 42 KB and 97 registers, three blocks (20 steps 4.6 ms, 5.7 before).
 template <int MODE, bool COLD, bool SINKS = false, bool MULTI = true>
 __global__ void __launch_bounds__(NSLOT, 5) k_hydro(HydroParams P, HydroState in, HydroState out,
                                                  const double *__restrict__ scal, const float *__restrict__ gx,

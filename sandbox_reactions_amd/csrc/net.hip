@@ -39,7 +39,10 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 #define DW_TW 32         // its tile
 #define DW_TH 4
 #define LOG_CLAMP 20.0f
-#define CONV_FILL 512  // blocks that a convolution's launch keeps the chip busy with
+// Blocks that a convolution's launch keeps the chip busy with: below it a wave takes half the rows. An application with 128,
+// 256, 512, 1024 and 2048: 91 / 91 / 87 / 90 / 90 us at 516 x 260, 112 / 102 / 99 / 99 / 108 at 512^2, 196 / 201 / 208 / 205
+// / 229 at 1024^2, 444 / 445 / 445 / 460 / 462 at 1540^2, 673 / 673 / 673 / 672 / 703 at 2048^2.
+#define CONV_FILL 512
 
 __device__ __forceinline__ bf16x8 ld8(const bf16 *p) { return *(const bf16x8 *)p; }
 __device__ __forceinline__ void st8(bf16 *p, bf16x8 v) { *(bf16x8 *)p = v; }
@@ -372,7 +375,8 @@ __global__ void __launch_bounds__(NTH) k_conv(ConvArgs a) {
 }
 
 // Rows per wave: the more rows, the fewer reads of LDS and of the halo per product (R + 2 for 3 R NT products), as long
-// as the launch still fills the chip; wide outputs keep four (their accumulators and weights take the registers).
+// as the launch still fills the chip; wide outputs keep four (eight take the registers of two waves a SIMD, and an
+// application at 2048^2 674 us as with four, a training step at 1024^2 972 against 965).
 template <int CIN, int COUT, int EPI = CONV_PLAIN> static void conv(hipStream_t s, const ConvArgs &a) {
     auto blocks = [&](int r) { return ((a.W + TW - 1) / TW) * ((a.H + r - 1) / r); };
     auto go = [&](auto kernel, int r) {

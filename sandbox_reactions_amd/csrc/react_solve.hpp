@@ -17,8 +17,9 @@ namespace sr {
 // The tables and the threads' private arrays in LDS: the cold pairs' ln u, f's tables, then per thread a value by species
 // (x while the rates are formed, dX after a solve), omega by record and the derivatives by entry. A species or record
 // index is the wave's own but not the compiler's, so such an array in registers would go to scratch memory (as the whole
-// pass's did: 587 us a pass at 512^2, 105 now). A thread's element k lies NT values from its element
-// k - 1: no bank conflicts. NT = 256 threads share the tables, so that two blocks (two waves a SIMD) fit a CU; with so many
+// pass's did: 587 us a pass at 512^2). What still goes there: 109 spilled registers (up to 153 with the neutrons) and the
+// arrays of the rare forms (the pivoted system, N_Fe's closed form), 1456 to 1552 bytes a lane. A thread's element k lies NT
+// values from its element k - 1: no bank conflicts. NT = 256 threads share the tables, so that two blocks (two waves a SIMD) fit a CU; with so many
 // inputs that they would not (the shipped records: 78 KB), 64.
 struct Lds {
     const double *cold, *ln_f;

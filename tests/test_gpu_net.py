@@ -308,7 +308,7 @@ def test_layers_match_over_every_tile_height(gpu_lib, w, h):
     assert float((z - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
 
 
-# one tile row, ragged tiles in both axes (32 x 4), and more tiles than blocks (each block walks five)
+# one tile row, ragged tiles in both axes (32 x 4), and more tiles than blocks (553 blocks walk two each)
 @pytest.mark.parametrize("w,h", [(32, 4), (68, 36), (516, 260)])
 def test_last_layers_weight_gradient_over_ragged_tiles(gpu_lib, w, h):
     """dW and db of the last 3x3 layer from its own input and output: ga = dL/d(out) w_out where the output is positive,
