@@ -1,7 +1,7 @@
 """The oracle: ctypes bindings to the f64 C restatement of the reference twin (liboracle.so).
 
 TEST INFRASTRUCTURE ONLY. The shipped library never imports this package; only tests/, the smoke check and the
-bench's CPU-baseline leg use it, and only as the checker. See sro.h for what each C function restates.
+bench's CPU-baseline leg use it, and only as the oracle. See sro.h for what each C function restates.
 """
 from __future__ import annotations
 

@@ -1,7 +1,7 @@
 /* The oracle: a CPU f64 restatement of the reference's twin for the grid-physics path.
  *
  * TEST INFRASTRUCTURE ONLY. Nothing in the shipped library links, loads or calls this code; only the test suite,
- * the smoke check and the bench's CPU-baseline leg use it, and only as the checker.
+ * the smoke check and the bench's CPU-baseline leg use it, and only as the oracle.
  *
  * Each function cites the reference file:line it restates (paths relative to the reference repository root).
  * Conventions follow the reference: channel-major planes, row-major cells, index = y * w + x, y down.

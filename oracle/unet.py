@@ -1,4 +1,4 @@
-"""The learned preconditioner's network, restated in numpy (f64) as the checker of the HIP forward and backward
+"""The learned preconditioner's network, restated in numpy (f64) as the oracle of the HIP forward and backward
 kernels. TEST INFRASTRUCTURE ONLY: the shipped library never imports it.
 
 The reference has no learned part (its FLD preconditioners are Jacobi and the multigrid of

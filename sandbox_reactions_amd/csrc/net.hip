@@ -3,7 +3,7 @@
 //
 // The reference has no learned part (its preconditioners are Jacobi and the multigrid of
 // crates/sr-engine/shaders/heat.wgsl:1160-1526); the network's definition is this library's, stated layer by layer in
-// the f64 numpy checker oracle/unet.py, whose names the kernels follow.
+// the f64 numpy oracle, oracle/unet.py, whose names the kernels follow.
 //
 //   * activations are channels-last BF16 (pixel-major, channels contiguous), so a lane's eight consecutive K values
 //     of the implicit GEMM are one 16-byte load;
